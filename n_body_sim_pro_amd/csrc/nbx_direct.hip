@@ -3,12 +3,11 @@
 // direct_fp64: bit-identical to the scalar reference kernel
 //   (src/c/physics/gravity.c:37-67). Every pair term is formed with the
 //   reference's operations in the reference's order (this file is compiled
-//   with -ffp-contract=off, FP64 sqrt and division are IEEE correctly
-//   rounded), and each target's three sums are accumulated in ascending j
-//   with j == i skipped. Only the term formation is parallel: four waves
-//   compute a 64-target x 32-source tile of terms into LDS, then three waves
-//   (one per component) add them in order. This keeps the serial dependency
-//   (one add per term) off the expensive part (div + sqrt per term).
+//   with -ffp-contract=off; nbx_exact.h gives the correctly rounded square
+//   root and reciprocal), and each target's three sums are accumulated in
+//   ascending j with j == i skipped. Only the term formation is parallel:
+//   several waves compute a tile of terms into LDS, one wave adds them in
+//   order; with enough targets one lane does both for its own target.
 //
 // direct_fp32: FP32 pair arithmetic on FP32-rounded positions/masses with a
 //   wave-uniform source index, so every source is fetched once per wave by
@@ -20,199 +19,316 @@
 //   in FP64, so a pair costs 12 full-rate VALU instructions and one
 //   v_rsq_f32.
 #include <mutex>
+#include <utility>
 
+#include "nbx_exact.h"
 #include "nbx_internal.h"
 #include "nbx_learned.h"
 
 namespace nbx {
 namespace {
 
-constexpr int kExactTargets = 64;
-constexpr int kExactSources = 16;
+constexpr int kExactTargets = 16;   // targets of a tile kernel's workgroup
 
-// One tile of terms: kExactSources sources (from j0) x the block's 64
-// targets, each of the block's WAVES waves forming kExactSources / WAVES
-// sources' terms with the reference's operations. STAGE: the tile's sources
-// (x, y, z, m) are read from the LDS stage `src`; otherwise from memory (the
-// last source repeated past n).
-template <int WAVES, bool STAGE>
-__device__ inline void exact_terms(double (*terms)[kExactSources][kExactTargets],
-                                   const double (*src)[kExactSources],
-                                   const double* __restrict__ px, const double* __restrict__ py,
-                                   const double* __restrict__ pz, const double* __restrict__ m,
-                                   int n, int j0, int wave, int lane, double xi, double yi,
-                                   double zi, double G, double eps2) {
-    constexpr int kPerWave = kExactSources / WAVES;
-    static_assert(kExactSources % WAVES == 0, "whole sources per wave");
+// The pair terms of K sources against one target per lane, with the
+// reference's operations in its order (gravity.c:46-57).
+template <int K>
+__device__ inline void exact_terms(const double (&sx)[K], const double (&sy)[K],
+                                   const double (&sz)[K], const double (&sm)[K], double xi,
+                                   double yi, double zi, double G, double eps2, double (&tx)[K],
+                                   double (&ty)[K], double (&tz)[K]) {
+    double r2[K], inv[K];
+    ExactGuard guard;
 #pragma unroll
-    for (int k = 0; k < kPerWave; ++k) {
-        const int jj = wave * kPerWave + k;
-        double sx, sy, sz, sm;
-        if (STAGE) {
-            sx = src[0][jj];
-            sy = src[1][jj];
-            sz = src[2][jj];
-            sm = src[3][jj];
-        } else {
-            const int j = j0 + jj;
-            const int jc = j < n ? j : n - 1;
-            sx = px[jc];
-            sy = py[jc];
-            sz = pz[jc];
-            sm = m[jc];
+    for (int k = 0; k < K; ++k) {
+        tx[k] = sx[k] - xi;
+        ty[k] = sy[k] - yi;
+        tz[k] = sz[k] - zi;
+        r2[k] = tx[k] * tx[k] + ty[k] * ty[k] + tz[k] * tz[k] + eps2;
+        inv[k] = exact_inv_sqrt(r2[k], guard);
+    }
+    if (__builtin_amdgcn_ballot_w64(guard.odd()) != 0) {
+        // (keeps the branch: flattened into selects, every term would pay
+        // for both paths)
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("");
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            inv[k] = 1.0 / sqrt(r2[k]);
         }
-        const double dx = sx - xi;
-        const double dy = sy - yi;
-        const double dz = sz - zi;
-        const double r2 = dx * dx + dy * dy + dz * dz + eps2;
-        const double inv = 1.0 / sqrt(r2);
-        const double inv3 = inv * inv * inv;
-        const double s = G * sm * inv3;
-        terms[0][jj][lane] = s * dx;
-        terms[1][jj][lane] = s * dy;
-        terms[2][jj][lane] = s * dz;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const double inv3 = inv[k] * inv[k] * inv[k];
+        const double s = G * sm[k] * inv3;
+        tx[k] = s * tx[k];
+        ty[k] = s * ty[k];
+        tz[k] = s * tz[k];
     }
 }
 
-// Loads (x, y, z, m) of the tile's kExactSources sources starting at j0 (the
-// last source repeated past n), one value per lane of the calling wave:
-// lane = field * kExactSources + source.
-static_assert(4 * kExactSources == kWave, "one staged source value per lane");
-__device__ inline double stage_value(const double* __restrict__ px, const double* __restrict__ py,
-                                     const double* __restrict__ pz, const double* __restrict__ m,
-                                     int n, int j0, int lane) {
-    const int f = lane / kExactSources;
-    const int j = j0 + lane % kExactSources;
-    const int jc = j < n ? j : n - 1;
-    const double* a = f == 0 ? px : (f == 1 ? py : (f == 2 ? pz : m));
-    return a[jc];
+// Adds COUNT terms, STRIDE doubles apart in LDS, in order; the loads of the
+// coming chunk are in flight during the adds of the current one, so the chain
+// is the adds alone.
+template <int COUNT, int STRIDE>
+__device__ inline double add_in_order(double acc, const double* row) {
+    constexpr int kChunk = COUNT % 16 == 0 ? 16 : 8;
+    static_assert(COUNT % kChunk == 0, "whole chunks");
+    double v[kChunk], w[kChunk];
+#pragma unroll
+    for (int e = 0; e < kChunk; ++e) {
+        v[e] = row[e * STRIDE];
+    }
+#pragma unroll
+    for (int c = kChunk; c < COUNT; c += kChunk) {
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) {
+            w[e] = row[(c + e) * STRIDE];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) {
+            acc += v[e];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < kChunk; ++e) {
+            v[e] = w[e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < kChunk; ++e) {
+        acc += v[e];
+    }
+    return acc;
 }
 
-// SUBSET: the block's targets are targets[k] for k = blockIdx.x * 64 + lane < count,
-// and the accelerations go to out[3k .. 3k+2].
-//
-// WAVES waves form the terms of a 16-source tile while waves 0-2 add the
-// previous tile's terms of one component each, in source order; two term
-// buffers alternate, one barrier per tile. (The serial sums are one add per
-// term; the terms, an IEEE divide and square root each, are spread over the
-// block's waves, which also hides their FP64 latency.) Sixteen waves suit
-// grids of under two blocks per CU, eight the larger ones; measured on
-// MI355X, ms per evaluation at N = 16384 / 65536 / 262144:
-//   16 waves: 1.18 / 11.96 / 179.9;  8 waves: 1.35 / 11.93 / 156.8;
-//   the earlier single-buffered 4-wave kernel: 1.69 / - / 192.
-// Loading a tile's 16 terms before its 16 adds (instead of one LDS wait per
-// add): 1.16 -> 0.82 / 11.9 -> 9.9 / 157 -> 136 ms with the dispatch above.
-// STAGE (from 32768 sources on): the sources come through an LDS stage that
-// the last wave fills one tile ahead (9.9 -> 9.4 ms at 65536, 136 -> 131 ms
-// at 262144, the 8192-target checker at 10M 0.57 -> 0.45 s; at 16384, where
-// the sources stay in cache, 0.82 -> 0.85 ms, so it is off there).
-template <bool SUBSET, int WAVES, bool STAGE>
-__global__ __launch_bounds__(WAVES * 64) void direct_fp64_kernel(
+// Lane LANE of each row of 16, in all lanes of that row.
+template <int LANE>
+__device__ inline double row_broadcast(double v) {
+    constexpr int kNewBcast = 0x150;   // row_newbcast:LANE
+    return __hiloint2double(
+        __builtin_amdgcn_update_dpp(0, __double2hiint(v), kNewBcast + LANE, 0xf, 0xf, true),
+        __builtin_amdgcn_update_dpp(0, __double2loint(v), kNewBcast + LANE, 0xf, 0xf, true));
+}
+
+template <int A, int... E>
+__device__ inline void row_fields(double v, double (&x)[A], double (&y)[A], double (&z)[A],
+                                  double (&m)[A], std::integer_sequence<int, E...>) {
+    ((x[E] = row_broadcast<E>(v), y[E] = row_broadcast<4 + E>(v), z[E] = row_broadcast<8 + E>(v),
+      m[E] = row_broadcast<12 + E>(v)), ...);
+}
+
+// Tile kernel: 16 targets per workgroup. WAVES waves form the terms of a tile
+// of 4 A WAVES sources (a wave's lanes are 16 targets x 4 sources, A
+// independent steps in flight), one more wave adds the previous tile's terms
+// in source order: lane = component * 16 + target, so one add serves all three
+// components. Two term buffers alternate, one barrier per tile. The own term
+// and the sources past n are written as +0.0, which leaves a sum bit for bit
+// as skipping them would (it starts at +0.0 and +0.0 + -0.0 is +0.0, so it is
+// never -0.0).
+// SUBSET: the targets are targets[k], k < count, and the accelerations go to
+// out[3k .. 3k+2].
+template <bool SUBSET, int WAVES, int A>
+__global__ __launch_bounds__((WAVES + 1) * 64) void direct_fp64_tile_kernel(
     const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
     const double* __restrict__ m, double* __restrict__ ax, double* __restrict__ ay,
     double* __restrict__ az, int n, double G, double eps2, const int64_t* __restrict__ targets,
     int count, double* __restrict__ out) {
-    __shared__ double terms[2][3][kExactSources][kExactTargets];
-    // sources of the next two tiles: the last wave loads tile t + 2's while
-    // the block forms tile t + 1's terms, so no wave waits on a global load
-    // after a barrier
-    __shared__ double src[2][4][kExactSources];
+    constexpr int kTile = 4 * A * WAVES;
+    constexpr int kRow = 3 * kExactTargets;
+    static_assert(A <= 4, "a row of lanes holds four sources' fields");
+    __shared__ double terms[2][kTile][kRow];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
-    const int k = blockIdx.x * kExactTargets + lane;
+    const int t = lane % kExactTargets;
+    const int q = lane / kExactTargets;   // source of a step, or component of the adder
+    const int k = blockIdx.x * kExactTargets + t;
+    const bool valid = SUBSET ? k < count : k < n;
+    const int i = !valid ? -1 : (SUBSET ? static_cast<int>(targets[k]) : k);
+    const int tiles = (n + kTile - 1) / kTile;
+    if (wave < WAVES) {
+        const int ic = valid ? i : n - 1;
+        const double xi = px[ic], yi = py[ic], zi = pz[ic];
+        const int s0 = wave * 4 * A + q;   // this lane's first source of a tile
+        // One load per tile: lane (q, 4 f + a) holds field f of the wave's
+        // source 4 a + q; a row broadcast then hands step a's four fields to
+        // the row's 16 targets. (With each lane loading its own steps'
+        // fields the vector memory path was the bound: N = 4096 64 us.)
+        const int field = t / 4;
+        const double* base = field == 0 ? px : (field == 1 ? py : (field == 2 ? pz : m));
+        const int mine = s0 + 4 * (t % 4);
+        auto load = [&](int j0) {
+            const int j = j0 + mine;
+            return base[j < n ? j : n - 1];
+        };
+        double next = load(0);
+        for (int b = 0; b < tiles; ++b) {
+            const int j0 = b * kTile;
+            const double cur = next;
+            if (b + 1 < tiles) {
+                next = load(j0 + kTile);   // in flight while this tile's terms are formed
+            }
+            double sx[A], sy[A], sz[A], sm[A], tx[A], ty[A], tz[A];
+            row_fields(cur, sx, sy, sz, sm, std::make_integer_sequence<int, A>{});
+            exact_terms<A>(sx, sy, sz, sm, xi, yi, zi, G, eps2, tx, ty, tz);
+            // the own source or the end of the sources within this wave's part
+            const int jw = j0 + wave * 4 * A;
+            const bool near = static_cast<unsigned>(i - jw) < 4u * A;
+            if (jw + 4 * A > n || __builtin_amdgcn_ballot_w64(near) != 0) {
+#pragma unroll
+                for (int a = 0; a < A; ++a) {
+                    const int j = j0 + s0 + 4 * a;
+                    const bool none = j >= n || j == i;
+                    tx[a] = none ? 0.0 : tx[a];
+                    ty[a] = none ? 0.0 : ty[a];
+                    tz[a] = none ? 0.0 : tz[a];
+                }
+            }
+            double (*row)[kRow] = terms[b & 1];
+#pragma unroll
+            for (int a = 0; a < A; ++a) {
+                row[s0 + 4 * a][t] = tx[a];
+                row[s0 + 4 * a][kExactTargets + t] = ty[a];
+                row[s0 + 4 * a][2 * kExactTargets + t] = tz[a];
+            }
+            __syncthreads();   // tile b written; the adder takes it
+        }
+    } else {
+        __builtin_amdgcn_s_setprio(3);   // the serial chain issues first
+        double acc = 0.0;
+        const int col = lane < kRow ? lane : kRow - 1;
+        for (int b = 0; b < tiles; ++b) {
+            __syncthreads();   // tile b written
+            acc = add_in_order<kTile, kRow>(acc, &terms[b & 1][0][col]);
+        }
+        if (valid && lane < kRow) {
+            if (SUBSET) {
+                out[3 * static_cast<size_t>(k) + q] = acc;
+            } else {
+                (q == 0 ? ax : (q == 1 ? ay : az))[i] = acc;
+            }
+        }
+    }
+}
+
+// One target per lane, sources in order through scalar loads, four sources'
+// terms formed side by side and added in order: no LDS, no barrier.
+template <bool SUBSET>
+__global__ __launch_bounds__(256) void direct_fp64_lane_kernel(
+    const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
+    const double* __restrict__ m, double* __restrict__ ax, double* __restrict__ ay,
+    double* __restrict__ az, int n, double G, double eps2, const int64_t* __restrict__ targets,
+    int count, double* __restrict__ out) {
+    constexpr int K = 4;
+    const int k = blockIdx.x * 256 + threadIdx.x;
     const bool valid = SUBSET ? k < count : k < n;
     const int i = !valid ? -1 : (SUBSET ? static_cast<int>(targets[k]) : k);
     const int ic = valid ? i : n - 1;
     const double xi = px[ic], yi = py[ic], zi = pz[ic];
-    double acc = 0.0;
-    const int tiles = (n + kExactSources - 1) / kExactSources;
-    constexpr int kLoader = WAVES - 1;
-    if (STAGE && wave == kLoader) {
-        (&src[0][0][0])[lane] = stage_value(px, py, pz, m, n, 0, lane);
-        (&src[1][0][0])[lane] = stage_value(px, py, pz, m, n, kExactSources, lane);
+    double acx = 0.0, acy = 0.0, acz = 0.0;
+    // sources of the coming group; its scalar loads are in flight while the
+    // current group's terms are formed
+    double nx[K], ny[K], nz[K], nm[K];
+    auto load = [&](int j0) {
+#pragma unroll
+        for (int e = 0; e < K; ++e) {
+            nx[e] = px[j0 + e];
+            ny[e] = py[j0 + e];
+            nz[e] = pz[j0 + e];
+            nm[e] = m[j0 + e];
+        }
+    };
+    const int whole = n / K * K;
+    if (whole > 0) {
+        load(0);
     }
-    __syncthreads();
-    exact_terms<WAVES, STAGE>(terms[0], src[0], px, py, pz, m, n, 0, wave, lane, xi, yi, zi, G,
-                              eps2);
-    __syncthreads();
-    for (int t = 0; t < tiles; ++t) {
-        const int j0 = t * kExactSources;
-        if (wave < 3) {
-            // in-order sum of tile t, one component per wave
-            const int jn = (n - j0) < kExactSources ? (n - j0) : kExactSources;
-            const double (*row)[kExactTargets] = terms[t & 1][wave];
-            if (jn == kExactSources) {
-                // all of the tile's loads first, then the adds: one LDS
-                // latency per tile instead of one per term. The own term
-                // adds +0.0, which leaves the sum bit for bit as skipping it
-                // would (the sum starts at +0.0, and +0.0 + -0.0 is +0.0,
-                // so it is never -0.0).
-                double v[kExactSources];
+    for (int j0 = 0; j0 < whole; j0 += K) {
+        double sx[K], sy[K], sz[K], sm[K], tx[K], ty[K], tz[K];
 #pragma unroll
-                for (int jj = 0; jj < kExactSources; ++jj) {
-                    v[jj] = row[jj][lane];
-                }
+        for (int e = 0; e < K; ++e) {
+            sx[e] = nx[e];
+            sy[e] = ny[e];
+            sz[e] = nz[e];
+            sm[e] = nm[e];
+        }
+        load(j0 + K < whole ? j0 + K : 0);
+        exact_terms<K>(sx, sy, sz, sm, xi, yi, zi, G, eps2, tx, ty, tz);
+        // the own term adds +0.0
+        const bool near = static_cast<unsigned>(i - j0) < static_cast<unsigned>(K);
+        if (__builtin_amdgcn_ballot_w64(near) != 0) {
 #pragma unroll
-                for (int jj = 0; jj < kExactSources; ++jj) {
-                    acc += (j0 + jj != i) ? v[jj] : 0.0;
-                }
-            } else {
-                for (int jj = 0; jj < jn; ++jj) {
-                    if (j0 + jj != i) {
-                        acc += row[jj][lane];
-                    }
-                }
+            for (int e = 0; e < K; ++e) {
+                const bool own = j0 + e == i;
+                tx[e] = own ? 0.0 : tx[e];
+                ty[e] = own ? 0.0 : ty[e];
+                tz[e] = own ? 0.0 : tz[e];
             }
         }
-        if (t + 1 < tiles) {
-            // tile t + 2's sources go to the stage tile t used
-            double next = 0.0;
-            if (STAGE && wave == kLoader) {
-                next = stage_value(px, py, pz, m, n, j0 + 2 * kExactSources, lane);
-            }
-            exact_terms<WAVES, STAGE>(terms[(t + 1) & 1], src[(t + 1) & 1], px, py, pz, m, n,
-                                      j0 + kExactSources, wave, lane, xi, yi, zi, G, eps2);
-            if (STAGE && wave == kLoader) {
-                (&src[t & 1][0][0])[lane] = next;
-            }
+#pragma unroll
+        for (int e = 0; e < K; ++e) {
+            acx += tx[e];
+            acy += ty[e];
+            acz += tz[e];
         }
-        __syncthreads();
     }
-    if (valid && wave < 3) {
+    for (int j = whole; j < n; ++j) {
+        const double sx[1] = {px[j]}, sy[1] = {py[j]}, sz[1] = {pz[j]}, sm[1] = {m[j]};
+        double tx[1], ty[1], tz[1];
+        exact_terms<1>(sx, sy, sz, sm, xi, yi, zi, G, eps2, tx, ty, tz);
+        acx += j == i ? 0.0 : tx[0];
+        acy += j == i ? 0.0 : ty[0];
+        acz += j == i ? 0.0 : tz[0];
+    }
+    if (valid) {
         if (SUBSET) {
-            out[3 * static_cast<size_t>(k) + wave] = acc;
+            double* o = out + 3 * static_cast<size_t>(k);
+            o[0] = acx;
+            o[1] = acy;
+            o[2] = acz;
         } else {
-            double* o = wave == 0 ? ax : (wave == 1 ? ay : az);
-            o[i] = acc;
+            ax[i] = acx;
+            ay[i] = acy;
+            az[i] = acz;
         }
     }
 }
 
 // Launches the FP64 all-pairs kernel over `count` targets (all n particles,
-// or the SUBSET `targets`) with the wave count that suits the grid.
+// or the SUBSET `targets`) that suits the grid. A workgroup of the tile kernel
+// takes 16 targets. Up to one per CU, eight waves form terms; up to three per
+// CU, six; beyond, three, of which four workgroups fit a CU. From 1.75 waves
+// of targets per SIMD on the lane kernel, which has no LDS traffic, fills the
+// chip by itself. Measured on MI355X, ms per evaluation with 8 / 6 / 3 waves
+// and the lane kernel (every result bit for bit the same):
+//   N = 1000   0.0137 / 0.0147 / 0.0178 / 0.096    N = 4096  0.0445 / 0.0476 / 0.0623 / 0.375
+//   N = 8192   0.163  / 0.147  / 0.164  / 0.75     N = 12288 0.353  / 0.314  / 0.320  / -
+//   N = 16384  0.604  / 0.522  / 0.492  / 1.54     N = 40000 3.44   / -      / 2.56   / 4.0
+//   N = 98304  3 waves 14.7, lane 15.7;  110000: 18.5, 17.8;  131072: 25.4, 22.9
+// The kernel this replaced (64 targets per workgroup, IEEE sqrt and divide):
+// 0.049 ms at 1000, 0.186 at 4096, 0.79 at 16384, 4.28 at 40000, 9.05 at 65536
+// (now 6.9). The bound is FP64 issue: about 38 instructions and a v_rsq_f64 a
+// pair, 84 ns per 64 pairs and SIMD, against 72 instructions and two
+// transcendentals before; a tile kernel's adder and row broadcasts add 12.
 template <bool SUBSET>
 void launch_direct_fp64(hipStream_t st, int cu_count, const double* px, const double* py,
                         const double* pz, const double* m, double* ax, double* ay, double* az,
                         int n, double G, double eps2, const int64_t* targets, int count,
                         double* out) {
+    auto go = [&](auto kernel, unsigned grid, unsigned threads) {
+        kernel<<<grid, threads, 0, st>>>(px, py, pz, m, ax, ay, az, n, G, eps2, targets, count,
+                                         out);
+    };
     const unsigned blocks = grid_for(static_cast<size_t>(count), kExactTargets);
-    const bool stage = n >= 32768;
-    if (blocks < 2u * static_cast<unsigned>(cu_count)) {
-        if (stage) {
-            direct_fp64_kernel<SUBSET, 16, true><<<blocks, 16 * 64, 0, st>>>(
-                px, py, pz, m, ax, ay, az, n, G, eps2, targets, count, out);
-        } else {
-            direct_fp64_kernel<SUBSET, 16, false><<<blocks, 16 * 64, 0, st>>>(
-                px, py, pz, m, ax, ay, az, n, G, eps2, targets, count, out);
-        }
+    const unsigned cus = static_cast<unsigned>(cu_count);
+    if (blocks <= cus) {
+        go(direct_fp64_tile_kernel<SUBSET, 8, 4>, blocks, 9 * kWave);
+    } else if (blocks <= 3 * cus) {
+        go(direct_fp64_tile_kernel<SUBSET, 6, 4>, blocks, 7 * kWave);
+    } else if (blocks < 28 * cus) {
+        go(direct_fp64_tile_kernel<SUBSET, 3, 4>, blocks, 4 * kWave);
     } else {
-        if (stage) {
-            direct_fp64_kernel<SUBSET, 8, true><<<blocks, 8 * 64, 0, st>>>(
-                px, py, pz, m, ax, ay, az, n, G, eps2, targets, count, out);
-        } else {
-            direct_fp64_kernel<SUBSET, 8, false><<<blocks, 8 * 64, 0, st>>>(
-                px, py, pz, m, ax, ay, az, n, G, eps2, targets, count, out);
-        }
+        go(direct_fp64_lane_kernel<SUBSET>, grid_for(static_cast<size_t>(count), 256), 256);
     }
 }
 

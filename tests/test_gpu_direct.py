@@ -182,3 +182,36 @@ def test_direct_fp32_zero_softening_is_finite(nbx):
     p = from_gen(d)
     acc = gpu_force(nbx, p, "hip_direct_fp32", 0.0)
     assert np.all(np.isfinite(acc))
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 127, 128, 129, 4096, 4097, 12289, 114701])
+def test_direct_fp64_kernel_edges_bit_identical(nbx, oracle, n):
+    """Around the tiles of 16 targets and 48 to 128 sources, and at the sizes
+    from which the launch takes another kernel on 256 CUs: rows of the whole
+    evaluation against the oracle, bit for bit."""
+    p = from_gen(nbx.plummer(n, seed=5)) if n > 1 else Particles(1, {"px": [0.5], "m": [1.0]})
+    acc = gpu_force(nbx, p, "hip_direct_fp64", 0.01, G=1.5)
+    rows = np.unique(np.r_[np.arange(min(n, 20)), np.arange(0, n, max(1, n // 200)),
+                           np.arange(max(0, n - 20), n)]).astype(np.int64)
+    out = np.zeros((rows.size, 3))
+    oracle.nbo_direct_openmp_subset(C.byref(p.view), C.byref(gravity(1.5, 0.01)),
+                                    rows.ctypes.data_as(C.POINTER(C.c_int64)), rows.size,
+                                    out.ctypes.data_as(C.POINTER(C.c_double)))
+    assert np.array_equal(acc[rows], out)
+
+
+@pytest.mark.parametrize("n", [40, 5000])
+@pytest.mark.parametrize("scale", [1.0, 1e-170, 1e-95, 1e95, 1e170])
+def test_direct_fp64_outside_the_fast_range_bit_identical(nbx, oracle, n, scale):
+    """Unsoftened sums with coincident particles (r = 0) and distances whose
+    squares leave 2^-600 .. 2^600, underflow or overflow: the IEEE path gives
+    the oracle's values, infinities and NaN included."""
+    d = nbx.plummer(n, seed=9)
+    pos = d["pos"] * scale
+    pos[7] = pos[3]
+    pos[n // 2] *= 1e3
+    p = Particles(n, {"px": pos[:, 0], "py": pos[:, 1], "pz": pos[:, 2], "m": d["m"]})
+    acc = gpu_force(nbx, p, "hip_direct_fp64", 0.0)
+    q = p.copy()
+    oracle.nbo_direct_openmp(C.byref(q.view), C.byref(gravity(1.0, 0.0)))
+    assert np.array_equal(acc, q.acc(), equal_nan=True)
