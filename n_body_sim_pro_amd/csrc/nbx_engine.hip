@@ -74,9 +74,9 @@ constexpr int kThreads = 256;
 // arrays, diagnostics scratch); the array's size follows the list.
 auto work_buffers(Engine* e) {
     BHState& s = e->bh;
-    return std::array{&s.b4, &s.partial, &s.flags, &s.mkey, &s.tkey, &s.sk0, &s.sk1, &s.sv0, &s.sv1,
-            &s.hist, &s.mperm, &s.mkey_sorted, &s.tperm, &s.trank, &s.tword, &s.ext, &s.delta,
-            &s.cnt, &s.scan, &s.scan_part, &s.sp4, &s.s4, &s.tile_hist, &s.tile_base, &s.n64,
+    return std::array{&s.b4, &s.partial, &s.flags, &s.sk0, &s.sk1, &s.sv0, &s.sv1, &s.hist,
+            &s.mkey, &s.mperm, &s.tperm, &s.tword, &s.ext, &s.ext_orig, &s.delta, &s.scan,
+            &s.sp4, &s.s4, &s.tile_hist, &s.tile_base, &s.n64,
             &s.n32, &s.icom, &s.irec, &s.idepth, &s.gnode, &s.im2, &s.gquad,
             &s.tmp32, &s.counters, &s.deferred, &e->scratch, &e->scratch2};
 }
@@ -407,7 +407,7 @@ void nbx_engine_destroy(NBXEngine* engine) {
     for (nbx::Buf* b : nbx::work_buffers(e)) {
         nbx::free_buf(*b);
     }
-    if (e->bh.host_flags != nullptr) (void)hipHostFree(e->bh.host_flags);
+    if (e->bh.report != nullptr) (void)hipHostFree(e->bh.report);
     if (e->mlp != nullptr) {
         nbx_mlp_release(e->mlp);
     }
@@ -668,6 +668,9 @@ NBodySimProStatus nbx_engine_bh_morton(NBXEngine* engine, double* root, uint64_t
     if (root != nullptr) {
         for (int k = 0; k < 4; ++k) root[k] = e->bh.root[k];
     }
+    if (keys != nullptr || permutation != nullptr) {
+        NBX_TRY(nbx::bh_morton_order(e, error));
+    }
     if (keys != nullptr) {
         NBX_HIP(error, hipMemcpy(keys, e->bh.mkey.p, n * sizeof(uint64_t), hipMemcpyDeviceToHost));
     }
@@ -719,7 +722,15 @@ NBodySimProStatus nbx_engine_bh_export_nodes(NBXEngine* engine, double* rows,
         for (size_t k = 0; k < nodes; ++k) leaf[k] = recs[k].leaf;
     }
     NBX_HIP(error, hipMemcpy(word.data(), s.tword.p, n * 8, hipMemcpyDeviceToHost));
-    NBX_HIP(error, hipMemcpy(trank.data(), s.trank.p, n * 4, hipMemcpyDeviceToHost));
+    {
+        // Morton rank of each tree position's particle
+        NBX_TRY(nbx::bh_morton_order(e, error));
+        std::vector<uint32_t> mperm(n), tperm(n), rank(n);
+        NBX_HIP(error, hipMemcpy(mperm.data(), s.mperm.p, n * 4, hipMemcpyDeviceToHost));
+        NBX_HIP(error, hipMemcpy(tperm.data(), s.tperm.p, n * 4, hipMemcpyDeviceToHost));
+        for (size_t k = 0; k < n; ++k) rank[mperm[k]] = static_cast<uint32_t>(k);
+        for (size_t k = 0; k < n; ++k) trank[k] = rank[tperm[k]];
+    }
     // A leaf's row comes from its tree position t: depth one below the deeper
     // neighbour cell, the particle itself as mass and centre of mass.
     std::vector<int32_t> delta(n);
@@ -747,10 +758,9 @@ NBodySimProStatus nbx_engine_bh_export_nodes(NBXEngine* engine, double* rows,
         cz[k] = sp[4 * t + 2];
         m[k] = sp[4 * t + 3];
     }
-    if (s.tie_path) {
+    if (s.ext_tree != nullptr) {
         ext.resize(n * 6);
-        NBX_HIP(error, hipMemcpy(ext.data(), static_cast<uint64_t*>(s.ext.p) + 2 * n * 6,
-                                 n * 6 * 8, hipMemcpyDeviceToHost));
+        NBX_HIP(error, hipMemcpy(ext.data(), s.ext_tree, n * 6 * 8, hipMemcpyDeviceToHost));
     }
     for (size_t k = 0; k < nodes; ++k) {
         // Replay the cell centre from the root along the node's octant path

@@ -98,35 +98,36 @@ struct BHState {
     size_t n = 0;             // particles in the last build
     size_t internal = 0;      // internal nodes in the last build
     size_t nodes = 0;         // n + internal
+    size_t cells = 0;         // internal cells the record buffers are sized for
+    size_t cells_n = 0;       // the particle count that size was chosen for
     int max_depth = 0;
-    bool tie_path = false;
-    bool mismatch_path = false;
     bool has_n64 = false;     // the last build wrote FP64 node records
     bool has_quad = false;    // the last build wrote quadrupole records
     bool has_n32 = false;     // the FP32 pre-order records of the last build are written
+    bool has_morton = false;  // mkey and mperm hold the last build's Morton order
     bool inputs_fp64 = false; // the last build ran on FP64 inputs (b4 and sp4 are double4)
-    const uint64_t* ext_tree = nullptr;   // tree-order extension words (tie path) or null
+    const uint64_t* ext_tree = nullptr;   // tree-order extension words or null (ext below)
     double root[4] = {0, 0, 0, 1};
-    // pinned host block the build reads its flags, per-depth counts and root
-    // cube into (asynchronous copies; owned here so they always land)
-    void* host_flags = nullptr;
+    // pinned host block the evaluation's flags, counts, root cube and
+    // interaction counters are reported into (BuildReport)
+    void* report = nullptr;
     // build inputs (x, y, z, m): FP32-rounded copies of the master arrays
     // (float4) or the FP64 values (double4)
     Buf b4;                   // (x, y, z, m) per particle in original order
     Buf partial;              // bbox partials + root
     Buf flags;                // flags, per-depth counts, offsets and cursors
-    Buf mkey, tkey;           // Morton / true-path keys in original order
     Buf sk0, sk1, sv0, sv1;   // sort ping-pong
     Buf hist;                 // sort histograms
-    Buf mperm;                // Morton order: sorted position -> original index
-    Buf mkey_sorted;          // Morton keys ascending
+    Buf mkey;                 // Morton keys in original order, on demand (true-path keys while
+                              // an order on all the bits is made)
+    Buf mperm;                // Morton order: sorted position -> original index, on demand
     Buf tperm;                // tree position -> original index
-    Buf trank;                // tree position -> Morton rank
     Buf tword;                // tree-order true keys (descending)
-    Buf ext;                  // extension key words (6 per particle) on the tie path
+    Buf ext;                  // extension key words (6 per tree position; only those of
+                              // positions that share their key with a neighbour are read)
+    Buf ext_orig;             // the same in original order (order on all the bits)
     Buf delta;                // int32 common levels between tree positions t, t+1
-    Buf cnt, scan;            // internal nodes started per tree position, exclusive scan
-    Buf scan_part;            // scan block partials
+    Buf scan;                 // internal cells started before each tree position
     Buf sp4;                  // tree-order FP64 (x, y, z, m), FP64 builds only
     Buf s4;                   // tree-order FP32 x, y, z, m
     Buf tile_hist, tile_base; // per-tile, per-depth internal-node counts and their scan
@@ -185,7 +186,11 @@ NBodySimProStatus bh_build(Engine* e, bool fp32_inputs, NBodySimProError* error,
 // The FP32 pre-order node records of the last build (NodeF32, for the
 // per-query walks and the node export), written once per build on first use.
 NBodySimProStatus bh_node_records(Engine* e, NBodySimProError* error);
-// One walk per bh_build: the build clears the walk's interaction counters.
+// The Morton keys and order of the last build (mkey, mperm), on demand.
+NBodySimProStatus bh_morton_order(Engine* e, NBodySimProError* error);
+// One walk per bh_build, before anything reads the build: bh_build only
+// enqueues, and the walk's end is where the host learns the tree's size (and
+// repairs a build whose flags say so). The build clears the walk's counters.
 NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exact,
                           float* features, NBodySimProError* error);
 NBodySimProStatus bh_learned(Engine* e, const NBodySimProGravity* g, NBodySimProError* error);
@@ -194,16 +199,13 @@ NBodySimProStatus bh_learned(Engine* e, const NBodySimProGravity* g, NBodySimPro
 // equal keys keep their input order. It sorts by key bits first_bit ..
 // first_bit + bits - 1 (the bits below first_bit are ignored: equal there
 // counts as equal). The result goes to keys_out/vals_out when given (they
-// must not alias the alternate buffers), else back into keys/vals.
+// must not alias the alternate buffers), else back into keys/vals. iota: the
+// values are the input positions (vals is not read).
 NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals,
                                    uint64_t* keys_alt, uint32_t* vals_alt, size_t n, int bits,
                                    Buf& hist, NBodySimProError* error,
                                    uint64_t* keys_out = nullptr, uint32_t* vals_out = nullptr,
-                                   int first_bit = 0);
-// Exclusive scan of uint32 (total written to out[n]).
-NBodySimProStatus exclusive_scan_u32(hipStream_t s, const uint32_t* in, uint32_t* out, size_t n,
-                                     Buf& partial, NBodySimProError* error);
-
+                                   int first_bit = 0, bool iota = false);
 // Bits of `mask` set in the lanes below this one (v_mbcnt_lo/hi: two VALU
 // instructions, where and-ing a per-lane mask and counting bits takes four).
 __device__ inline unsigned lanes_below(uint64_t mask) {

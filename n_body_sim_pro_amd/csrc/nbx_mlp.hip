@@ -751,7 +751,7 @@ NBodySimProStatus bh_learned(Engine* e, const NBodySimProGravity* g, NBodySimPro
     tm.tree_ms = t[3] - t[9];
     tm.com_ms = t[4] - t[3];
     float walk_ms = 0.f;
-    NBX_HIP(error, hipEventElapsedTime(&walk_ms, e->ev[5], e->ev[6]));
+    NBX_HIP(error, hipEventElapsedTime(&walk_ms, e->ev[4], e->ev[6]));
     tm.walk_ms = walk_ms;
     tm.force_ms = t[8];
     tm.kernel_ms = walk_ms;

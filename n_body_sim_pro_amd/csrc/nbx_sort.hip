@@ -1,12 +1,12 @@
-// nbx_sort.hip - stable LSD radix sort of (u64 key, u32 value) pairs and an
-// exclusive u32 scan, both for gfx950 (wave64).
+// nbx_sort.hip - stable LSD radix sort of (u64 key, u32 value) pairs for gfx950
+// (wave64).
 //
 // The reference sorts a size_t permutation by 63-bit Morton keys with three
 // stable 21-bit LSD passes and a 2^21-entry counting array
 // (src/c/barnes_hut/barnes_hut.c:312-339). Any stable sort on the full key
 // yields the same permutation (ties keep ascending original index). Here the
 // digit is 9 bits (7 passes cover 63 bits; a caller may sort a window of the
-// key bits, as the Morton sort does with the top 36) and a pass is three
+// key bits, as the tree order does with the top 36) and a pass is three
 // launches:
 //   sort_histogram   per-tile digit counts (2048-item tiles, 4096 for large
 //                    inputs; LDS atomics);
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter(
         unsigned d = 0;
         if (valid) {
             key = kin[i];
-            val = vin[i];
+            val = vin != nullptr ? vin[i] : static_cast<uint32_t>(i);
             d = digit_of(key, shift);
         }
         uint64_t peers = __ballot(valid);
@@ -226,102 +226,12 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter(
     }
 }
 
-constexpr int kScanThreads = 256;
-constexpr int kScanIpt = 4;
-constexpr int kScanTile = kScanThreads * kScanIpt;
-
-__device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* s, uint32_t* total) {
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < kScanThreads; off <<= 1) {
-        const uint32_t t = threadIdx.x >= static_cast<unsigned>(off) ? s[threadIdx.x - off] : 0u;
-        __syncthreads();
-        s[threadIdx.x] += t;
-        __syncthreads();
-    }
-    const uint32_t incl = s[threadIdx.x];
-    *total = s[kScanThreads - 1];
-    __syncthreads();
-    return incl - v;
-}
-
-__global__ __launch_bounds__(kScanThreads) void scan_tiles(const uint32_t* __restrict__ in,
-                                                          size_t n,
-                                                          uint32_t* __restrict__ partial) {
-    __shared__ uint32_t s[kScanThreads];
-    const size_t base = static_cast<size_t>(blockIdx.x) * kScanTile + threadIdx.x * kScanIpt;
-    uint32_t sum = 0;
-#pragma unroll
-    for (int k = 0; k < kScanIpt; ++k) {
-        sum += (base + k < n) ? in[base + k] : 0u;
-    }
-    uint32_t total;
-    block_exclusive_scan(sum, s, &total);
-    if (threadIdx.x == 0) {
-        partial[blockIdx.x] = total;
-    }
-}
-
-// One workgroup: each thread sums a contiguous chunk of the tile totals, one
-// block scan of the chunk sums, then each thread writes its chunk's running
-// offsets. (Measured on MI355X: 9,766 tiles at 10M particles took 42 us as
-// one block scan per 256 totals.)
-__global__ __launch_bounds__(kScanThreads) void scan_partials(uint32_t* __restrict__ partial,
-                                                             unsigned count) {
-    __shared__ uint32_t s[kScanThreads];
-    const unsigned per = (count + kScanThreads - 1) / kScanThreads;
-    const unsigned lo = min(count, threadIdx.x * per);
-    const unsigned hi = min(count, lo + per);
-    uint32_t sum = 0;
-    for (unsigned i = lo; i < hi; ++i) {
-        sum += partial[i];
-    }
-    uint32_t total;
-    uint32_t run = block_exclusive_scan(sum, s, &total);
-    for (unsigned i = lo; i < hi; ++i) {
-        const uint32_t v = partial[i];
-        partial[i] = run;
-        run += v;
-    }
-    if (threadIdx.x == 0) {
-        partial[count] = total;
-    }
-}
-
-__global__ __launch_bounds__(kScanThreads) void scan_apply(const uint32_t* __restrict__ in,
-                                                          size_t n,
-                                                          const uint32_t* __restrict__ partial,
-                                                          unsigned tiles,
-                                                          uint32_t* __restrict__ out) {
-    __shared__ uint32_t s[kScanThreads];
-    const size_t base = static_cast<size_t>(blockIdx.x) * kScanTile + threadIdx.x * kScanIpt;
-    uint32_t v[kScanIpt];
-    uint32_t sum = 0;
-#pragma unroll
-    for (int k = 0; k < kScanIpt; ++k) {
-        v[k] = (base + k < n) ? in[base + k] : 0u;
-        sum += v[k];
-    }
-    uint32_t total;
-    uint32_t run = block_exclusive_scan(sum, s, &total) + partial[blockIdx.x];
-#pragma unroll
-    for (int k = 0; k < kScanIpt; ++k) {
-        if (base + k < n) {
-            out[base + k] = run;
-        }
-        run += v[k];
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        out[n] = partial[tiles];
-    }
-}
-
 }  // namespace
 
 NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals,
                                    uint64_t* keys_alt, uint32_t* vals_alt, size_t n, int bits,
                                    Buf& hist, NBodySimProError* error, uint64_t* keys_out,
-                                   uint32_t* vals_out, int first_bit) {
+                                   uint32_t* vals_out, int first_bit, bool iota) {
     if (keys_out == nullptr || vals_out == nullptr) {
         keys_out = keys;
         vals_out = vals;
@@ -333,6 +243,9 @@ NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals
         NBX_FAIL(error, N_BODY_SIM_PRO_STATUS_INVALID_ARGUMENT, "sort size exceeds 2^32");
     }
     if (n == 1) {
+        if (iota) {
+            NBX_HIP(error, hipMemsetAsync(vals, 0, sizeof(uint32_t), s));
+        }
         if (keys_out != keys) {
             NBX_HIP(error, hipMemcpyAsync(keys_out, keys, sizeof(uint64_t), hipMemcpyDeviceToDevice, s));
             NBX_HIP(error, hipMemcpyAsync(vals_out, vals, sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
@@ -346,7 +259,7 @@ NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals
     uint32_t* totals = h + static_cast<size_t>(kRadix) * tiles;
     const int passes = (bits + kDigitBits - 1) / kDigitBits;
     const uint64_t* kin = keys;
-    const uint32_t* vin = vals;
+    const uint32_t* vin = iota ? nullptr : vals;
     for (int p = 0; p < passes; ++p) {
         const int shift = first_bit + kDigitBits * p;
         // ping-pong between the two buffers; the last pass writes the output
@@ -355,7 +268,7 @@ NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals
         uint32_t* vout = last ? vals_out : ((p & 1) ? vals : vals_alt);
         if (last && (kout == kin || static_cast<const uint32_t*>(vout) == vin)) {
             kout = (kin == keys) ? keys_alt : keys;     // output aliases the input: one more hop
-            vout = (vin == vals) ? vals_alt : vals;
+            vout = (kout == keys) ? vals : vals_alt;
         }
         if (large) {
             sort_histogram<8><<<tiles, kSortThreads, 0, s>>>(kin, n, shift, h, tiles);
@@ -378,22 +291,6 @@ NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals
         NBX_HIP(error, hipMemcpyAsync(keys_out, kin, n * sizeof(uint64_t), hipMemcpyDeviceToDevice, s));
         NBX_HIP(error, hipMemcpyAsync(vals_out, vin, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
     }
-    return N_BODY_SIM_PRO_STATUS_OK;
-}
-
-NBodySimProStatus exclusive_scan_u32(hipStream_t s, const uint32_t* in, uint32_t* out, size_t n,
-                                     Buf& partial, NBodySimProError* error) {
-    if (n == 0) {
-        NBX_HIP(error, hipMemsetAsync(out, 0, sizeof(uint32_t), s));
-        return N_BODY_SIM_PRO_STATUS_OK;
-    }
-    const unsigned tiles = grid_for(n, kScanTile);
-    NBX_TRY(partial.need<uint32_t>(tiles + 1, error));
-    uint32_t* part = partial.as<uint32_t>();
-    scan_tiles<<<tiles, kScanThreads, 0, s>>>(in, n, part);
-    scan_partials<<<1, kScanThreads, 0, s>>>(part, tiles);
-    scan_apply<<<tiles, kScanThreads, 0, s>>>(in, n, part, tiles, out);
-    NBX_HIP(error, hipGetLastError());
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 

@@ -338,3 +338,66 @@ def test_member_test_still_refines_reference_lists(nbx, theta):
     # reference lists (medians of 2048 sampled particles, 2% slack)
     assert out["box"][1] <= 1.02 * out["member"][1]
     assert out["member"][1] <= 1.02 * out["reference"][1]
+
+
+def build_edge_inputs(case, n):
+    rng = np.random.default_rng(n)
+    if case == "uniform":
+        pos = rng.uniform(-1, 1, size=(n, 3))
+    elif case == "plummer_like":
+        pos = rng.normal(size=(n, 3)) / np.maximum(rng.uniform(size=(n, 1)), 1e-3)
+    else:
+        # pairs: chains of single-child cells above each (more cells than
+        # particles, tiles with more cells than LDS holds); 1e-9 apart the two
+        # share all 21 levels of the key
+        gap = {"pairs": 1e-5, "tied_pairs": 1e-9}[case]
+        base = rng.uniform(-1, 1, size=((n + 1) // 2, 3))
+        pos = np.concatenate([base, base + rng.uniform(0.1, 1, size=base.shape) * gap])[:n]
+        pos = pos[rng.permutation(n)]
+    return pos, rng.uniform(0.5, 1.0, n)
+
+
+@pytest.mark.parametrize("case,n", [
+    ("uniform", 2), ("uniform", 63), ("uniform", 65), ("uniform", 1024), ("uniform", 1025),
+    ("plummer_like", 32768), ("plummer_like", 32769), ("uniform", 65536), ("uniform", 65537),
+    ("plummer_like", 70001), ("pairs", 3001), ("pairs", 40001), ("tied_pairs", 3001),
+    ("tied_pairs", 40001)])
+def test_bh_build_edges_bit_identical(nbx, oracle, case, n):
+    """Around the sizes at which the build takes another path (tiles of 1,024
+    positions, groups of 64 tiles, the two ways of ordering), and trees with
+    more cells than the records or a tile's LDS table hold at first: keys,
+    order, nodes and exact walk against the oracle, twice on one engine."""
+    pos, m = build_edge_inputs(case, n)
+    p = Particles(n, {"px": pos[:, 0], "py": pos[:, 1], "pz": pos[:, 2], "m": m})
+    st, oacc, os_, okeys, operm, oroot, orows = oracle_bh(oracle, p, 0.7, 0.01)
+    assert st == 0
+    with nbx.Engine(n, theta=0.7) as e:
+        e.upload_view(p.view)
+        for _ in range(2):
+            e.compute_force("hip_barnes_hut_fp64", eps=0.01)
+            assert np.array_equal(e.accelerations(), oacc)
+            assert stats_tuple(e.stats()) == stats_tuple(os_)
+        root, keys, perm = e.bh_morton()
+        rows = e.bh_export_nodes()
+    assert np.array_equal(root, oroot)
+    assert np.array_equal(keys, okeys)
+    assert np.array_equal(perm, operm)
+    assert np.array_equal(sort_rows(rows), sort_rows(orows))
+
+
+def test_bh_long_run_next_to_ties_in_a_large_system(nbx, oracle):
+    """A run of equal top key bits too long for the order kernel, with tied
+    pairs elsewhere: ordered on all the bits."""
+    pos, m = build_edge_inputs("tied_pairs", 40000)
+    rng = np.random.default_rng(1)
+    pos = np.concatenate([pos, np.array([0.3, 0.3, 0.3]) + rng.uniform(-1e-6, 1e-6, (100, 3))])
+    m = np.concatenate([m, np.ones(100)])
+    p = Particles(len(m), {"px": pos[:, 0], "py": pos[:, 1], "pz": pos[:, 2], "m": m})
+    st, oacc, os_, okeys, operm, oroot, orows = oracle_bh(oracle, p, 0.5, 0.01)
+    assert st == 0
+    e, acc, s = gpu_bh(nbx, p, 0.5, 0.01, "hip_barnes_hut_fp64")
+    rows = e.bh_export_nodes()
+    e.close()
+    assert np.array_equal(acc, oacc)
+    assert stats_tuple(s) == stats_tuple(os_)
+    assert np.array_equal(sort_rows(rows), sort_rows(orows))
