@@ -9,15 +9,16 @@
 //   several waves compute a tile of terms into LDS, one wave adds them in
 //   order; with enough targets one lane does both for its own target.
 //
-// direct_fp32: FP32 pair arithmetic on FP32-rounded positions/masses with a
-//   wave-uniform source index, so every source is fetched once per wave by
-//   scalar loads and broadcast through SGPR operands (no LDS traffic). Each
-//   lane owns one target; its sources are split over S waves of the block.
-//   Partial sums of T sources are folded into a per-target compensated
-//   (Kahan-Babuska) accumulator once per tile, and the S ranges' accumulators
-//   are combined in LDS in range order. G multiplies each target's sum once,
-//   in FP64, so a pair costs 12 full-rate VALU instructions and one
-//   v_rsq_f32.
+// direct_fp32: FP32 pair arithmetic on FP32-rounded positions/masses. Each lane
+//   owns one target. In large systems the source index is wave-uniform, so
+//   every source is fetched once per wave by scalar loads and broadcast
+//   through SGPR operands (no LDS traffic), and a target's sources are split
+//   over the 16 waves of its workgroup; small systems spread a wave over 16
+//   targets x 4 sources. Partial sums of a few dozen sources are folded into a
+//   per-target compensated (Kahan-Babuska) accumulator, and the ranges'
+//   accumulators are combined in LDS in range order. G multiplies each
+//   target's sum once, in FP64, so a pair costs 12 full-rate VALU instructions
+//   and one v_rsq_f32.
 #include <mutex>
 #include <utility>
 
@@ -340,22 +341,38 @@ __device__ inline void two_sum_add(float& s, float& c, float v) {
     c += e;
 }
 
-// One target per lane. A block's four waves cover 256 / S targets: each
-// target's sources are split into S ranges of whole tiles, one per wave, and
-// the partial sums meet in LDS in range order (deterministic).
+// One pair term m / r^3 d added to (ax, ay, az): 12 full-rate VALU instructions
+// and one v_rsq_f32.
+template <bool ZERO_EPS>
+__device__ inline void fp32_pair(const float4& q, float xi, float yi, float zi, float eps2,
+                                 float& ax, float& ay, float& az) {
+    const float dx = q.x - xi;
+    const float dy = q.y - yi;
+    const float dz = q.z - zi;
+    const float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
+    float inv = __builtin_amdgcn_rsqf(r2);
+    if (ZERO_EPS) {
+        inv = r2 > 0.f ? inv : 0.f;
+    }
+    const float inv2 = inv * inv;
+    const float s = (q.w * inv) * inv2;
+    ax = fmaf(s, dx, ax);
+    ay = fmaf(s, dy, ay);
+    az = fmaf(s, dz, az);
+}
+
+// One target per lane, 64 per workgroup. The targets' sources are split into S
+// ranges of whole tiles, one per wave, and the partial sums meet in LDS in
+// range order (deterministic).
 template <int S, bool ZERO_EPS>
-__global__ __launch_bounds__(256) void direct_fp32_kernel(const float4* __restrict__ pos,
-                                                          double* __restrict__ ax,
-                                                          double* __restrict__ ay,
-                                                          double* __restrict__ az, int n,
-                                                          double G, float eps2, int tile) {
-    static_assert(S == 1 || S == 2 || S == 4, "source ranges per target");
-    constexpr int kTargetWaves = 4 / S;
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+__global__ __launch_bounds__(S * kWave) void direct_fp32_kernel(const float4* __restrict__ pos,
+                                                                double* __restrict__ ax,
+                                                                double* __restrict__ ay,
+                                                                double* __restrict__ az, int n,
+                                                                double G, float eps2, int tile) {
+    const int part = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
     const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
-    const int part = wave / kTargetWaves;                  // source range of this wave
-    const int t = (wave % kTargetWaves) * kWave + lane;    // target within the block
-    const int i = blockIdx.x * (kWave * kTargetWaves) + t;
+    const int i = blockIdx.x * kWave + lane;
     const float4 p = pos[i < n ? i : n - 1];
     const float xi = p.x, yi = p.y, zi = p.z;
     const int tiles = (n + tile - 1) / tile;
@@ -368,55 +385,108 @@ __global__ __launch_bounds__(256) void direct_fp32_kernel(const float4* __restri
         float px = 0.f, py = 0.f, pz = 0.f;
 #pragma unroll 4
         for (int j = j0; j < j1; ++j) {
-            const float4 q = pos[j];
-            const float dx = q.x - xi;
-            const float dy = q.y - yi;
-            const float dz = q.z - zi;
-            const float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-            float inv = __builtin_amdgcn_rsqf(r2);
-            if (ZERO_EPS) {
-                inv = r2 > 0.f ? inv : 0.f;
-            }
-            const float inv2 = inv * inv;
-            const float s = (q.w * inv) * inv2;
-            px = fmaf(s, dx, px);
-            py = fmaf(s, dy, py);
-            pz = fmaf(s, dz, pz);
+            fp32_pair<ZERO_EPS>(pos[j], xi, yi, zi, eps2, px, py, pz);
         }
         two_sum_add(sx, cx, px);
         two_sum_add(sy, cy, py);
         two_sum_add(sz, cz, pz);
     }
-    if (S > 1) {
-        __shared__ float part_sums[S > 1 ? S - 1 : 1][6][kWave * kTargetWaves];
-        if (part > 0) {
-            float* r = &part_sums[part - 1][0][0];
-            constexpr int kStride = kWave * kTargetWaves;
-            r[0 * kStride + t] = sx;
-            r[1 * kStride + t] = sy;
-            r[2 * kStride + t] = sz;
-            r[3 * kStride + t] = cx;
-            r[4 * kStride + t] = cy;
-            r[5 * kStride + t] = cz;
+    __shared__ float part_sums[S - 1][6][kWave];
+    if (part > 0) {
+        float* r = &part_sums[part - 1][0][lane];
+        r[0 * kWave] = sx;
+        r[1 * kWave] = sy;
+        r[2 * kWave] = sz;
+        r[3 * kWave] = cx;
+        r[4 * kWave] = cy;
+        r[5 * kWave] = cz;
+    }
+    __syncthreads();
+    if (part == 0) {
+        for (int k = 0; k < S - 1; ++k) {
+            two_sum_add(sx, cx, part_sums[k][0][lane]);
+            two_sum_add(sy, cy, part_sums[k][1][lane]);
+            two_sum_add(sz, cz, part_sums[k][2][lane]);
+            cx += part_sums[k][3][lane];
+            cy += part_sums[k][4][lane];
+            cz += part_sums[k][5][lane];
         }
-        __syncthreads();
-        if (part == 0) {
-#pragma unroll
-            for (int k = 0; k < S - 1; ++k) {
-                two_sum_add(sx, cx, part_sums[k][0][t]);
-                two_sum_add(sy, cy, part_sums[k][1][t]);
-                two_sum_add(sz, cz, part_sums[k][2][t]);
-                cx += part_sums[k][3][t];
-                cy += part_sums[k][4][t];
-                cz += part_sums[k][5][t];
-            }
+        if (i < n) {
+            // G applied once per target, in FP64 (exact for G = 1)
+            ax[i] = G * (static_cast<double>(sx) + static_cast<double>(cx));
+            ay[i] = G * (static_cast<double>(sy) + static_cast<double>(cy));
+            az[i] = G * (static_cast<double>(sz) + static_cast<double>(cz));
         }
     }
-    if (part == 0 && i < n) {
-        // G applied once per target, in FP64 (exact for G = 1)
-        ax[i] = G * (static_cast<double>(sx) + static_cast<double>(cx));
-        ay[i] = G * (static_cast<double>(sy) + static_cast<double>(cy));
-        az[i] = G * (static_cast<double>(sz) + static_cast<double>(cz));
+}
+
+// Small systems: 16 targets per workgroup; a wave's lanes are 16 targets x 4
+// sources, the 16 waves take every 16th group of four, and the 64 partial sums
+// of a target (at most 192 plain terms each) meet by compensated adds, over the
+// lanes and then over the waves in order. STAGE: one launch, every workgroup
+// rounds all the sources to FP32 into LDS itself; otherwise they come from the
+// staged positions `pos`.
+constexpr int kStageN = 4096;
+constexpr int kSmallN = 12288;
+constexpr int kSmallTargets = 16;
+constexpr int kSmallWaves = 16;
+template <bool ZERO_EPS, bool STAGE>
+__global__ __launch_bounds__(kSmallWaves * kWave) void direct_fp32_small_kernel(
+    const double* __restrict__ px, const double* __restrict__ py, const double* __restrict__ pz,
+    const double* __restrict__ m, const float4* __restrict__ pos, double* __restrict__ ax, double* __restrict__ ay,
+    double* __restrict__ az, int n, double G, float eps2) {
+    __shared__ float4 stage[STAGE ? kStageN : 1];
+    __shared__ float part_sums[kSmallWaves][6][kSmallTargets];
+    if (STAGE) {
+        for (int j = threadIdx.x; j < n; j += kSmallWaves * kWave) {
+            stage[j] = make_float4(static_cast<float>(px[j]), static_cast<float>(py[j]),
+                                   static_cast<float>(pz[j]), static_cast<float>(m[j]));
+        }
+        __syncthreads();
+    }
+    const float4* src = STAGE ? stage : pos;
+    const int wave = static_cast<int>(threadIdx.x) / kWave;
+    const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+    const int t = lane % kSmallTargets;
+    const int i = blockIdx.x * kSmallTargets + t;
+    const float4 p = src[i < n ? i : n - 1];
+    float s[3] = {0.f, 0.f, 0.f}, c[3] = {0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int j = wave * (kWave / kSmallTargets) + lane / kSmallTargets; j < n;
+         j += kSmallWaves * (kWave / kSmallTargets)) {
+        fp32_pair<ZERO_EPS>(src[j], p.x, p.y, p.z, eps2, s[0], s[1], s[2]);
+    }
+#pragma unroll
+    for (int off = kSmallTargets; off < kWave; off <<= 1) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const float so = __shfl_xor(s[k], off), co = __shfl_xor(c[k], off);
+            two_sum_add(s[k], c[k], so);
+            c[k] += co;
+        }
+    }
+    if (lane < kSmallTargets) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            part_sums[wave][k][t] = s[k];
+            part_sums[wave][3 + k][t] = c[k];
+        }
+    }
+    __syncthreads();
+    // thread = component * 16 + target
+    if (threadIdx.x < 3 * kSmallTargets) {
+        const int k = threadIdx.x / kSmallTargets;
+        float sum = 0.f, comp = 0.f;
+#pragma unroll
+        for (int w = 0; w < kSmallWaves; ++w) {
+            two_sum_add(sum, comp, part_sums[w][k][t]);
+            comp += part_sums[w][3 + k][t];
+        }
+        if (i < n) {
+            // G applied once per target, in FP64 (exact for G = 1)
+            (k == 0 ? ax : (k == 1 ? ay : az))[i] =
+                G * (static_cast<double>(sum) + static_cast<double>(comp));
+        }
     }
 }
 
@@ -427,6 +497,53 @@ __global__ void refresh_pos4_kernel(const double* __restrict__ px, const double*
     if (i < n) {
         out[i] = make_float4(static_cast<float>(px[i]), static_cast<float>(py[i]),
                              static_cast<float>(pz[i]), static_cast<float>(m[i]));
+    }
+}
+
+// Up to kStageN sources a workgroup stages all of them itself; up to kSmallN 16
+// targets per workgroup give the chip more of them to run; beyond, 64 targets
+// and 16 source ranges. Measured on MI355X, us per evaluation, against four
+// ranges of 256-source tiles for all sizes (the kernel alone; in front of it a
+// staging launch, which the first line no longer needs):
+//   N = 1000 17.8 -> 6.8, 4096 58.8 -> 13.2  (all staged, 16 targets)
+//   N = 5000 71.8 -> 23.7, 8192 113 -> 37.7, 12000 161 -> 75  (16 targets;
+//     with 64 targets 36.7, 56.1, 83; at 16384 135 against 113)
+//   N = 16384 221 -> 113, 32768 396 -> 363, 65536 1533 -> 1305,
+//     131072 5668 -> 5064, 262144 20800 -> 19800  (8 ranges: 111, 387, 1363,
+//     5151, 19965; 256-source tiles instead of 64: 262144 20046)
+// At 262144 that is 3,470 G pairs/s: the issue bound of 12 full-rate
+// instructions per pair is 3,277 at the nominal 2.4 GHz.
+template <bool ZERO_EPS>
+void launch_direct_fp32(hipStream_t st, const double* px, const double* py, const double* pz,
+                        const double* m, const float4* pos, double* ax, double* ay, double* az,
+                        int n, double G, float eps2) {
+    if (n <= kSmallN) {
+        const unsigned grid = grid_for(static_cast<size_t>(n), kSmallTargets);
+        if (n <= kStageN) {
+            direct_fp32_small_kernel<ZERO_EPS, true><<<grid, kSmallWaves * kWave, 0, st>>>(
+                px, py, pz, m, pos, ax, ay, az, n, G, eps2);
+        } else {
+            direct_fp32_small_kernel<ZERO_EPS, false><<<grid, kSmallWaves * kWave, 0, st>>>(
+                px, py, pz, m, pos, ax, ay, az, n, G, eps2);
+        }
+        return;
+    }
+    constexpr int kRanges = 16, kSourceTile = 64;
+    direct_fp32_kernel<kRanges, ZERO_EPS>
+        <<<grid_for(static_cast<size_t>(n), kWave), kRanges * kWave, 0, st>>>(
+            pos, ax, ay, az, n, G, eps2, kSourceTile);
+}
+
+// The FP32 all-pairs evaluation on staged positions (unused up to kStageN).
+void launch_direct_fp32(hipStream_t st, const double* px, const double* py, const double* pz,
+                        const double* m, const float4* pos, double* ax, double* ay, double* az,
+                        int n, const NBodySimProGravity* g) {
+    const double G = g->gravitational_constant;
+    const float eps2 = static_cast<float>(g->softening_squared);
+    if (eps2 > 0.f) {
+        launch_direct_fp32<false>(st, px, py, pz, m, pos, ax, ay, az, n, G, eps2);
+    } else {
+        launch_direct_fp32<true>(st, px, py, pz, m, pos, ax, ay, az, n, G, eps2);
     }
 }
 
@@ -473,23 +590,12 @@ NBodySimProStatus direct_fp32(Engine* e, const NBodySimProGravity* g, NBodySimPr
         return N_BODY_SIM_PRO_STATUS_OK;
     }
     NBX_HIP(error, hipEventRecord(e->ev[0], e->stream));
-    NBX_TRY(refresh_pos4(e, error));
-    NBX_HIP(error, hipEventRecord(e->ev[1], e->stream));
-    // Four source ranges per target: 16 waves per SIMD at N = 262144.
-    // Measured on MI355X at that size: 3,311 Ginteractions/s, against 3,206
-    // with two ranges and 2,935 with one (one target per lane throughout;
-    // two targets per lane and one range: 2,640).
-    constexpr int S = 4;
-    const unsigned grid = grid_for(n, 256 / S);
-    const double G = g->gravitational_constant;
-    const float eps2 = static_cast<float>(g->softening_squared);
-    if (eps2 > 0.f) {
-        direct_fp32_kernel<S, false><<<grid, 256, 0, e->stream>>>(e->pos4, e->ax, e->ay, e->az,
-                                                                  static_cast<int>(n), G, eps2, 256);
-    } else {
-        direct_fp32_kernel<S, true><<<grid, 256, 0, e->stream>>>(e->pos4, e->ax, e->ay, e->az,
-                                                                 static_cast<int>(n), G, eps2, 256);
+    if (n > static_cast<size_t>(kStageN)) {
+        NBX_TRY(refresh_pos4(e, error));
     }
+    NBX_HIP(error, hipEventRecord(e->ev[1], e->stream));
+    launch_direct_fp32(e->stream, e->px, e->py, e->pz, e->m, e->pos4, e->ax, e->ay, e->az,
+                       static_cast<int>(n), g);
     NBX_HIP(error, hipGetLastError());
     NBX_HIP(error, hipEventRecord(e->ev[2], e->stream));
     NBX_HIP(error, hipEventSynchronize(e->ev[2]));
@@ -603,20 +709,13 @@ extern "C" NBodySimProStatus nbx_direct_fp32_noalloc(
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int n = static_cast<int>(count);
-    nbx::refresh_pos4_kernel<<<nbx::grid_for(count, 256), 256, 0, st>>>(
-        positions_x, positions_y, positions_z, masses, staging, n);
-    // same kernel, source split and tile as nbx_hip_direct_fp32 (identical results)
-    constexpr int S = 4;
-    const unsigned grid = nbx::grid_for(count, 256 / S);
-    const double G = gravity->gravitational_constant;
-    const float eps2 = static_cast<float>(gravity->softening_squared);
-    if (eps2 > 0.f) {
-        nbx::direct_fp32_kernel<S, false><<<grid, 256, 0, st>>>(
-            staging, accelerations_x, accelerations_y, accelerations_z, n, G, eps2, 256);
-    } else {
-        nbx::direct_fp32_kernel<S, true><<<grid, 256, 0, st>>>(
-            staging, accelerations_x, accelerations_y, accelerations_z, n, G, eps2, 256);
+    if (count > static_cast<size_t>(nbx::kStageN)) {
+        nbx::refresh_pos4_kernel<<<nbx::grid_for(count, 256), 256, 0, st>>>(
+            positions_x, positions_y, positions_z, masses, staging, n);
     }
+    // the same kernels as nbx_hip_direct_fp32 (identical results)
+    nbx::launch_direct_fp32(st, positions_x, positions_y, positions_z, masses, staging,
+                            accelerations_x, accelerations_y, accelerations_z, n, gravity);
     NBX_HIP(error, hipGetLastError());
     return N_BODY_SIM_PRO_STATUS_OK;
 }

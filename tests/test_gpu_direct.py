@@ -215,3 +215,24 @@ def test_direct_fp64_outside_the_fast_range_bit_identical(nbx, oracle, n, scale)
     q = p.copy()
     oracle.nbo_direct_openmp(C.byref(q.view), C.byref(gravity(1.0, 0.0)))
     assert np.array_equal(acc, q.acc(), equal_nan=True)
+
+
+@pytest.mark.parametrize("eps", [0.01, 0.0])
+@pytest.mark.parametrize("n", [1, 2, 15, 17, 1000, 4096, 4097, 12288, 12289, 20001])
+def test_direct_fp32_kernel_edges(nbx, oracle, n, eps):
+    """Around the workgroup's 16 or 64 targets and the sizes at which another
+    kernel takes over: the stated median of 1e-6 against the oracle's FP64 sums
+    on the FP32-rounded inputs, a maximum of 1e-4 (close pairs cancel), no NaN
+    from the own term."""
+    p = from_gen(nbx.plummer(n, seed=6)) if n > 1 else Particles(1, {"px": [0.5], "m": [1.0]})
+    acc = gpu_force(nbx, p, "hip_direct_fp32", eps)
+    q = Particles(n, {k: p.a[k].astype(np.float32).astype(np.float64)
+                      for k in ("px", "py", "pz", "m")})
+    rows = np.unique(np.linspace(0, n - 1, 400).astype(np.int64))
+    out = np.zeros((rows.size, 3))
+    oracle.nbo_direct_openmp_subset(C.byref(q.view), C.byref(gravity(1.0, eps)),
+                                    rows.ctypes.data_as(C.POINTER(C.c_int64)), rows.size,
+                                    out.ctypes.data_as(C.POINTER(C.c_double)))
+    err = rel_err_per_particle(acc[rows], out)
+    assert np.isfinite(acc).all()
+    assert np.median(err) <= 1e-6 and err.max() <= 1e-4
