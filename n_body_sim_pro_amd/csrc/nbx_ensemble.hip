@@ -3,12 +3,15 @@
 // Work decomposition. A work item is (cluster, 64*R consecutive targets of it)
 // with R = targets per lane chosen per cluster-size bucket. Items are sorted
 // by cost (targets x cluster size, longest first) and dealt round-robin to 8
-// per-XCD queues; a persistent grid (blocks_per_cu x CUs) pulls items wave by
-// wave from its XCD's queue, claiming the next item before computing the
-// current one so the atomic's latency is hidden. The source loop of an item
-// is wave-uniform (scalar loads, SGPR operands) exactly as in hip_direct_fp32,
-// with the same tile-compensated FP32 accumulation; results are identical
-// for any R or blocks-per-CU choice (only source_tile moves the fold points).
+// per-XCD queues; a persistent grid (blocks_per_cu x CUs) pulls items workgroup
+// by workgroup from its XCD's queue, claiming the next item before computing the
+// current one so the atomic's latency is hidden. A workgroup's four waves split
+// the cluster's sources, which keeps an item short (the largest clusters' items
+// set the time of a small ensemble) and four waves on the same targets. The
+// source loop is wave-uniform (scalar loads, SGPR operands) exactly as in
+// hip_direct_fp32, with the same tile-compensated FP32 accumulation; results
+// are identical for any R or blocks-per-CU choice (only source_tile moves the
+// fold points).
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -71,13 +74,22 @@ __device__ inline void kb_add(float& s, float& c, float v) {
     c += e;
 }
 
+// A workgroup's four waves share an item's targets: each takes a quarter of
+// the cluster's sources (a multiple of four, so the split depends on the
+// cluster's size alone) and the sums meet in LDS in source order.
+constexpr int kSplit = kThreads / kWave;
+
 // ZERO_EPS: unsoftened sums; the self pair (r2 == 0) and coincident pairs
 // contribute nothing instead of rsq(0) = inf times 0 = NaN.
 template <int R, bool ZERO_EPS>
 __device__ inline void tile_force(const float4* __restrict__ pos, double* __restrict__ ax,
                                   double* __restrict__ ay, double* __restrict__ az,
-                                  const WorkItem& w, int lane, float G, float eps2, int tile) {
+                                  const WorkItem& w, int lane, int part, float* fold, float G,
+                                  float eps2, int tile) {
     const int end = w.off + w.n;
+    const int per = (w.n + 4 * kSplit - 1) / (4 * kSplit) * 4;
+    const int jb = min(end, w.off + part * per);
+    const int je = min(end, w.off + (part + 1) * per);
     float xi[R], yi[R], zi[R], sx[R], sy[R], sz[R], cx[R], cy[R], cz[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -88,8 +100,8 @@ __device__ inline void tile_force(const float4* __restrict__ pos, double* __rest
         zi[r] = p.z;
         sx[r] = sy[r] = sz[r] = cx[r] = cy[r] = cz[r] = 0.f;
     }
-    for (int j0 = w.off; j0 < end; j0 += tile) {
-        const int j1 = (j0 + tile) < end ? (j0 + tile) : end;
+    for (int j0 = jb; j0 < je; j0 += tile) {
+        const int j1 = (j0 + tile) < je ? (j0 + tile) : je;
         float px[R], py[R], pz[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -121,8 +133,36 @@ __device__ inline void tile_force(const float4* __restrict__ pos, double* __rest
             kb_add(sz[r], cz[r], pz[r]);
         }
     }
+    // fold[(part - 1) * 6 + field][r * 64 + lane]
+    constexpr int kRow = R * kWave;
+    if (part > 0) {
+        float* f = fold + (part - 1) * 6 * kRow + lane;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            f[0 * kRow + r * kWave] = sx[r];
+            f[1 * kRow + r * kWave] = sy[r];
+            f[2 * kRow + r * kWave] = sz[r];
+            f[3 * kRow + r * kWave] = cx[r];
+            f[4 * kRow + r * kWave] = cy[r];
+            f[5 * kRow + r * kWave] = cz[r];
+        }
+    }
+    __syncthreads();
+    if (part > 0) {
+        return;
+    }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
+#pragma unroll
+        for (int k = 0; k < kSplit - 1; ++k) {
+            const float* f = fold + k * 6 * kRow + r * kWave + lane;
+            kb_add(sx[r], cx[r], f[0 * kRow]);
+            kb_add(sy[r], cy[r], f[1 * kRow]);
+            kb_add(sz[r], cz[r], f[2 * kRow]);
+            cx[r] += f[3 * kRow];
+            cy[r] += f[4 * kRow];
+            cz[r] += f[5 * kRow];
+        }
         const int i = w.off + w.start + r * kWave + lane;
         if (i < end) {
             ax[i] = static_cast<double>(G) * (static_cast<double>(sx[r]) + static_cast<double>(cx[r]));
@@ -132,34 +172,43 @@ __device__ inline void tile_force(const float4* __restrict__ pos, double* __rest
     }
 }
 
-// Persistent launch: waves pull items from their XCD's queue until it is empty.
-template <bool ZERO_EPS>
+// Persistent launch: workgroups pull items from their XCD's queue until it is
+// empty. RMAX: the most targets per lane of any item (one per lane takes 38
+// VGPRs and runs at full residency, four 120).
+template <bool ZERO_EPS, int RMAX>
 __global__ __launch_bounds__(kThreads) void ens_force_kernel(
     const float4* __restrict__ pos, double* __restrict__ ax, double* __restrict__ ay,
     double* __restrict__ az, const WorkItem* __restrict__ items, int nitems,
     unsigned* __restrict__ queues, float G, float eps2, int tile) {
+    __shared__ float fold[(kSplit - 1) * 6 * RMAX * kWave];
+    __shared__ unsigned claim;
     const int lane = threadIdx.x & (kWave - 1);
+    const int part = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
     const int qid = blockIdx.x % kQueues;
     unsigned* q = queues + qid;
-    unsigned k = 0;
-    if (lane == 0) {
-        k = atomicAdd(q, 1u);
+    if (threadIdx.x == 0) {
+        claim = atomicAdd(q, 1u);
     }
-    int item = __builtin_amdgcn_readfirstlane(static_cast<int>(k)) * kQueues + qid;
+    __syncthreads();
+    int item = __builtin_amdgcn_readfirstlane(static_cast<int>(claim)) * kQueues + qid;
     while (item < nitems) {
         unsigned kn = 0;
-        if (lane == 0) {
+        if (threadIdx.x == 0) {
             kn = atomicAdd(q, 1u);  // claim the next item before computing this one
         }
         const WorkItem w = items[item];
-        if (w.r == 4) {
-            tile_force<4, ZERO_EPS>(pos, ax, ay, az, w, lane, G, eps2, tile);
-        } else if (w.r == 2) {
-            tile_force<2, ZERO_EPS>(pos, ax, ay, az, w, lane, G, eps2, tile);
+        if (RMAX >= 4 && w.r == 4) {
+            tile_force<4, ZERO_EPS>(pos, ax, ay, az, w, lane, part, fold, G, eps2, tile);
+        } else if (RMAX >= 2 && w.r == 2) {
+            tile_force<2, ZERO_EPS>(pos, ax, ay, az, w, lane, part, fold, G, eps2, tile);
         } else {
-            tile_force<1, ZERO_EPS>(pos, ax, ay, az, w, lane, G, eps2, tile);
+            tile_force<1, ZERO_EPS>(pos, ax, ay, az, w, lane, part, fold, G, eps2, tile);
         }
-        item = __builtin_amdgcn_readfirstlane(static_cast<int>(kn)) * kQueues + qid;
+        if (threadIdx.x == 0) {
+            claim = kn;
+        }
+        __syncthreads();   // the next claim written, this item's sums read
+        item = __builtin_amdgcn_readfirstlane(static_cast<int>(claim)) * kQueues + qid;
     }
 }
 
@@ -182,6 +231,38 @@ __global__ void ens_kick_drift_kernel(double* __restrict__ px, double* __restric
         const double nvx = vx[i] + ax[i] * half;
         const double nvy = vy[i] + ay[i] * half;
         const double nvz = vz[i] + az[i] * half;
+        vx[i] = nvx;
+        vy[i] = nvy;
+        vz[i] = nvz;
+        const double x = px[i] + nvx * dt;
+        const double y = py[i] + nvy * dt;
+        const double z = pz[i] + nvz * dt;
+        px[i] = x;
+        py[i] = y;
+        pz[i] = z;
+        pos4[i] = make_float4(static_cast<float>(x), static_cast<float>(y), static_cast<float>(z),
+                              static_cast<float>(m[i]));
+    }
+}
+
+// The kick that ends a step and the kick and drift that begin the next, with
+// the same two roundings of the velocity (72 bytes a particle less than the
+// two kernels: 49 us a step at 3.9M particles).
+__global__ void ens_kick_kick_drift_kernel(double* __restrict__ px, double* __restrict__ py,
+                                           double* __restrict__ pz, double* __restrict__ vx,
+                                           double* __restrict__ vy, double* __restrict__ vz,
+                                           const double* __restrict__ ax,
+                                           const double* __restrict__ ay,
+                                           const double* __restrict__ az,
+                                           const double* __restrict__ m,
+                                           float4* __restrict__ pos4, int n, double half,
+                                           double dt) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) {
+        const double hx = ax[i] * half, hy = ay[i] * half, hz = az[i] * half;
+        const double nvx = (vx[i] + hx) + hx;
+        const double nvy = (vy[i] + hy) + hy;
+        const double nvz = (vz[i] + hz) + hz;
         vx[i] = nvx;
         vy[i] = nvy;
         vz[i] = nvz;
@@ -289,10 +370,16 @@ int bucket_of(uint32_t n) {
 }
 
 void default_tile(NBXTileConfig* t) {
+    // One target per lane at full residency. Measured on MI355X, ms per step
+    // of 4,096 / 512 / 64 clusters of 64 to 4,096 particles, 8 blocks per CU:
+    // one target per lane 2.55 / 0.461 / 0.122, two 2.66 / 0.491 / 0.147, one,
+    // two and four by size 2.70 / 0.573 / 0.208; with 4 blocks per CU 3.16 /
+    // 0.517 / 0.132. (A wave per item instead of a workgroup, with one, two
+    // and four targets by size and 4 blocks per CU: 3.82 / 1.22 / 0.69.)
     for (int b = 0; b < kBuckets; ++b) {
-        t->targets_per_lane[b] = b < 2 ? 1 : (b < 5 ? 2 : 4);
+        t->targets_per_lane[b] = 1;
     }
-    t->blocks_per_cu = 4;
+    t->blocks_per_cu = 8;
     t->source_tile = 256;
 }
 
@@ -340,14 +427,17 @@ NBodySimProStatus upload_items(Ensemble& s, const std::vector<WorkItem>& v,
 void launch_force(Ensemble& s, float G, float eps2) {
     ens_reset_kernel<<<1, kQueues, 0, s.stream>>>(s.queue);
     const unsigned grid = static_cast<unsigned>(s.cu_count * s.tile.blocks_per_cu);
+    auto go = [&](auto kernel) {
+        kernel<<<grid, kThreads, 0, s.stream>>>(s.pos4, s.ax, s.ay, s.az, s.items.as<WorkItem>(),
+                                                s.nitems, s.queue, G, eps2, s.tile.source_tile);
+    };
+    const int widest = *std::max_element(s.tile.targets_per_lane, s.tile.targets_per_lane + kBuckets);
     if (eps2 > 0.f) {
-        ens_force_kernel<false><<<grid, kThreads, 0, s.stream>>>(
-            s.pos4, s.ax, s.ay, s.az, s.items.as<WorkItem>(), s.nitems, s.queue, G, eps2,
-            s.tile.source_tile);
+        widest == 1 ? go(ens_force_kernel<false, 1>)
+                    : (widest == 2 ? go(ens_force_kernel<false, 2>) : go(ens_force_kernel<false, 4>));
     } else {
-        ens_force_kernel<true><<<grid, kThreads, 0, s.stream>>>(
-            s.pos4, s.ax, s.ay, s.az, s.items.as<WorkItem>(), s.nitems, s.queue, G, eps2,
-            s.tile.source_tile);
+        widest == 1 ? go(ens_force_kernel<true, 1>)
+                    : (widest == 2 ? go(ens_force_kernel<true, 2>) : go(ens_force_kernel<true, 4>));
     }
 }
 
@@ -364,10 +454,11 @@ void enqueue_steps(Ensemble& s, float G, float eps2, double dt, int steps) {
     const unsigned g = grid_for(s.total, kThreads);
     const double half = 0.5 * dt;
     for (int k = 0; k < steps; ++k) {
-        ens_kick_drift_kernel<<<g, kThreads, 0, s.stream>>>(s.px, s.py, s.pz, s.vx, s.vy, s.vz,
-                                                            s.ax, s.ay, s.az, s.m, s.pos4, n, half,
-                                                            dt);
+        (k == 0 ? ens_kick_drift_kernel : ens_kick_kick_drift_kernel)<<<g, kThreads, 0, s.stream>>>(
+            s.px, s.py, s.pz, s.vx, s.vy, s.vz, s.ax, s.ay, s.az, s.m, s.pos4, n, half, dt);
         launch_force(s, G, eps2);
+    }
+    if (steps > 0) {
         ens_kick_kernel<<<g, kThreads, 0, s.stream>>>(s.vx, s.vy, s.vz, s.ax, s.ay, s.az, n, half);
     }
 }

@@ -138,3 +138,30 @@ def test_autotune_returns_valid_cached_config(nbx, small_ensemble, tmp_path):
         assert rep2["targets_per_lane"] == rep["targets_per_lane"]
     err = rel_err_per_particle(acc, ref)
     assert np.median(err) < 1e-6
+
+
+@pytest.mark.parametrize("eps", [0.01, 0.0])
+@pytest.mark.parametrize("targets_per_lane", [1, 2, 4])
+def test_cluster_sizes_around_the_source_split(nbx, oracle, targets_per_lane, eps):
+    """Clusters from one particle up, around the waves' quarters of the sources
+    (multiples of four), the 64 targets of a wave and the source tile: the
+    same bars as above, on the FP32-rounded inputs (close pairs cancel)."""
+    sizes = np.array([1, 2, 3, 4, 5, 15, 16, 17, 63, 64, 65, 255, 256, 257, 1023, 1029],
+                     dtype=np.uint32)
+    d = nbx.ensemble_clusters(sizes, seed=3)
+    d = {k: v.astype(np.float32).astype(np.float64) for k, v in d.items()}
+    with nbx.Ensemble(sizes) as ens:
+        ens.set_tile([targets_per_lane] * 8, 8, 64)
+        ens.upload(d["pos"], d["vel"], d["m"])
+        ens.force(eps=eps)
+        acc = ens.download()["acc"]
+    assert np.isfinite(acc).all()
+    errs, off = [], 0
+    for n in sizes:
+        p = cluster_particles(d, off, int(n))
+        oracle.nbo_direct_openmp(C.byref(p.view), C.byref(gravity(1.0, eps)))
+        errs.append(rel_err_per_particle(acc[off:off + n], p.acc()))
+        off += int(n)
+    err = np.concatenate(errs)
+    assert np.median(err) <= 1e-6
+    assert err.max() < 1e-4
