@@ -107,6 +107,40 @@ def test_training_lowers_loss(learned):
     assert hist[-1] < hist[0]
 
 
+@pytest.mark.parametrize("n,batch", [(1, 1), (17, 64), (240, 240), (300, 300), (1024, 64),
+                                     (4160, 4160)])
+def test_training_steps(learned, n, batch):
+    """Batches of 4 (the fewest), 16, 20 and 260 waves: one Adam step from the
+    gradients' own values, the loss of the weights it left, and an epoch's mean
+    loss. Tolerances: a loss or gradient is a sum in another sample order over
+    at most 260 waves and 6 exchanges, 270 x 6e-8 = 1.6e-5 either side; Adam's
+    first step is lr g / (|g| + eps), right to some FP32 roundings."""
+    p, mean, std = _random_model(21)
+    f = _feats(n, 22)
+    t = np.random.default_rng(23).normal(0, 1, (n, 3)).astype(np.float32)
+    lr = 1e-3
+    one_batch = batch >= n
+    with learned.Mlp() as m, learned.Mlp() as two:
+        for k in (m, two):
+            k.set_params(p, mean, std, 1.0)
+            k.load_dataset(f, t)
+        g, loss = m.gradients(f, t)
+        if one_batch:
+            hist = m.train(1, batch, lr, 5)
+            q = m.get_params()["params"]
+            big = np.abs(g) > 1e-3 * np.abs(g).max()
+            step = lr * g / (np.abs(g) + 1e-8)
+            assert np.all(np.abs(q - (p - step))[big] <= (1e-5 * lr + 1.2e-7 * np.abs(p))[big])
+            assert hist[0] == pytest.approx(loss, rel=4e-5)
+            _, after = m.gradients(f, t)
+            hist2 = two.train(2, batch, lr, 5)
+            assert hist2[0] == hist[0]
+            assert hist2[1] == pytest.approx(after, rel=4e-5)
+        else:
+            hist = m.train(2, batch, 1e-12, 5)
+            assert hist == pytest.approx([loss, loss], rel=4e-5)
+
+
 # ---- feature walk: numpy restatement over the exported tree ----
 
 def _walk_features_numpy(rows, perm, pos32, m32, root_h, theta, eps2):
