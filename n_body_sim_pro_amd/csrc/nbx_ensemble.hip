@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "nbx_ensemble.h"
+#include "nbx_exact.h"
 #include "nbx_internal.h"
 
 namespace nbx {
@@ -315,17 +316,18 @@ __global__ __launch_bounds__(kWave) void ens_energy_kernel(
     const int lane = threadIdx.x;
     const int end = w.off + w.n;
     const int i = w.off + w.start + lane;
+    const int ic = min(i, end - 1);
+    const double x = px[ic], y = py[ic], z = pz[ic], mi = m[ic];
     double ke = 0.0, pot = 0.0;
     if (i < end) {
-        const double mi = m[i];
         ke = 0.5 * mi * (vx[i] * vx[i] + vy[i] * vy[i] + vz[i] * vz[i]);
-        const double x = px[i], y = py[i], z = pz[i];
-        for (int j = i + 1; j < end; ++j) {
-            const double dx = px[j] - x;
-            const double dy = py[j] - y;
-            const double dz = pz[j] - z;
-            const double d = sqrt(dx * dx + dy * dy + dz * dz + eps2);
-            pot += mi * m[j] / d;
+    }
+    const int first = w.off + w.start;
+    for (int j0 = first; j0 < end; j0 += kPotSources) {
+        if (j0 < first + kWave || j0 + kPotSources > end) {
+            pot += pot_unit<true>(px, py, pz, m, end, j0, i, x, y, z, mi, eps2);
+        } else {
+            pot += pot_unit<false>(px, py, pz, m, end, j0, i, x, y, z, mi, eps2);
         }
     }
     __shared__ double s[2][kWave];

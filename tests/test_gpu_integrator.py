@@ -57,6 +57,40 @@ def test_diagnostics_closed_forms(nbx):
         assert e.diagnostics(eps=0.0)["potential_energy"] == pytest.approx(-1.0, abs=1e-15)
 
 
+@pytest.mark.parametrize("n,eps,scale", [
+    (1, 0.01, 1.0), (2, 0.01, 1.0), (16, 0.0, 1.0), (17, 0.01, 1.0), (64, 0.01, 1.0),
+    (65, 0.0, 1.0), (129, 0.01, 1.0), (1000, 0.01, 1.0),
+    (4099, 0.01, 1.0),     # more units than waves
+    (70, 0.0, 1e-158),     # squared distances below the normal range
+    (70, 0.0, 1e160),      # and past the largest number
+])
+def test_potential_units(nbx, n, eps, scale):
+    """Edges of the potential's 64-target by 16-source units. All terms have one
+    sign; each is right to 3 roundings and passes at most 16 + 24 + 8 + 8
+    additions: 60 x 1.1e-16."""
+    rng = np.random.default_rng(n)
+    q = rng.normal(0, 1, (3, n)) * scale
+    m = rng.uniform(0.5, 1.5, n)
+    with np.errstate(over="ignore"):
+        u = np.longdouble(0)
+        for i in range(n - 1):
+            d = q[:, i + 1:] - q[:, i:i + 1]
+            r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] + eps * eps
+            u += np.sum((m[i] * m[i + 1:] / np.sqrt(r2)).astype(np.longdouble))
+    p = Particles(n, {"px": q[0], "py": q[1], "pz": q[2], "m": m})
+    with nbx.Engine(n) as e:
+        e.upload_view(p.view)
+        got = e.diagnostics(eps=eps)["potential_energy"]
+    assert abs(got + float(u)) <= 7e-15 * abs(float(u))
+
+
+def test_potential_of_coincident_pair(nbx):
+    p = Particles(40, {"px": [*range(39), 7], "py": [0] * 40, "pz": [0] * 40, "m": [1.0] * 40})
+    with nbx.Engine(40) as e:
+        e.upload_view(p.view)
+        assert e.diagnostics(eps=0.0)["potential_energy"] == -np.inf
+
+
 @pytest.mark.parametrize("integrator", [1, 2])
 def test_two_body_orbit_regression(nbx, integrator):
     """two_body_test.c:57-184: 8 orbits x 500 steps, eps=0."""
