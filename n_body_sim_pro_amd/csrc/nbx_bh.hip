@@ -1930,8 +1930,8 @@ __global__ __launch_bounds__(kThreads) void walk_f32_kernel(
     }
 }
 
-// Group walk (FP32). A wave takes 64 Q consecutive tree positions (Q per
-// lane) as one group and walks the tree once for the group's bounding box: a
+// Group walk (FP32). A wave, or in small systems a team of waves, takes 64
+// consecutive tree positions as one group and walks the tree once for the group's bounding box: a
 // cell is accepted when the reference's test (d^2 > 0 and 4h^2 < theta^2 d^2)
 // holds for the box distance d, which implies it holds for every member, so
 // each member's interaction set refines its reference set. The walk runs on
@@ -1992,28 +1992,48 @@ __device__ inline bool run_compact(const uint64_t* __restrict__ w, const uint64_
     const int first = a - kRunStride * kl - __popcll(fine >> 32);
     return last - first + 1 <= kGroupCell;
 }
-#ifndef NBX_GROUP_THREADS
-#define NBX_GROUP_THREADS 64
-#endif
-// Groups are dealt to the XCDs in chunks of kGroupChunk consecutive groups
+// Groups are dealt to the XCDs in chunks of 2^chunk_log consecutive groups
 // (chunk c to XCD c mod 8, each XCD's chunks in tree order): every XCD gets a
 // share of the dense and the sparse regions, and a chunk's waves still share
 // cell records in their XCD's L2. (Measured on MI355X, two-galaxy: with each
 // XCD on one contiguous eighth of the groups, the XCDs finished between 630
 // and 846 us at 1M and between 12.8 and 16.2 ms at 10M, theta = 0.5; walk
 // 0.78 / 16.4 ms. Chunks of 8, 32, 128 groups: 0.80 / 14.4, 0.80 / 14.2,
-// 0.78 / 14.2 ms.)
-constexpr int kGroupChunk = 128;
+// 0.78 / 14.2 ms. Teams of four, Plummer, chunks of 32 and 128: 86 and 111 us
+// at 10,000, where 128 leave six XCDs without a group, 102 and 135 at 30,000.)
+constexpr int kChunkLog = 7;        // a wave a group
+constexpr int kTeamChunkLog = 5;    // a team of waves a group
 
-__device__ inline int group_of_block(int b) {
+__device__ inline int group_of_block(int b, int chunk_log) {
     const int slot = b / kXcds;   // workgroup b runs on XCD b mod 8
-    return ((slot / kGroupChunk) * kXcds + b % kXcds) * kGroupChunk + slot % kGroupChunk;
+    return (((slot >> chunk_log) * kXcds + b % kXcds) << chunk_log) +
+           (slot & ((1 << chunk_log) - 1));
 }
 
-// One wave per workgroup: a wave's LDS is released as soon as it finishes
-// (waves of one region take very different times; measured on MI355X, 1M
-// particles: 1.45 ms with one wave per workgroup, 1.66 ms with four).
-constexpr int kGroupThreads = NBX_GROUP_THREADS;
+// W waves walk one group, a workgroup. One wave, in a large system: its LDS is
+// released as soon as it finishes (waves of one region take very different
+// times; measured on MI355X, 1M particles: 1.45 ms with one group per
+// workgroup, 1.66 ms with four). In a small system the chip is idle and the
+// time is that of the longest group, a chain of steps (pop, record load, test,
+// push) and of list entries: there two or four waves take one group. They pop
+// from one common stack, 64 W cells a step with two barriers, stage and
+// evaluate their own cells' lists, and add their sums at the end. A group in
+// more than kTeamRanges ranges gives each range to one wave instead. The lists
+// are the same for every W; only the order of the FP32 sums differs.
+// (Measured on MI355X, walk with its events, theta = 0.7, two-galaxy / Plummer,
+// W = 1, 2, 4: 10,000 particles 92, 74, 63 / 153, 110, 87 us; 100,000: 328, 186,
+// 144 / 275, 241, 207; 262,144, W = 2, 4: 270, 288 / 321, 352; 500,000, W = 1, 2:
+// 450, 435 / 535, 520; 1M: 778, 752 / 862, 916 us. Eight waves: 75 / 82 us at
+// 10,000. Ranges up to which the team stays together, 1, 3, 7: 74, 69, 91 us for
+// two galaxies of 10,000, 98, 95, 138 for 30,000.)
+constexpr int kTeamRanges = 3;
+
+// Waves per group for `groups` groups.
+inline int walk_team(size_t groups, int cu_count) {
+    const size_t cus = static_cast<size_t>(cu_count);
+    return groups <= 8 * cus ? 4 : (groups <= 32 * cus ? 2 : 1);
+}
+
 // One query per lane in the group walk (measured on MI355X: two per lane, a
 // group of 128, is 7% slower at 10M particles and 16% slower at 1M).
 
@@ -2060,8 +2080,8 @@ __device__ inline void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <bool FEATURES>
-__global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
+template <bool FEATURES, int W>
+__global__ __launch_bounds__(W * kWave) void group_walk_kernel(
     const unsigned* __restrict__ flags, int* __restrict__ deferred,
     const GroupNode* __restrict__ gnode, const float4* __restrict__ s4,
     const uint32_t* __restrict__ tperm, const uint64_t* __restrict__ tword,
@@ -2069,12 +2089,13 @@ __global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
     double* __restrict__ ax, double* __restrict__ ay,
     double* __restrict__ az, unsigned long long* __restrict__ counters,
     float* __restrict__ features, const float4* __restrict__ gquad,
-    int max_walks, bool member_test) {
-    constexpr int kWaves = kGroupThreads / kWave;
+    int max_walks, bool member_test, int chunk_log) {
+    constexpr int kWaves = W;
     // per wave: pending cells; staged cells (COM, mass; with FEATURES the
     // quadrupole record); staged leaves (tree position, then position and
     // mass); whether each lane's own leaf was staged; pending sub-ranges
-    __shared__ int stack_all[kWaves][kGroupStack];
+    __shared__ int pending_all[kWaves * (kGroupStack + kGroupLeaves + 1)];
+    __shared__ int pushed_all[kWaves];
     // FEATURES stages fewer cells per flush: their quadrupole records take LDS.
     // (Measured on MI355X, learned walk at 10M: 96 or 128 staged cells, 8.9 or
     // 10.4 KB of LDS, are 4% and 17% slower; six waves per SIMD through 80
@@ -2084,7 +2105,8 @@ __global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
     // FEATURES the two quadrupole float4), so one LDS pointer walks the list.
     constexpr int kList = FEATURES ? kGroupList / 2 : kGroupList;
     static_assert(kList >= kWave, "a step stages up to one accepted cell per lane");
-    static_assert(kGroupLeaves >= kWave, "the member test stages a step's candidates in lleaf");
+    constexpr int kTests = 4;   // candidates of the member test side by side
+    static_assert(kGroupLeaves >= kWave + kTests, "the member test stages a step's candidates in lleaf");
     // The plain walk evaluates its staged lists four entries per loop trip
     // (LDS loads run ahead, one address update per four; same summation
     // order). Measured on MI355X against one per trip: walk 7% faster at 1M
@@ -2093,20 +2115,18 @@ __global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
     constexpr int kEvalUnroll = FEATURES ? 1 : 4;
     constexpr int kCellWords = FEATURES ? 3 : 1;
     __shared__ float4 lcell_all[kWaves][kList * kCellWords];
-    __shared__ int ltag_all[kWaves][kGroupLeaves];
     __shared__ float4 lleaf_all[kWaves][kGroupLeaves];
     __shared__ unsigned char selfhit_all[kWaves][kWave];
     __shared__ int2 ranges_all[kWaves][kRangeStack];
     const int lane = threadIdx.x & (kWave - 1);
-    const int wid = threadIdx.x / kWave;
-    int* stack = stack_all[wid];
+    const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
     float4* lcell = lcell_all[wid];
-    int* ltag = ltag_all[wid];
+    const int ltag_at = kWaves * kGroupStack + wid * (kGroupLeaves + 1);
+    int* ltag = pending_all + ltag_at;
     float4* lleaf = lleaf_all[wid];
     unsigned char* selfhit = selfhit_all[wid];
     int2* ranges = ranges_all[wid];
-    static_assert(kWaves == 1, "one group per workgroup");
-    const int wave = group_of_block(static_cast<int>(blockIdx.x));
+    const int wave = group_of_block(static_cast<int>(blockIdx.x), chunk_log);
     const int t0 = wave * kWave;
     if (t0 >= n || build_failed(flags)) {
         return;   // whole wave beyond the particles, or no tree to walk
@@ -2123,7 +2143,7 @@ __global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
     // group: box acceptance against the members' bounding box. Returns false,
     // with the members' sums cleared, when the pending cells would overflow
     // the stack.
-    auto shared_walk = [&](int a, int b) -> bool {
+    auto shared_walk = [&](int a, int b, bool team) -> bool {
         const bool member = valid && t >= a && t <= b;
         const float bx0 = wave_min(member ? qx : 3.0e38f);
         const float by0 = wave_min(member ? qy : 3.0e38f);
@@ -2133,12 +2153,22 @@ __global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
         const float bz1 = wave_max(member ? qz : -3.0e38f);
         int ccnt = 0, lcnt = 0;            // staged cells, leaves (wave-uniform)
         unsigned ncell = 0, nleaf = 0;     // evaluated per member (wave-uniform)
+        // a team's pending cells are its waves' stacks put together
+        const int stack_at = team ? 0 : wid * kGroupStack;
+        const int room_for = team ? kWaves * kGroupStack : kGroupStack;
+        const int lanes = team ? kWaves * kWave : kWave;
+        int* stack = pending_all + stack_at;
         selfhit[lane] = 0;
         // evaluate the staged lists for every member
         auto flush = [&]() {
             wave_lds_fence();
             for (int e = lane; e < lcnt; e += kWave) {
-                lleaf[e] = s4[ltag[e]];
+                const int tag = ltag[e];
+                lleaf[e] = s4[tag];
+                const unsigned rel = static_cast<unsigned>(tag - t0);
+                if (rel < static_cast<unsigned>(kWave)) {
+                    selfhit[rel] = 1;
+                }
             }
             wave_lds_fence();
             if (member) {
@@ -2183,13 +2213,17 @@ __global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
         };
         int sp = 0;   // pending cells (wave-uniform); the root is level index 0
         if (n > 1) {
-            if (lane == 0) {
+            if (lane == 0 && (!team || wid == 0)) {
                 stack[0] = 0;
             }
             sp = 1;
         }
         bool overflow = false;
-        wave_lds_fence();
+        if (team) {
+            lds_barrier();
+        } else {
+            wave_lds_fence();
+        }
         while (sp > 0) {
             // (sp goes through readfirstlane so the compiler keeps it, and
             // every test on it, in scalar registers; with the unmasked record
@@ -2199,11 +2233,12 @@ __global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
             // pop at most 64 cells, and few enough that their children (8
             // each) fit: a wide level then spreads over more steps instead
             // of overflowing
-            const int room = (kGroupStack - sp) / 8;
-            const int cap = room > 1 ? (room < kWave ? room : kWave) : 1;
+            const int room = (room_for - sp) / 8;
+            const int cap = room > 1 ? (room < lanes ? room : lanes) : 1;
             const int take = sp < cap ? sp : cap;
-            const bool act = lane < take;
-            const int ref = act ? stack[sp - take + lane] : 0;
+            const int pop = team ? lane * kWaves + wid : lane;
+            const bool act = pop < take;
+            const int ref = act ? stack[sp - take + pop] : 0;
             sp = __builtin_amdgcn_readfirstlane(sp - take);
             wave_lds_fence();   // pops read before pushes reuse their slots
             // Every lane loads a record (the lanes past `take` the root's) and
@@ -2249,18 +2284,28 @@ __global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
                     wave_lds_fence();
                     const int nc = static_cast<int>(__popcll(pending));
                     uint64_t pass = 0;   // bit j: every member accepts candidate j
-                    for (int j = 0; j < nc; ++j) {
-                        const float4 cj = lleaf[j];
-                        const float dx = cj.x - qx;
-                        const float dy = cj.y - qy;
-                        const float dz = cj.z - qz;
-                        const float dj2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                        // (each comparison balloted on its own: its lane
-                        // mask is the ballot, with no VALU round trip)
-                        const uint64_t ok = __builtin_amdgcn_ballot_w64(dj2 > 0.f) &
-                                            __builtin_amdgcn_ballot_w64(cj.w < theta2 * dj2);
-                        if ((members & ~ok) == 0) {
-                            pass |= 1ull << j;
+                    for (int j = 0; j < nc; j += kTests) {
+                        float4 cj[kTests];
+#pragma unroll
+                        for (int u = 0; u < kTests; ++u) {
+                            cj[u] = lleaf[j + u];   // (past the last: not looked up)
+                        }
+                        uint64_t open_for[kTests];
+#pragma unroll
+                        for (int u = 0; u < kTests; ++u) {
+                            const float dx = cj[u].x - qx;
+                            const float dy = cj[u].y - qy;
+                            const float dz = cj[u].z - qz;
+                            const float dj2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                            // (each comparison balloted on its own: its lane
+                            // mask is the ballot, with no VALU round trip)
+                            const uint64_t ok = __builtin_amdgcn_ballot_w64(dj2 > 0.f) &
+                                                __builtin_amdgcn_ballot_w64(cj[u].w < theta2 * dj2);
+                            open_for[u] = members & ~ok;
+                        }
+#pragma unroll
+                        for (int u = 0; u < kTests; ++u) {
+                            pass |= open_for[u] == 0 ? 1ull << (j + u) : 0ull;
                         }
                     }
                     wave_lds_fence();   // candidates read before the buffer is reused
@@ -2284,39 +2329,107 @@ __global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
             // (at most 64 new leaves and 64 new cells per round)
             const bool open = act && !accepted;
             const int kid[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+            if (FEATURES) {
 #pragma unroll
-            for (int o = 0; o < 8; ++o) {
-                const int ch = open ? kid[o] : -1;
-                const uint64_t lb = __ballot(ch < -1);
-                const uint64_t ib = __ballot(ch >= 0);
-                if (lb != 0) {
-                    if (lcnt > kGroupLeaves - kWave) {
-                        flush();
-                    }
-                    if (ch < -1) {
-                        const int tag = -ch - 2;
-                        ltag[lcnt + static_cast<int>(lanes_below(lb))] = tag;
-                        const unsigned rel = static_cast<unsigned>(tag - t0);
-                        if (rel < static_cast<unsigned>(kWave)) {
-                            selfhit[rel] = 1;
+                for (int o = 0; o < 8; ++o) {
+                    const int ch = open ? kid[o] : -1;
+                    const uint64_t lb = __ballot(ch < -1);
+                    const uint64_t ib = __ballot(ch >= 0);
+                    if (lb != 0) {
+                        if (lcnt > kGroupLeaves - kWave) {
+                            flush();
                         }
+                        if (ch < -1) {
+                            ltag[lcnt + static_cast<int>(lanes_below(lb))] = -ch - 2;
+                        }
+                        lcnt += static_cast<int>(__popcll(lb));
                     }
-                    lcnt += static_cast<int>(__popcll(lb));
+                    const int np = static_cast<int>(__popcll(ib));
+                    if (sp + np > room_for) {
+                        overflow = true;
+                    } else if (np != 0) {
+                        if (ch >= 0) {
+                            stack[sp + static_cast<int>(lanes_below(ib))] = ch;
+                        }
+                        sp = __builtin_amdgcn_readfirstlane(sp + np);
+                    }
                 }
-                const int np = static_cast<int>(__popcll(ib));
-                if (sp + np > kGroupStack) {
-                    overflow = true;
-                } else if (np != 0) {
-                    if (ch >= 0) {
-                        stack[sp + static_cast<int>(lanes_below(ib))] = ch;
+            } else {
+                uint64_t lb[8], ib[8];
+                int leaves = 0, cells = 0;
+#pragma unroll
+                for (int o = 0; o < 8; ++o) {
+                    const int ch = open ? kid[o] : -1;
+                    lb[o] = __builtin_amdgcn_ballot_w64(ch < -1);
+                    ib[o] = __builtin_amdgcn_ballot_w64(ch >= 0);
+                    leaves += static_cast<int>(__popcll(lb[o]));
+                    cells += static_cast<int>(__popcll(ib[o]));
+                }
+                int at = sp, all = cells;
+                if (team) {
+                    // room on the common stack, in the waves' order; no wave
+                    // pushes before all have popped
+                    if (lane == 0) {
+                        pushed_all[wid] = cells;
                     }
-                    sp = __builtin_amdgcn_readfirstlane(sp + np);
+                    lds_barrier();
+                    all = 0;
+#pragma unroll
+                    for (int w = 0; w < kWaves; ++w) {
+                        const int theirs = __builtin_amdgcn_readfirstlane(pushed_all[w]);
+                        at += w < wid ? theirs : 0;
+                        all += theirs;
+                    }
+                }
+                overflow = sp + all > room_for;
+                if (lcnt + leaves > kGroupLeaves) {
+                    flush();
+                }
+                if (leaves <= kGroupLeaves && !overflow) {
+                    sp += all;
+                    at += stack_at;
+#pragma unroll
+                    for (int o = 0; o < 8; ++o) {
+                        const int ch = open ? kid[o] : -1;
+                        const int cell = at + static_cast<int>(lanes_below(ib[o]));
+                        const int leaf = ltag_at + lcnt + static_cast<int>(lanes_below(lb[o]));
+                        const int slot = ch >= 0 ? cell : (ch < -1 ? leaf : ltag_at + kGroupLeaves);
+                        pending_all[slot] = ch >= 0 ? ch : -ch - 2;
+                        at += static_cast<int>(__popcll(ib[o]));
+                        lcnt += static_cast<int>(__popcll(lb[o]));
+                    }
+                } else if (!overflow) {
+                    // more leaves than the list holds: an octant at a time
+                    sp += all;
+                    at += stack_at;
+#pragma unroll
+                    for (int o = 0; o < 8; ++o) {
+                        const int ch = open ? kid[o] : -1;
+                        const uint64_t leaf = __builtin_amdgcn_ballot_w64(ch < -1);
+                        const uint64_t cell = __builtin_amdgcn_ballot_w64(ch >= 0);
+                        if (lcnt > kGroupLeaves - kWave) {
+                            flush();
+                        }
+                        if (ch < -1) {
+                            ltag[lcnt + static_cast<int>(lanes_below(leaf))] = -ch - 2;
+                        }
+                        if (ch >= 0) {
+                            pending_all[at + static_cast<int>(lanes_below(cell))] = ch;
+                        }
+                        at += static_cast<int>(__popcll(cell));
+                        lcnt += static_cast<int>(__popcll(leaf));
+                    }
                 }
             }
             if (overflow) {
                 break;
             }
-            wave_lds_fence();   // pushes visible before the next pops
+            // pushes visible before the next pops
+            if (team) {
+                lds_barrier();
+            } else {
+                wave_lds_fence();
+            }
         }
         if (!overflow && ccnt + lcnt > 0) {
             flush();
@@ -2386,12 +2499,44 @@ __global__ __launch_bounds__(kGroupThreads) void group_walk_kernel(
             continue;
         }
         if (shared) {
-            ++walks;
-            if (!shared_walk(a, b)) {
-                per_query = per_query || (valid && t >= a && t <= b);
+            if (lane == 0) {
+                ranges[kRangeStack - 1 - walks] = make_int2(a, b);
             }
+            ++walks;
         } else {
             per_query = per_query || (valid && t >= a && t <= b);
+        }
+    }
+    wave_lds_fence();
+    // few ranges: all waves on each in turn; more: a wave a range
+    const bool team = W > 1 && walks <= kTeamRanges;
+    for (int k = team ? 0 : wid; k < walks; k += team ? 1 : W) {
+        const int2 r = ranges[kRangeStack - 1 - k];
+        const int a = __builtin_amdgcn_readfirstlane(r.x);
+        const int b = __builtin_amdgcn_readfirstlane(r.y);
+        if (!shared_walk(a, b, team)) {
+            per_query = per_query || (valid && t >= a && t <= b);
+        }
+    }
+    if constexpr (W > 1) {
+        // The group's sums: the waves' in their order
+        lcell[lane] = make_float4(acc.ax, acc.ay, acc.az, per_query ? 1.f : 0.f);
+        lcell[kWave + lane] = make_float4(__uint_as_float(acc.approx), __uint_as_float(acc.exact),
+                                          0.f, 0.f);
+        __syncthreads();
+        if (wid != 0) {
+            return;
+        }
+#pragma unroll
+        for (int w = 1; w < W; ++w) {
+            const float4 sum = lcell_all[w][lane];
+            const float4 count = lcell_all[w][kWave + lane];
+            acc.ax += sum.x;
+            acc.ay += sum.y;
+            acc.az += sum.z;
+            per_query = per_query || sum.w != 0.f;
+            acc.approx += __float_as_uint(count.x);
+            acc.exact += __float_as_uint(count.y);
         }
     }
     // The lanes whose range could not share a list go to the deferred list
@@ -2838,21 +2983,32 @@ NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exac
         // theta = 1.0, 10M: 9.61 -> 7.96 ms.)
         const bool member_test =
             features != nullptr || (e->flags & NBX_FLAG_BH_BOX_TEST) == 0;
+        // (the feature walk's sums keep their order: one wave a group)
+        const size_t groups = (s.n + kWave - 1) / kWave;
+        const int team = features != nullptr ? 1 : walk_team(groups, e->cu_count);
+        const int chunk_log = team > 1 ? kTeamChunkLog : kChunkLog;
         // whole rounds of one chunk per XCD (blocks past the last group exit)
-        const size_t chunks = (s.n + static_cast<size_t>(kWave) * kGroupChunk - 1) /
-                              (static_cast<size_t>(kWave) * kGroupChunk);
-        const unsigned grid_g =
-            static_cast<unsigned>((chunks + kXcds - 1) / kXcds * kXcds * kGroupChunk);
+        const size_t round = static_cast<size_t>(kXcds) << chunk_log;
+        const unsigned grid_g = static_cast<unsigned>((groups + round - 1) / round * round);
         if (features != nullptr) {
-            group_walk_kernel<true><<<grid_g, kGroupThreads, 0, st>>>(
+            group_walk_kernel<true, 1><<<grid_g, kWave, 0, st>>>(
                 flags, deferred, gn, B<float4>(s.s4), B<uint32_t>(s.tperm),
                 B<uint64_t>(s.tword), s.ext_tree, ni, Gf, e2, th2, e->ax, e->ay, e->az, cnts,
-                features, gq, max_walks, member_test);
+                features, gq, max_walks, member_test, chunk_log);
         } else {
-            group_walk_kernel<false><<<grid_g, kGroupThreads, 0, st>>>(
-                flags, deferred, gn, B<float4>(s.s4), B<uint32_t>(s.tperm),
-                B<uint64_t>(s.tword), s.ext_tree, ni, Gf, e2, th2, e->ax, e->ay, e->az, cnts,
-                nullptr, nullptr, max_walks, member_test);
+            auto go = [&](auto kernel) {
+                kernel<<<grid_g, team * kWave, 0, st>>>(
+                    flags, deferred, gn, B<float4>(s.s4), B<uint32_t>(s.tperm),
+                    B<uint64_t>(s.tword), s.ext_tree, ni, Gf, e2, th2, e->ax, e->ay, e->az, cnts,
+                    nullptr, nullptr, max_walks, member_test, chunk_log);
+            };
+            if (team == 4) {
+                go(group_walk_kernel<false, 4>);
+            } else if (team == 2) {
+                go(group_walk_kernel<false, 2>);
+            } else {
+                go(group_walk_kernel<false, 1>);
+            }
         }
     };
     const bool group = !fp64_exact && !(e->flags & NBX_FLAG_BH_REFERENCE_LISTS);

@@ -315,6 +315,30 @@ def test_group_walk_features_are_consistent(nbx):
     assert not f[:, 10:].any()
 
 
+@pytest.mark.parametrize("n,eps", [
+    (2, 0.01), (64, 0.01), (65, 0.0), (700, 0.01), (3000, 0.0), (20_000, 0.01),
+    (131_072, 0.01),    # the last size of four waves a group
+    (131_073, 0.01),    # two waves, the last group of one particle
+    (524_289, 0.01),    # one wave a group
+])
+def test_walk_teams_take_the_groups_lists(nbx, n, eps):
+    """The plain walk by teams of waves against the feature walk, which always
+    takes one wave a group: the same interactions. FP32 sums of up to some 4,000
+    terms in another order differ by sqrt(4000) x 6e-8 of the sum of the terms'
+    sizes, some times |a|."""
+    d = nbx.two_galaxy(n, seed=8)
+    with nbx.Engine(n, theta=0.7) as e:
+        e.upload(d["pos"], d["m"])
+        e.bh_features(1.0, eps)
+        one, one_stats = e.accelerations(), e.stats()
+        e.compute_force("hip_barnes_hut", 1.0, eps)
+        team, team_stats = e.accelerations(), e.stats()
+    a = np.linalg.norm(one, axis=1)
+    assert np.all(np.linalg.norm(team - one, axis=1) <= 3e-5 * np.maximum(a, a.mean()))
+    for k in ("accepted_approximations", "exact_interactions"):
+        assert team_stats[k] == one_stats[k]
+
+
 def test_feature_walk_fallback_is_the_reference_list_walk(nbx):
     """With the split off (NBX_FLAG_BH_NO_SPLIT) the feature walk leaves the
     particles of non-compact groups to the per-query walk that runs after
