@@ -194,6 +194,20 @@ __device__ inline void block_bounds(const double (&lo)[3], const double (&hi)[3]
     }
 }
 
+// The walk's counters: cell terms, leaf terms, deferred queries. Behind them the
+// device clock at the start of each phase of an evaluation: its first
+// kernel's first workgroup writes it, all on one XCD. (An event between two
+// kernels kept the stream idle for 5.8 us: six of them were a sixth of an
+// evaluation of 10,000 particles.)
+constexpr int kCounters = 3;
+enum { PHASE_KEYS, PHASE_SORT, PHASE_TREE, PHASE_COM, PHASE_WALK, PHASE_END, kPhases };
+
+__device__ inline void phase_begins(unsigned long long* __restrict__ counters, int phase) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        counters[kCounters + phase] = static_cast<unsigned long long>(wall_clock64());
+    }
+}
+
 // The first workgroup also clears the build's flag words and the walk's
 // counters (interactions, deferred queries), which only later kernels touch.
 template <typename In>
@@ -206,10 +220,11 @@ __global__ __launch_bounds__(kThreads) void bbox_partial_kernel(
         for (int k = threadIdx.x; k < flag_words; k += kThreads) {
             flags[k] = 0u;
         }
-        if (threadIdx.x < 3) {
+        if (threadIdx.x < kCounters) {
             counters[threadIdx.x] = 0ull;
         }
     }
+    phase_begins(counters, PHASE_KEYS);
     const double4 p0 = widen(build_input<In>(px, py, pz, m, 0));
     double lo[3] = {p0.x, p0.y, p0.z};
     double hi[3] = {lo[0], lo[1], lo[2]};
@@ -547,7 +562,9 @@ __device__ inline void bitonic_sort(SortItem (&e)[kSortItems], int tid, uint64_t
 template <typename In>
 __global__ __launch_bounds__(kThreads) void tile_sort_kernel(
     const In* __restrict__ b4, int n, const double* __restrict__ partial, int bb_blocks,
-    double* __restrict__ root, uint64_t* __restrict__ kout, uint32_t* __restrict__ vout) {
+    double* __restrict__ root, uint64_t* __restrict__ kout, uint32_t* __restrict__ vout,
+    unsigned long long* __restrict__ counters) {
+    phase_begins(counters, PHASE_SORT);
     __shared__ double s[6][kThreads];
     __shared__ double cube[4];
     __shared__ uint64_t skey[kSortTile1];
@@ -746,9 +763,11 @@ __global__ __launch_bounds__(kThreads) void delta_kernel(const uint64_t* __restr
                                                         const uint64_t* __restrict__ ext, int n,
                                                         int tiles, int32_t* __restrict__ delta,
                                                         unsigned* __restrict__ flags,
-                                                        unsigned* __restrict__ tile_hist) {
+                                                        unsigned* __restrict__ tile_hist,
+                                                        unsigned long long* __restrict__ counters) {
     __shared__ unsigned hist[kTopoRows];
     __shared__ unsigned tile_flags;
+    phase_begins(counters, PHASE_TREE);
     if (build_failed(flags)) {
         return;
     }
@@ -1444,8 +1463,12 @@ template <bool QUAD, typename In, int T>
 __global__ __launch_bounds__(T) void span_com_kernel(int unit_tiles, int group_units, int tiles,
                                                      const unsigned* __restrict__ flags,
                                                      const unsigned* __restrict__ tile_base,
-                                                     CellData<In> c) {
+                                                     CellData<In> c,
+                                                     unsigned long long* __restrict__ counters) {
     __shared__ SpanTable<T> s;
+    if (unit_tiles == 1) {
+        phase_begins(counters, PHASE_COM);
+    }
     if (build_failed(flags)) {
         return;
     }
@@ -1589,7 +1612,7 @@ __global__ __launch_bounds__(kThreads) void node_records_kernel(
 struct BuildReport {
     unsigned flags[kFlagWords];
     double root[4];
-    unsigned long long counters[3];
+    unsigned long long counters[kCounters + kPhases];
 };
 
 __global__ __launch_bounds__(kThreads) void report_kernel(const unsigned* __restrict__ flags,
@@ -1603,8 +1626,10 @@ __global__ __launch_bounds__(kThreads) void report_kernel(const unsigned* __rest
     if (k < 4) {
         out->root[k] = root[k];
     }
-    if (k < 3) {
+    if (k < kCounters + kPhases - 1) {
         out->counters[k] = counters[k];
+    } else if (k == kCounters + PHASE_END) {
+        out->counters[k] = static_cast<unsigned long long>(wall_clock64());
     }
 }
 
@@ -1618,6 +1643,7 @@ __global__ __launch_bounds__(kThreads) void walk_f64_kernel(
     double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
     unsigned long long* __restrict__ counters) {
     __shared__ unsigned long long block_counts[2];
+    phase_begins(counters, PHASE_WALK);
     if (build_failed(flags)) {
         return;
     }
@@ -2090,6 +2116,7 @@ __global__ __launch_bounds__(W * kWave) void group_walk_kernel(
     double* __restrict__ az, unsigned long long* __restrict__ counters,
     float* __restrict__ features, const float4* __restrict__ gquad,
     int max_walks, bool member_test, int chunk_log) {
+    phase_begins(counters, PHASE_WALK);
     constexpr int kWaves = W;
     // per wave: pending cells; staged cells (COM, mass; with FEATURES the
     // quadrupole record); staged leaves (tree position, then position and
@@ -2612,16 +2639,16 @@ NBodySimProStatus enqueue_order(Engine* e, NBodySimProError* error) {
     unsigned* flags = B<unsigned>(s.flags);
     In* b4 = B<In>(s.b4);
     double* root = root_of(s);
+    unsigned long long* cnts = B<unsigned long long>(s.counters);
     double4* sp4 = std::is_same_v<In, double4> ? B<double4>(s.sp4) : nullptr;
     const unsigned bb_blocks = g < static_cast<unsigned>(kBBoxBlocks) ? g : kBBoxBlocks;
     bbox_partial_kernel<In><<<bb_blocks, kThreads, 0, st>>>(
         e->px, e->py, e->pz, e->m, b4, ni, B<double>(s.partial), flags, kFlagWords,
-        B<unsigned long long>(s.counters));
+        cnts);
     if (s.n <= static_cast<size_t>(kSmallSort)) {
-        NBX_HIP(error, hipEventRecord(e->ev[1], st));
         tile_sort_kernel<In><<<grid_for(s.n, kSortTile1), kThreads, 0, st>>>(
             b4, ni, B<double>(s.partial), static_cast<int>(bb_blocks), root, B<uint64_t>(s.sk0),
-            B<uint32_t>(s.sv0));
+            B<uint32_t>(s.sv0), cnts);
         merge_order_kernel<In><<<grid_for(s.n * kMergeLanes, kThreads), kThreads, 0, st>>>(
             B<uint64_t>(s.sk0), B<uint32_t>(s.sv0), ni, b4, B<uint32_t>(s.tperm),
             B<uint64_t>(s.tword), sp4, B<float4>(s.s4));
@@ -2630,21 +2657,20 @@ NBodySimProStatus enqueue_order(Engine* e, NBodySimProError* error) {
         keys_kernel<In><<<g < 1024u ? g : 1024u, kThreads, 0, st>>>(
             b4, ni, B<double>(s.partial), static_cast<int>(bb_blocks), root, B<uint64_t>(s.sk0));
         NBX_HIP(error, hipGetLastError());
-        NBX_HIP(error, hipEventRecord(e->ev[1], st));
         NBX_TRY(s.ext.need<uint64_t>(s.n * kExtWords, error));
         // stable on the top key bits (the result stays in sk0/sv0), then the
         // short runs. (Measured on MI355X, two-galaxy, against seven passes
         // on all 63 bits: sort 1M 0.171 -> 0.108 ms, 10M 0.894 -> 0.641 ms.)
         NBX_TRY(radix_sort_pairs(st, B<uint64_t>(s.sk0), B<uint32_t>(s.sv0), B<uint64_t>(s.sk1),
                                  B<uint32_t>(s.sv1), s.n, kSortTopBits, s.hist, error, nullptr,
-                                 nullptr, kSortLowBits, true));
+                                 nullptr, kSortLowBits, true,
+                                 cnts + kCounters + PHASE_SORT));
         order_kernel<In><<<g, kThreads, 0, st>>>(B<uint64_t>(s.sk0), B<uint32_t>(s.sv0), ni, b4,
                                                  root, B<uint32_t>(s.tperm), B<uint64_t>(s.tword),
                                                  B<uint64_t>(s.ext), sp4, B<float4>(s.s4), flags);
         s.ext_tree = B<uint64_t>(s.ext);
     }
     NBX_HIP(error, hipGetLastError());
-    NBX_HIP(error, hipEventRecord(e->ev[9], st));
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 
@@ -2699,7 +2725,8 @@ NBodySimProStatus enqueue_depths(Engine* e, NBodySimProError* error) {
     const int nt = static_cast<int>((s.n + kTopoTile - 1) / kTopoTile);
     unsigned* flags = B<unsigned>(s.flags);
     delta_kernel<<<nt, kThreads, 0, st>>>(B<uint64_t>(s.tword), s.ext_tree, ni, nt,
-                                          B<int32_t>(s.delta), flags, B<unsigned>(s.tile_hist));
+                                          B<int32_t>(s.delta), flags, B<unsigned>(s.tile_hist),
+                                          B<unsigned long long>(s.counters));
     depth_scan_kernel<<<kTopoRows, kThreads, 0, st>>>(B<unsigned>(s.tile_hist), nt,
                                                       B<unsigned>(s.tile_base), flags);
     NBX_HIP(error, hipGetLastError());
@@ -2739,21 +2766,20 @@ NBodySimProStatus enqueue_cells(Engine* e, NBodySimProError* error) {
     c.gquad = QUAD ? B<float4>(s.gquad) : nullptr;
     unsigned* flags = B<unsigned>(s.flags);
     const unsigned* base = B<unsigned>(s.tile_base);
+    unsigned long long* cnts = B<unsigned long long>(s.counters);
     build_kernel<QUAD, In><<<nt, kBuildThreads, 0, st>>>(
         B<uint64_t>(s.tword), s.ext_tree, B<int32_t>(s.delta), ni, nt, static_cast<int>(s.cells),
         flags, base, B<uint32_t>(s.scan), c);
-    NBX_HIP(error, hipGetLastError());
-    NBX_HIP(error, hipEventRecord(e->ev[3], st));
     if (nt > 1) {
         span_com_kernel<QUAD, In, 512><<<grid_for(nt, kSpanTiles), 512, 0, st>>>(
-            1, kSpanTiles, nt, flags, base, c);
+            1, kSpanTiles, nt, flags, base, c, cnts);
     }
     if (nt > kSpanTiles) {
         const int units = (nt + kSpanTiles - 1) / kSpanTiles;
-        span_com_kernel<QUAD, In, 1024><<<1, 1024, 0, st>>>(kSpanTiles, units, nt, flags, base, c);
+        span_com_kernel<QUAD, In, 1024><<<1, 1024, 0, st>>>(kSpanTiles, units, nt, flags, base, c,
+                                                           cnts);
     }
     NBX_HIP(error, hipGetLastError());
-    NBX_HIP(error, hipEventRecord(e->ev[4], st));
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 
@@ -2853,7 +2879,7 @@ NBodySimProStatus bh_build(Engine* e, bool fp32_inputs, NBodySimProError* error,
         NBX_TRY(s.sp4.need<double4>(n, error));
     }
     NBX_TRY(s.s4.need<float4>(n, error));
-    NBX_TRY(s.counters.need<unsigned long long>(3, error));
+    NBX_TRY(s.counters.need<unsigned long long>(kCounters + kPhases, error));
     NBX_TRY(s.deferred.need<int32_t>(n, error));
     const size_t tiles = (n + kTopoTile - 1) / kTopoTile;
     NBX_TRY(s.tile_hist.need<unsigned>(kTopoRows * tiles, error));
@@ -2871,7 +2897,6 @@ NBodySimProStatus bh_build(Engine* e, bool fp32_inputs, NBodySimProError* error,
     s.inputs_fp64 = !fp32_inputs;
     s.has_n64 = !fp32_inputs;
     s.has_quad = quadrupoles;
-    NBX_HIP(error, hipEventRecord(e->ev[0], e->stream));
     NBX_TRY(fp32_inputs ? enqueue_order<float4>(e, error) : enqueue_order<double4>(e, error));
     NBX_TRY(enqueue_depths(e, error));
     return enqueue_cells(e, error);
@@ -3013,6 +3038,7 @@ NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exac
     };
     const bool group = !fp64_exact && !(e->flags & NBX_FLAG_BH_REFERENCE_LISTS);
     const bool lists = !fp64_exact && !group;
+    float per_query_ms = 0.f;
     // Each repetition follows a repaired build: an order on all the bits, then
     // room for its cells, at most.
     bool again = true;
@@ -3026,7 +3052,6 @@ NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exac
             group_walk();
         }
         NBX_HIP(error, hipGetLastError());
-        NBX_HIP(error, hipEventRecord(e->ev[6], st));
         const NBodySimProStatus status = read_build(e, &again, error);
         if (status != N_BODY_SIM_PRO_STATUS_OK) {
             s.n = 0;   // no tree
@@ -3048,38 +3073,57 @@ NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exac
             NBX_FAIL(error, N_BODY_SIM_PRO_STATUS_INVALID_STATE,
                      "deferred query count out of range");
         }
+        NBX_HIP(error, hipEventRecord(e->ev[0], st));
         NBX_TRY(lists ? per_query_walk(nullptr, ni)
                       : per_query_walk(B<int32_t>(s.deferred), static_cast<int>(deferred)));
-        NBX_HIP(error, hipEventRecord(e->ev[6], st));
+        NBX_HIP(error, hipEventRecord(e->ev[1], st));
         unsigned long long counts[2] = {0, 0};
         NBX_HIP(error, hipMemcpyAsync(counts, s.counters.p, sizeof(counts),
                                       hipMemcpyDeviceToHost, st));
         NBX_HIP(error, hipStreamSynchronize(st));
         e->stats.accepted_approximations = counts[0];
         e->stats.exact_interactions = counts[1];
+        NBX_HIP(error, hipEventElapsedTime(&per_query_ms, e->ev[0], e->ev[1]));
     }
+    s.per_query_ms = per_query_ms;
+    s.walked_lists = lists;
     return N_BODY_SIM_PRO_STATUS_OK;
+}
+
+void bh_timings(Engine* e) {
+    BHState& s = e->bh;
+    // the phases' starts on the device clock, a phase that had no kernel at
+    // the next one's
+    unsigned long long* at = static_cast<BuildReport*>(s.report)->counters + kCounters;
+    if (s.walked_lists) {
+        at[PHASE_WALK] = at[PHASE_END];
+    }
+    if (s.n <= static_cast<size_t>(kTopoTile)) {
+        at[PHASE_COM] = at[PHASE_WALK];
+    }
+    auto ms = [&](int from, int to) {
+        return at[to] > at[from] ? static_cast<double>(at[to] - at[from]) / e->clock_khz : 0.0;
+    };
+    NBXTimings tm{};
+    tm.bbox_keys_ms = ms(PHASE_KEYS, PHASE_SORT);
+    tm.sort_ms = ms(PHASE_SORT, PHASE_TREE);
+    tm.tree_ms = ms(PHASE_TREE, PHASE_COM);
+    tm.com_ms = ms(PHASE_COM, PHASE_WALK);
+    tm.walk_ms = ms(PHASE_WALK, PHASE_END) + s.per_query_ms;
+    tm.force_ms = ms(PHASE_KEYS, PHASE_END) + s.per_query_ms;
+    tm.kernel_ms = tm.walk_ms;
+    tm.kernel_flops = 20.0 * static_cast<double>(e->stats.accepted_approximations +
+                                                 e->stats.exact_interactions);
+    e->timings = tm;
+    e->stats.build_time_seconds = ms(PHASE_KEYS, PHASE_WALK) * 1e-3;
+    e->stats.evaluation_time_seconds = tm.walk_ms * 1e-3;
 }
 
 NBodySimProStatus barnes_hut(Engine* e, const NBodySimProGravity* g, bool fp64_exact,
                              NBodySimProError* error) {
     NBX_TRY(bh_build(e, !fp64_exact, error));
     NBX_TRY(bh_walk(e, g, fp64_exact, nullptr, error));
-    float t[10] = {0};
-    for (int k : {1, 3, 4, 6, 9}) {
-        NBX_HIP(error, hipEventElapsedTime(&t[k], e->ev[0], e->ev[k]));
-    }
-    NBXTimings tm{};
-    tm.bbox_keys_ms = t[1];
-    tm.sort_ms = t[9] - t[1];
-    tm.tree_ms = t[3] - t[9];
-    tm.com_ms = t[4] - t[3];
-    tm.walk_ms = t[6] - t[4];   // the walk follows the centre of mass
-    tm.force_ms = t[6];
-    tm.kernel_ms = tm.walk_ms;
-    const double interactions = static_cast<double>(e->stats.accepted_approximations +
-                                                    e->stats.exact_interactions);
-    tm.kernel_flops = 20.0 * interactions;
+    bh_timings(e);
     // walk bytes: every query reads its position (and permutation entry) and
     // writes 3 doubles; the cell records the walk reads are counted once per
     // launch (they stay in L2 across waves): GroupNode records for the group
@@ -3089,11 +3133,8 @@ NBodySimProStatus barnes_hut(Engine* e, const NBodySimProGravity* g, bool fp64_e
         fp64_exact ? static_cast<double>(e->bh.nodes) * sizeof(NodeF64)
         : group    ? static_cast<double>(e->bh.internal) * sizeof(GroupNode)
                    : static_cast<double>(e->bh.nodes) * sizeof(NodeF32);
-    tm.kernel_bytes = static_cast<double>(e->bh.n) * ((fp64_exact ? 24.0 : 16.0) + 24.0 + 4.0) +
+    e->timings.kernel_bytes = static_cast<double>(e->bh.n) * ((fp64_exact ? 24.0 : 16.0) + 24.0 + 4.0) +
                       node_bytes;
-    e->timings = tm;
-    e->stats.build_time_seconds = t[4] * 1e-3;
-    e->stats.evaluation_time_seconds = tm.walk_ms * 1e-3;
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 

@@ -450,6 +450,11 @@ NBXEngine* nbx_engine_create(const NBXConfig* config, NBodySimProError* error) {
         cus > 0) {
         e->cu_count = cus;
     }
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, e->device) == hipSuccess &&
+        khz > 0) {
+        e->clock_khz = khz;
+    }
     double** arrays[] = {&e->px, &e->py, &e->pz, &e->vx, &e->vy, &e->vz,
                          &e->ax, &e->ay, &e->az, &e->m};
     for (double** a : arrays) {

@@ -111,6 +111,8 @@ struct BHState {
     // pinned host block the evaluation's flags, counts, root cube and
     // interaction counters are reported into (BuildReport)
     void* report = nullptr;
+    float per_query_ms = 0.f;      // the per-query walk that followed the last walk
+    bool walked_lists = false;     // there was no other
     // build inputs (x, y, z, m): FP32-rounded copies of the master arrays
     // (float4) or the FP64 values (double4)
     Buf b4;                   // (x, y, z, m) per particle in original order
@@ -152,6 +154,7 @@ struct BHState {
 struct Engine {
     int device = 0;
     int cu_count = 256;       // compute units of the device (grid shape choices)
+    double clock_khz = 1e5;   // rate of the device's wall clock
     hipStream_t stream = nullptr;
     size_t capacity = 0;
     size_t n = 0;
@@ -170,7 +173,7 @@ struct Engine {
     NodeF32* learned_dummy = nullptr;
     NBodySimProBarnesHutStats stats{};
     NBXTimings timings{};
-    hipEvent_t ev[12]{};
+    hipEvent_t ev[3]{};
     // learned BH correction
     void* mlp = nullptr;
 };
@@ -193,6 +196,8 @@ NBodySimProStatus bh_morton_order(Engine* e, NBodySimProError* error);
 // repairs a build whose flags say so). The build clears the walk's counters.
 NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exact,
                           float* features, NBodySimProError* error);
+// e->timings and the times in e->stats of the evaluation that bh_walk ended.
+void bh_timings(Engine* e);
 NBodySimProStatus bh_learned(Engine* e, const NBodySimProGravity* g, NBodySimProError* error);
 
 // Stable LSD radix sort of (64-bit key, 32-bit value) pairs, ascending key;
@@ -205,7 +210,8 @@ NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals
                                    uint64_t* keys_alt, uint32_t* vals_alt, size_t n, int bits,
                                    Buf& hist, NBodySimProError* error,
                                    uint64_t* keys_out = nullptr, uint32_t* vals_out = nullptr,
-                                   int first_bit = 0, bool iota = false);
+                                   int first_bit = 0, bool iota = false,
+                                   unsigned long long* start_clock = nullptr);
 // Bits of `mask` set in the lanes below this one (v_mbcnt_lo/hi: two VALU
 // instructions, where and-ing a per-lane mask and counting bits takes four).
 __device__ inline unsigned lanes_below(uint64_t mask) {

@@ -838,7 +838,7 @@ NBodySimProStatus bh_learned(Engine* e, const NBodySimProGravity* g, NBodySimPro
     NBX_TRY(e->scratch2.need<float>(s.n * kWalkRecord, error));
     float* walkf = e->scratch2.as<float>();
     NBX_TRY(bh_walk(e, g, false, walkf, error));
-    NBX_HIP(error, hipEventRecord(e->ev[7], e->stream));
+    NBX_HIP(error, hipEventRecord(e->ev[0], e->stream));
     // One resident round of workgroups that stride over the 64-query tiles:
     // a grid beyond what fits leaves a second, partial round on some CUs.
     // (Measured on MI355X at 10M: 4 workgroups per CU requested with 3
@@ -854,31 +854,14 @@ NBodySimProStatus bh_learned(Engine* e, const NBodySimProGravity* g, NBodySimPro
         static_cast<float>(std::log2(2.0 * s.root[3])),
         static_cast<float>(g->gravitational_constant), e->ax, e->ay, e->az);
     NBX_HIP(error, hipGetLastError());
-    NBX_HIP(error, hipEventRecord(e->ev[8], e->stream));
-    NBX_HIP(error, hipEventSynchronize(e->ev[8]));
-    float t[10] = {0};
-    for (int k : {1, 3, 4, 6, 8, 9}) {
-        NBX_HIP(error, hipEventElapsedTime(&t[k], e->ev[0], e->ev[k]));
-    }
+    NBX_HIP(error, hipEventRecord(e->ev[1], e->stream));
+    NBX_HIP(error, hipEventSynchronize(e->ev[1]));
     float mlp_ms = 0.f;
-    NBX_HIP(error, hipEventElapsedTime(&mlp_ms, e->ev[7], e->ev[8]));
-    NBXTimings tm{};
-    tm.bbox_keys_ms = t[1];
-    tm.sort_ms = t[9] - t[1];
-    tm.tree_ms = t[3] - t[9];
-    tm.com_ms = t[4] - t[3];
-    float walk_ms = 0.f;
-    NBX_HIP(error, hipEventElapsedTime(&walk_ms, e->ev[4], e->ev[6]));
-    tm.walk_ms = walk_ms;
-    tm.force_ms = t[8];
-    tm.kernel_ms = walk_ms;
-    tm.mlp_ms = mlp_ms;
-    const double interactions = static_cast<double>(e->stats.accepted_approximations +
-                                                    e->stats.exact_interactions);
-    tm.kernel_flops = 20.0 * interactions;
-    e->timings = tm;
-    e->stats.build_time_seconds = t[4] * 1e-3;
-    e->stats.evaluation_time_seconds = (t[8] - t[4]) * 1e-3;
+    NBX_HIP(error, hipEventElapsedTime(&mlp_ms, e->ev[0], e->ev[1]));
+    bh_timings(e);
+    e->timings.mlp_ms = mlp_ms;
+    e->timings.force_ms += mlp_ms;
+    e->stats.evaluation_time_seconds += mlp_ms * 1e-3;
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 

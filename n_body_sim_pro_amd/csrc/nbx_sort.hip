@@ -40,9 +40,13 @@ template <int IPT>
 __global__ __launch_bounds__(kSortThreads) void sort_histogram(const uint64_t* __restrict__ keys,
                                                               size_t n, int shift,
                                                               uint32_t* __restrict__ hist,
-                                                              unsigned tiles) {
+                                                              unsigned tiles,
+                                                              unsigned long long* start_clock) {
     constexpr int kSortTile = kSortThreads * IPT;
     __shared__ uint32_t h[kRadix];
+    if (start_clock != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
+        *start_clock = static_cast<unsigned long long>(wall_clock64());
+    }
     const unsigned tile = blockIdx.x;
     for (int k = threadIdx.x; k < kRadix; k += kSortThreads) {
         h[k] = 0;
@@ -231,7 +235,8 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter(
 NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals,
                                    uint64_t* keys_alt, uint32_t* vals_alt, size_t n, int bits,
                                    Buf& hist, NBodySimProError* error, uint64_t* keys_out,
-                                   uint32_t* vals_out, int first_bit, bool iota) {
+                                   uint32_t* vals_out, int first_bit, bool iota,
+                                   unsigned long long* start_clock) {
     if (keys_out == nullptr || vals_out == nullptr) {
         keys_out = keys;
         vals_out = vals;
@@ -271,10 +276,13 @@ NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals
             vout = (kout == keys) ? vals : vals_alt;
         }
         if (large) {
-            sort_histogram<8><<<tiles, kSortThreads, 0, s>>>(kin, n, shift, h, tiles);
+            sort_histogram<8><<<tiles, kSortThreads, 0, s>>>(kin, n, shift, h, tiles,
+                                                             start_clock);
         } else {
-            sort_histogram<4><<<tiles, kSortThreads, 0, s>>>(kin, n, shift, h, tiles);
+            sort_histogram<4><<<tiles, kSortThreads, 0, s>>>(kin, n, shift, h, tiles,
+                                                             start_clock);
         }
+        start_clock = nullptr;   // the first pass's
         sort_scan_digit<<<kRadix, kSortThreads, 0, s>>>(h, tiles, totals);
         if (large) {
             sort_scatter<8><<<tiles, kSortThreads, 0, s>>>(kin, vin, kout, vout, n, shift, h,
