@@ -1614,6 +1614,7 @@ struct BuildReport {
     double root[4];
     unsigned long long counters[kCounters + kPhases];
 };
+static_assert(sizeof(BuildReport) <= kReportBytes, "the engine's pinned block holds a report");
 
 __global__ __launch_bounds__(kThreads) void report_kernel(const unsigned* __restrict__ flags,
                                                           const double* __restrict__ root,
@@ -2881,12 +2882,12 @@ NBodySimProStatus bh_build(Engine* e, bool fp32_inputs, NBodySimProError* error,
     NBX_TRY(s.s4.need<float4>(n, error));
     NBX_TRY(s.counters.need<unsigned long long>(kCounters + kPhases, error));
     NBX_TRY(s.deferred.need<int32_t>(n, error));
+    if (s.report == nullptr) {
+        NBX_HIP(error, hipHostMalloc(&s.report, kReportBytes, hipHostMallocDefault));
+    }
     const size_t tiles = (n + kTopoTile - 1) / kTopoTile;
     NBX_TRY(s.tile_hist.need<unsigned>(kTopoRows * tiles, error));
     NBX_TRY(s.tile_base.need<unsigned>(kTopoRows * tiles, error));
-    if (s.report == nullptr) {
-        NBX_HIP(error, hipHostMalloc(&s.report, sizeof(BuildReport), hipHostMallocDefault));
-    }
     // Room for the cells of usual inputs (about n / 2); a tree with more
     // raises FLAG_CELLS and is built again with room for its count.
     if (s.cells_n != n) {

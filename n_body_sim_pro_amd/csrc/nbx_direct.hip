@@ -563,51 +563,66 @@ NBodySimProStatus refresh_pos4(Engine* e, NBodySimProError* error) {
 
 NBodySimProStatus direct_fp64(Engine* e, const NBodySimProGravity* g, NBodySimProError* error) {
     const size_t n = e->n;
+    e->pending = 0;
     if (n == 0) {
         return N_BODY_SIM_PRO_STATUS_OK;
     }
-    NBX_HIP(error, hipEventRecord(e->ev[0], e->stream));
+    if (e->timed) {
+        NBX_HIP(error, hipEventRecord(e->ev[0], e->stream));
+    }
     launch_direct_fp64<false>(e->stream, e->cu_count, e->px, e->py, e->pz, e->m, e->ax, e->ay,
                               e->az, static_cast<int>(n), g->gravitational_constant,
                               g->softening_squared, nullptr, static_cast<int>(n), nullptr);
     NBX_HIP(error, hipGetLastError());
-    NBX_HIP(error, hipEventRecord(e->ev[1], e->stream));
-    NBX_HIP(error, hipEventSynchronize(e->ev[1]));
-    float ms = 0.f;
-    NBX_HIP(error, hipEventElapsedTime(&ms, e->ev[0], e->ev[1]));
-    e->timings = NBXTimings{};
-    e->timings.force_ms = ms;
-    e->timings.kernel_ms = ms;
-    const double pairs = static_cast<double>(n) * static_cast<double>(n - 1);
-    e->timings.kernel_flops = 20.0 * pairs;
-    e->timings.kernel_bytes = 4.0 * 8.0 * static_cast<double>(n) + 3.0 * 8.0 * static_cast<double>(n);
+    if (e->timed) {
+        NBX_HIP(error, hipEventRecord(e->ev[1], e->stream));
+        e->pending = 2;
+    }
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 
 NBodySimProStatus direct_fp32(Engine* e, const NBodySimProGravity* g, NBodySimProError* error) {
     const size_t n = e->n;
+    e->pending = 0;
     if (n == 0) {
         return N_BODY_SIM_PRO_STATUS_OK;
     }
-    NBX_HIP(error, hipEventRecord(e->ev[0], e->stream));
+    if (e->timed) {
+        NBX_HIP(error, hipEventRecord(e->ev[0], e->stream));
+    }
     if (n > static_cast<size_t>(kStageN)) {
         NBX_TRY(refresh_pos4(e, error));
     }
-    NBX_HIP(error, hipEventRecord(e->ev[1], e->stream));
+    if (e->timed) {
+        NBX_HIP(error, hipEventRecord(e->ev[1], e->stream));
+    }
     launch_direct_fp32(e->stream, e->px, e->py, e->pz, e->m, e->pos4, e->ax, e->ay, e->az,
                        static_cast<int>(n), g);
     NBX_HIP(error, hipGetLastError());
-    NBX_HIP(error, hipEventRecord(e->ev[2], e->stream));
-    NBX_HIP(error, hipEventSynchronize(e->ev[2]));
-    float total = 0.f, kern = 0.f;
-    NBX_HIP(error, hipEventElapsedTime(&total, e->ev[0], e->ev[2]));
-    NBX_HIP(error, hipEventElapsedTime(&kern, e->ev[1], e->ev[2]));
+    if (e->timed) {
+        NBX_HIP(error, hipEventRecord(e->ev[2], e->stream));
+        e->pending = 3;
+    }
+    return N_BODY_SIM_PRO_STATUS_OK;
+}
+
+NBodySimProStatus direct_timings(Engine* e, NBodySimProError* error) {
+    const int events = e->pending;
+    if (events == 0) {
+        return N_BODY_SIM_PRO_STATUS_OK;
+    }
+    e->pending = 0;
+    NBX_HIP(error, hipEventSynchronize(e->ev[events - 1]));
+    float total = 0.f, kernel = 0.f;
+    NBX_HIP(error, hipEventElapsedTime(&total, e->ev[0], e->ev[events - 1]));
+    NBX_HIP(error, hipEventElapsedTime(&kernel, e->ev[events - 2], e->ev[events - 1]));
+    const double n = static_cast<double>(e->n);
     e->timings = NBXTimings{};
     e->timings.force_ms = total;
-    e->timings.kernel_ms = kern;
-    const double pairs = static_cast<double>(n) * static_cast<double>(n - 1);
-    e->timings.kernel_flops = 20.0 * pairs;
-    e->timings.kernel_bytes = 16.0 * static_cast<double>(n) + 24.0 * static_cast<double>(n);
+    e->timings.kernel_ms = kernel;
+    e->timings.kernel_flops = 20.0 * n * (n - 1.0);
+    // FP64: x, y, z, m of each; FP32: one float4; three doubles out
+    e->timings.kernel_bytes = ((events == 2 ? 4.0 * 8.0 : 16.0) + 3.0 * 8.0) * n;
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 

@@ -93,6 +93,8 @@ struct alignas(16) NodeF64 {
     int32_t leaf;
 };
 
+constexpr size_t kReportBytes = 4096;
+
 // Barnes-Hut device workspace (all sized by particle or node capacity).
 struct BHState {
     size_t n = 0;             // particles in the last build
@@ -109,7 +111,7 @@ struct BHState {
     const uint64_t* ext_tree = nullptr;   // tree-order extension words or null (ext below)
     double root[4] = {0, 0, 0, 1};
     // pinned host block the evaluation's flags, counts, root cube and
-    // interaction counters are reported into (BuildReport)
+    // interaction counters are reported into (BuildReport, kReportBytes)
     void* report = nullptr;
     float per_query_ms = 0.f;      // the per-query walk that followed the last walk
     bool walked_lists = false;     // there was no other
@@ -174,13 +176,23 @@ struct Engine {
     NBodySimProBarnesHutStats stats{};
     NBXTimings timings{};
     hipEvent_t ev[3]{};
+    void* stage = nullptr;    // pinned host memory of the small transfers
+    size_t stage_bytes = 0;
+    bool stage_in_report = false;   // it is the rest of bh.report's block
+    // all-pairs evaluations: what direct_timings has to read, and whether the
+    // coming one is to be timed at all
+    bool timed = true;
+    int pending = 0;          // 0 nothing, else the number of events recorded
     // learned BH correction
     void* mlp = nullptr;
 };
 
 // ---- entry points implemented per translation unit ----
+// The all-pairs evaluations only enqueue; direct_timings waits for the last
+// one and reads its times into e->timings (nothing pending: returns at once).
 NBodySimProStatus direct_fp64(Engine* e, const NBodySimProGravity* g, NBodySimProError* error);
 NBodySimProStatus direct_fp32(Engine* e, const NBodySimProGravity* g, NBodySimProError* error);
+NBodySimProStatus direct_timings(Engine* e, NBodySimProError* error);
 NBodySimProStatus refresh_pos4(Engine* e, NBodySimProError* error);
 NBodySimProStatus barnes_hut(Engine* e, const NBodySimProGravity* g, bool fp64_exact,
                              NBodySimProError* error);

@@ -57,6 +57,40 @@ def test_diagnostics_closed_forms(nbx):
         assert e.diagnostics(eps=0.0)["potential_energy"] == pytest.approx(-1.0, abs=1e-15)
 
 
+@pytest.mark.parametrize("n,capacity", [(1, 1), (255, 300), (257, 257), (32768, 32768),
+                                        (32769, 40000)])
+def test_transfers_bring_every_array(nbx, n, capacity):
+    """Ten arrays up to 32768 particles go through the pinned block, more by
+    copy commands; arrays that a view leaves out keep their values."""
+    rng = np.random.default_rng(n)
+    names = ("px", "py", "pz", "vx", "vy", "vz", "ax", "ay", "az", "m")
+    a = {k: rng.normal(size=n) for k in names}
+    b = {k: np.full(n, np.nan) for k in names}
+    with nbx.Engine(capacity) as e:
+        e.upload_view(nbx.make_view(n, **a))
+        e.download_view(nbx.make_view(n, **b))
+        for k in names:
+            assert np.array_equal(a[k], b[k]), k
+        c = {k: rng.normal(size=n) for k in ("px", "py", "pz", "m")}
+        e.upload_view(nbx.make_view(n, **c))
+        part = {k: np.full(n, np.nan) for k in ("vx", "az", "m")}
+        e.download_view(nbx.make_view(n, **part))
+        assert np.array_equal(part["vx"], a["vx"]) and np.array_equal(part["az"], a["az"])
+        assert np.array_equal(part["m"], c["m"])
+
+
+def test_all_pairs_advance_times_its_last_evaluation(nbx):
+    p = Particles(500, {k: np.random.default_rng(7).normal(size=500) for k in ("px", "py", "pz", "m")})
+    for alg, per in (("hip_direct_fp64", 56.0), ("hip_direct_fp32", 40.0)):
+        with nbx.Engine(500) as e:
+            e.upload_view(p.view)
+            e.compute_force(alg, eps=0.05)
+            e.advance(alg, dt=1e-3, steps=4, eps=0.05)
+            t = e.timings()
+        assert t["kernel_ms"] > 0.0 and t["integrate_ms"] > t["kernel_ms"]
+        assert t["kernel_bytes"] == per * 500 and t["kernel_flops"] == 20.0 * 500 * 499
+
+
 @pytest.mark.parametrize("n,eps,scale", [
     (1, 0.01, 1.0), (2, 0.01, 1.0), (16, 0.0, 1.0), (17, 0.01, 1.0), (64, 0.01, 1.0),
     (65, 0.0, 1.0), (129, 0.01, 1.0), (1000, 0.01, 1.0),
