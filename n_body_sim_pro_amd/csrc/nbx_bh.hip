@@ -1613,13 +1613,15 @@ struct BuildReport {
     unsigned flags[kFlagWords];
     double root[4];
     unsigned long long counters[kCounters + kPhases];
+    unsigned number;   // of the evaluation, written last: the host waits for it
 };
-static_assert(sizeof(BuildReport) <= kReportBytes, "the engine's pinned block holds a report");
+static_assert(2 * sizeof(BuildReport) <= kReportBytes, "the engine's pinned block holds a report");
 
 __global__ __launch_bounds__(kThreads) void report_kernel(const unsigned* __restrict__ flags,
                                                           const double* __restrict__ root,
                                                           const unsigned long long* __restrict__ counters,
-                                                          BuildReport* __restrict__ out) {
+                                                          BuildReport* __restrict__ out,
+                                                          unsigned number) {
     const int k = threadIdx.x;
     if (k < kFlagWords) {
         out->flags[k] = flags[k];
@@ -1631,6 +1633,11 @@ __global__ __launch_bounds__(kThreads) void report_kernel(const unsigned* __rest
         out->counters[k] = counters[k];
     } else if (k == kCounters + PHASE_END) {
         out->counters[k] = static_cast<unsigned long long>(wall_clock64());
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (k == 0) {
+        __hip_atomic_store(&out->number, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -2792,18 +2799,61 @@ NBodySimProStatus enqueue_cells(Engine* e, NBodySimProError* error) {
                           : enqueue_cells<false, float4>(e, error);
 }
 
-// Reads what the evaluation's kernels left in the flag words, once they have
-// run. `again` says that the tree was not valid (the walk did nothing) and
-// that the part in question has been enqueued anew.
-NBodySimProStatus read_build(Engine* e, bool* again, NBodySimProError* error) {
+BuildReport* report_of(BHState& s, int slot) {
+    return static_cast<BuildReport*>(s.report) + slot;
+}
+
+// Enqueues the report of the evaluation before it in the stream into a slot.
+NBodySimProStatus enqueue_report(Engine* e, int slot, NBodySimProError* error) {
+    BHState& s = e->bh;
+    s.number[slot] = ++s.evaluations;
+    report_kernel<<<1, kThreads, 0, e->stream>>>(B<unsigned>(s.flags), root_of(s),
+                                                 B<unsigned long long>(s.counters),
+                                                 report_of(s, slot), s.number[slot]);
+    NBX_HIP(error, hipGetLastError());
+    return N_BODY_SIM_PRO_STATUS_OK;
+}
+
+// Waits until a slot holds its report. (Polled: the wait then costs no packet
+// in the stream, and whatever is enqueued behind the report runs on.)
+NBodySimProStatus await_report(Engine* e, int slot, NBodySimProError* error) {
+    BHState& s = e->bh;
+    const unsigned* number = &report_of(s, slot)->number;
+    for (;;) {
+        for (int spin = 0; spin < 20000; ++spin) {
+            if (__atomic_load_n(number, __ATOMIC_ACQUIRE) == s.number[slot]) {
+                return N_BODY_SIM_PRO_STATUS_OK;
+            }
+            __builtin_ia32_pause();
+        }
+        // the stream is done or has failed: the report is there, or never will be
+        const hipError_t state = hipStreamQuery(e->stream);
+        if (state == hipErrorNotReady) {
+            (void)hipGetLastError();
+            continue;
+        }
+        NBX_HIP(error, state);
+        if (__atomic_load_n(number, __ATOMIC_ACQUIRE) != s.number[slot]) {
+            NBX_FAIL(error, N_BODY_SIM_PRO_STATUS_INVALID_STATE,
+                     "a Barnes-Hut evaluation ended without its report");
+        }
+    }
+}
+
+// Whether a report's evaluation needs nothing more from the host.
+bool report_clean(const BuildReport* r) {
+    return (r->flags[0] | r->flags[1] | r->flags[2] | r->flags[3]) == 0 && r->counters[2] == 0;
+}
+
+// Waits for the evaluation in `slot` and reads what its kernels left in the
+// flag words. `again` says that the tree was not valid (the walk did nothing)
+// and that the part in question has been enqueued anew.
+NBodySimProStatus read_build(Engine* e, int slot, bool* again, NBodySimProError* error) {
     BHState& s = e->bh;
     hipStream_t st = e->stream;
     unsigned* flags = B<unsigned>(s.flags);
-    BuildReport* report = static_cast<BuildReport*>(s.report);
-    report_kernel<<<1, kThreads, 0, st>>>(flags, root_of(s), B<unsigned long long>(s.counters),
-                                          report);
-    NBX_HIP(error, hipGetLastError());
-    NBX_HIP(error, hipStreamSynchronize(st));
+    NBX_TRY(await_report(e, slot, error));
+    const BuildReport* report = report_of(s, slot);
     *again = false;
     if (report->flags[FLAG_LONG_RUN] != 0 || report->flags[FLAG_TIE] != 0) {
         NBX_HIP(error, hipMemsetAsync(flags, 0, kFlagWords * sizeof(unsigned), st));
@@ -2884,6 +2934,7 @@ NBodySimProStatus bh_build(Engine* e, bool fp32_inputs, NBodySimProError* error,
     NBX_TRY(s.deferred.need<int32_t>(n, error));
     if (s.report == nullptr) {
         NBX_HIP(error, hipHostMalloc(&s.report, kReportBytes, hipHostMallocDefault));
+        std::memset(s.report, 0, kReportBytes);   // no evaluation's number
     }
     const size_t tiles = (n + kTopoTile - 1) / kTopoTile;
     NBX_TRY(s.tile_hist.need<unsigned>(kTopoRows * tiles, error));
@@ -2954,8 +3005,16 @@ NBodySimProStatus bh_morton_order(Engine* e, NBodySimProError* error) {
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 
-NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exact, float* features,
-                          NBodySimProError* error) {
+namespace {
+
+bool walks_lists(const Engine* e, bool fp64_exact) {
+    return !fp64_exact && (e->flags & NBX_FLAG_BH_REFERENCE_LISTS) != 0;
+}
+
+// The walk of the build before it in the stream (nothing where the reference
+// lists are asked for: those wait for the node records).
+NBodySimProStatus enqueue_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exact,
+                               float* features, NBodySimProError* error) {
     BHState& s = e->bh;
     hipStream_t st = e->stream;
     const int ni = static_cast<int>(s.n);
@@ -2976,26 +3035,6 @@ NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exac
     const float th2 = static_cast<float>(theta2);
     const unsigned* flags = B<unsigned>(s.flags);
     unsigned long long* cnts = B<unsigned long long>(s.counters);
-    // per-query reference-list walk of nq queries (all tree positions, or the
-    // listed ones) on the FP32 pre-order records
-    auto per_query_walk = [&](const int* list, int nq) -> NBodySimProStatus {
-        NBX_TRY(bh_node_records(e, error));
-        const unsigned wblocks = grid_for(static_cast<size_t>(nq), kThreads * kWalkQueries);
-        const unsigned wgrid = (wblocks + kXcds - 1) / kXcds * kXcds;
-        const NodeF32* n32 = B<NodeF32>(s.n32);
-        const int nn = static_cast<int>(s.nodes);
-        if (features != nullptr) {
-            walk_f32_kernel<true, kWalkQueries><<<wgrid, kThreads, 0, st>>>(
-                n32, nn, B<float4>(s.s4), B<uint32_t>(s.tperm), list, nq, Gf, e2, th2, e->ax,
-                e->ay, e->az, cnts, features, gq);
-        } else {
-            walk_f32_kernel<false, kWalkQueries><<<wgrid, kThreads, 0, st>>>(
-                n32, nn, B<float4>(s.s4), B<uint32_t>(s.tperm), list, nq, Gf, e2, th2, e->ax,
-                e->ay, e->az, cnts, nullptr, nullptr);
-        }
-        NBX_HIP(error, hipGetLastError());
-        return N_BODY_SIM_PRO_STATUS_OK;
-    };
     auto group_walk = [&]() {
         const GroupNode* gn = B<GroupNode>(s.gnode);
         int* deferred = B<int32_t>(s.deferred);
@@ -3037,34 +3076,96 @@ NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exac
             }
         }
     };
-    const bool group = !fp64_exact && !(e->flags & NBX_FLAG_BH_REFERENCE_LISTS);
-    const bool lists = !fp64_exact && !group;
+    if (fp64_exact) {
+        walk_f64_kernel<<<blocks, kThreads, 0, st>>>(
+            flags, B<NodeF64>(s.n64), B<double4>(s.sp4), B<uint32_t>(s.tperm), ni,
+            g->gravitational_constant, g->softening_squared, theta2, e->ax, e->ay, e->az, cnts);
+    } else if (!walks_lists(e, fp64_exact)) {
+        group_walk();
+    }
+    NBX_HIP(error, hipGetLastError());
+    return N_BODY_SIM_PRO_STATUS_OK;
+}
+
+}  // namespace
+
+NBodySimProStatus bh_enqueue(Engine* e, const NBodySimProGravity* g, bool fp64_exact, int slot,
+                             NBodySimProError* error) {
+    NBX_TRY(bh_build(e, !fp64_exact, error));
+    NBX_TRY(enqueue_walk(e, g, fp64_exact, nullptr, error));
+    return enqueue_report(e, slot, error);
+}
+
+NBodySimProStatus bh_peek(Engine* e, int slot, bool* clean, NBodySimProError* error) {
+    NBX_TRY(await_report(e, slot, error));
+    *clean = report_clean(report_of(e->bh, slot));
+    return N_BODY_SIM_PRO_STATUS_OK;
+}
+
+bool bh_runs_ahead(const Engine* e, NBXAlgorithm algorithm) {
+    return (algorithm == NBX_ALGORITHM_BARNES_HUT &&
+            (e->flags & NBX_FLAG_BH_REFERENCE_LISTS) == 0) ||
+           algorithm == NBX_ALGORITHM_BARNES_HUT_FP64;
+}
+
+EvaluationGate bh_gate(Engine* e) {
+    return {B<uint4>(e->bh.flags), B<unsigned long long>(e->bh.counters) + 2};
+}
+
+NBodySimProStatus bh_finish(Engine* e, const NBodySimProGravity* g, bool fp64_exact,
+                            float* features, int slot, NBodySimProError* error) {
+    BHState& s = e->bh;
+    hipStream_t st = e->stream;
+    const int ni = static_cast<int>(s.n);
+    const float4* gq = features != nullptr ? B<float4>(s.gquad) : nullptr;
+    const float Gf = static_cast<float>(g->gravitational_constant);
+    const float e2 = static_cast<float>(g->softening_squared);
+    const float th2 = static_cast<float>(e->theta * e->theta);
+    unsigned long long* cnts = B<unsigned long long>(s.counters);
+    // per-query reference-list walk of nq queries (all tree positions, or the
+    // listed ones) on the FP32 pre-order records
+    auto per_query_walk = [&](const int* list, int nq) -> NBodySimProStatus {
+        NBX_TRY(bh_node_records(e, error));
+        const unsigned wblocks = grid_for(static_cast<size_t>(nq), kThreads * kWalkQueries);
+        const unsigned wgrid = (wblocks + kXcds - 1) / kXcds * kXcds;
+        const NodeF32* n32 = B<NodeF32>(s.n32);
+        const int nn = static_cast<int>(s.nodes);
+        if (features != nullptr) {
+            walk_f32_kernel<true, kWalkQueries><<<wgrid, kThreads, 0, st>>>(
+                n32, nn, B<float4>(s.s4), B<uint32_t>(s.tperm), list, nq, Gf, e2, th2, e->ax,
+                e->ay, e->az, cnts, features, gq);
+        } else {
+            walk_f32_kernel<false, kWalkQueries><<<wgrid, kThreads, 0, st>>>(
+                n32, nn, B<float4>(s.s4), B<uint32_t>(s.tperm), list, nq, Gf, e2, th2, e->ax,
+                e->ay, e->az, cnts, nullptr, nullptr);
+        }
+        NBX_HIP(error, hipGetLastError());
+        return N_BODY_SIM_PRO_STATUS_OK;
+    };
+    const bool lists = walks_lists(e, fp64_exact);
+    const bool group = !fp64_exact && !lists;
     float per_query_ms = 0.f;
+    s.slot = slot;
     // Each repetition follows a repaired build: an order on all the bits, then
     // room for its cells, at most.
     bool again = true;
     for (int attempt = 0; again && attempt < 4; ++attempt) {
-        if (fp64_exact) {
-            walk_f64_kernel<<<blocks, kThreads, 0, st>>>(
-                flags, B<NodeF64>(s.n64), B<double4>(s.sp4), B<uint32_t>(s.tperm), ni,
-                g->gravitational_constant, g->softening_squared, theta2, e->ax, e->ay, e->az,
-                cnts);
-        } else if (group) {
-            group_walk();
+        if (attempt > 0) {
+            NBX_TRY(enqueue_walk(e, g, fp64_exact, features, error));
+            NBX_TRY(enqueue_report(e, slot, error));
         }
-        NBX_HIP(error, hipGetLastError());
-        const NBodySimProStatus status = read_build(e, &again, error);
+        const NBodySimProStatus status = read_build(e, slot, &again, error);
         if (status != N_BODY_SIM_PRO_STATUS_OK) {
             s.n = 0;   // no tree
             return status;
         }
+        s.clean = attempt == 0 && !again && report_of(s, slot)->counters[2] == 0;
     }
     if (again) {
         s.n = 0;
         NBX_FAIL(error, N_BODY_SIM_PRO_STATUS_INVALID_STATE, "the tree build did not settle");
     }
-    BuildReport* report = static_cast<BuildReport*>(s.report);
-    const unsigned long long deferred = report->counters[2];
+    const unsigned long long deferred = report_of(s, slot)->counters[2];
     if (lists || (group && deferred > 0)) {
         // Reference lists for all queries, or for those the group walk could
         // not give a shared list (a range the split could not make compact
@@ -3091,11 +3192,18 @@ NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exac
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 
+NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exact, float* features,
+                          NBodySimProError* error) {
+    NBX_TRY(enqueue_walk(e, g, fp64_exact, features, error));
+    NBX_TRY(enqueue_report(e, 0, error));
+    return bh_finish(e, g, fp64_exact, features, 0, error);
+}
+
 void bh_timings(Engine* e) {
     BHState& s = e->bh;
     // the phases' starts on the device clock, a phase that had no kernel at
     // the next one's
-    unsigned long long* at = static_cast<BuildReport*>(s.report)->counters + kCounters;
+    unsigned long long* at = report_of(s, s.slot)->counters + kCounters;
     if (s.walked_lists) {
         at[PHASE_WALK] = at[PHASE_END];
     }
@@ -3122,14 +3230,19 @@ void bh_timings(Engine* e) {
 
 NBodySimProStatus barnes_hut(Engine* e, const NBodySimProGravity* g, bool fp64_exact,
                              NBodySimProError* error) {
-    NBX_TRY(bh_build(e, !fp64_exact, error));
-    NBX_TRY(bh_walk(e, g, fp64_exact, nullptr, error));
+    NBX_TRY(bh_enqueue(e, g, fp64_exact, 0, error));
+    return bh_end(e, g, fp64_exact, 0, error);
+}
+
+NBodySimProStatus bh_end(Engine* e, const NBodySimProGravity* g, bool fp64_exact, int slot,
+                         NBodySimProError* error) {
+    NBX_TRY(bh_finish(e, g, fp64_exact, nullptr, slot, error));
     bh_timings(e);
     // walk bytes: every query reads its position (and permutation entry) and
     // writes 3 doubles; the cell records the walk reads are counted once per
     // launch (they stay in L2 across waves): GroupNode records for the group
     // walk, pre-order node records for the per-query walks.
-    const bool group = !fp64_exact && !(e->flags & NBX_FLAG_BH_REFERENCE_LISTS);
+    const bool group = !fp64_exact && !walks_lists(e, fp64_exact);
     const double node_bytes =
         fp64_exact ? static_cast<double>(e->bh.nodes) * sizeof(NodeF64)
         : group    ? static_cast<double>(e->bh.internal) * sizeof(GroupNode)

@@ -124,16 +124,17 @@ __global__ void kick_drift_kernel(double* __restrict__ px, double* __restrict__ 
 // The kick that ends a step and the kick and drift that begin the next
 // (integrator.c:77-83 and :64-75), with the same two roundings of the
 // velocity: 72 bytes a particle less than the two kernels (1M particles: 14 +
-// 20 us, now 20).
+// 20 us, now 20). Nothing moves unless the gate is open: the evaluation before
+// may have been left unfinished, which the host learns later.
 __global__ void kick_kick_drift_kernel(double* __restrict__ px, double* __restrict__ py,
                                        double* __restrict__ pz, double* __restrict__ vx,
                                        double* __restrict__ vy, double* __restrict__ vz,
                                        const double* __restrict__ ax,
                                        const double* __restrict__ ay,
                                        const double* __restrict__ az, int n, double half,
-                                       double dt) {
+                                       double dt, EvaluationGate gate) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
+    if (i < n && gate.open()) {
         const double hx = ax[i] * half, hy = ay[i] * half, hz = az[i] * half;
         const double nvx = (vx[i] + hx) + hx;
         const double nvy = (vy[i] + hy) + hy;
@@ -387,6 +388,7 @@ bool pinned_both(Engine* e) {
     if (!pinned(&e->bh.report, kReportBytes + bytes)) {
         return false;
     }
+    std::memset(e->bh.report, 0, kReportBytes);
     e->stage = static_cast<char*>(e->bh.report) + kReportBytes;
     e->stage_bytes = bytes;
     e->stage_in_report = true;
@@ -770,32 +772,95 @@ NBodySimProStatus nbx_engine_advance(NBXEngine* engine, NBXAlgorithm algorithm,
     const unsigned g = nbx::grid_for(e->n, nbx::kThreads);
     const double half = 0.5 * timestep;
     NBodySimProStatus st = N_BODY_SIM_PRO_STATUS_OK;
-    for (int k = 0; k < steps && st == N_BODY_SIM_PRO_STATUS_OK; ++k) {
-        e->timed = k + 1 == steps;   // the timings tell of the last evaluation
-        if (integrator == N_BODY_SIM_PRO_INTEGRATOR_EULER) {
-            st = nbx::compute_force(e, algorithm, gravity, error);
-            if (st != N_BODY_SIM_PRO_STATUS_OK) break;
-            nbx::euler_kernel<<<g, nbx::kThreads, 0, e->stream>>>(e->px, e->py, e->pz, e->vx, e->vy,
-                                                                  e->vz, e->ax, e->ay, e->az, n,
-                                                                  timestep);
-            e->pos4_valid = false;
-        } else {
-            // the previous step's closing kick rides along
-            (k == 0 ? nbx::kick_drift_kernel
-                    : nbx::kick_kick_drift_kernel)<<<g, nbx::kThreads, 0, e->stream>>>(
-                e->px, e->py, e->pz, e->vx, e->vy, e->vz, e->ax, e->ay, e->az, n, half, timestep);
-            e->pos4_valid = false;
-            st = nbx::compute_force(e, algorithm, gravity, error);
-            if (st != N_BODY_SIM_PRO_STATUS_OK) break;
-            if (k + 1 == steps) {
-                nbx::kick_kernel<<<g, nbx::kThreads, 0, e->stream>>>(e->vx, e->vy, e->vz, e->ax,
-                                                                     e->ay, e->az, n, half);
-            }
-        }
+    auto launched = [&]() {
         if (hipGetLastError() != hipSuccess) {
             nbx::set_error(error, N_BODY_SIM_PRO_STATUS_INVALID_STATE, __FILE__, __LINE__,
                            "integrator kernel launch failed");
             st = N_BODY_SIM_PRO_STATUS_INVALID_STATE;
+        }
+        return st == N_BODY_SIM_PRO_STATUS_OK;
+    };
+    auto kick_drift = [&](int k, nbx::EvaluationGate gate) {
+        if (k == 0) {
+            nbx::kick_drift_kernel<<<g, nbx::kThreads, 0, e->stream>>>(
+                e->px, e->py, e->pz, e->vx, e->vy, e->vz, e->ax, e->ay, e->az, n, half, timestep);
+        } else {   // the previous step's closing kick rides along
+            nbx::kick_kick_drift_kernel<<<g, nbx::kThreads, 0, e->stream>>>(
+                e->px, e->py, e->pz, e->vx, e->vy, e->vz, e->ax, e->ay, e->az, n, half, timestep,
+                gate);
+        }
+        e->pos4_valid = false;
+        return launched();
+    };
+    auto euler = [&]() {
+        for (int k = 0; k < steps; ++k) {
+            e->timed = k + 1 == steps;   // the timings tell of the last evaluation
+            st = nbx::compute_force(e, algorithm, gravity, error);
+            if (st != N_BODY_SIM_PRO_STATUS_OK) return;
+            nbx::euler_kernel<<<g, nbx::kThreads, 0, e->stream>>>(e->px, e->py, e->pz, e->vx, e->vy,
+                                                                  e->vz, e->ax, e->ay, e->az, n,
+                                                                  timestep);
+            e->pos4_valid = false;
+            if (!launched()) return;
+        }
+    };
+    auto leapfrog = [&]() {
+        for (int k = 0; k < steps; ++k) {
+            if (!kick_drift(k, {nullptr, nullptr})) return;
+            e->timed = k + 1 == steps;
+            st = nbx::compute_force(e, algorithm, gravity, error);
+            if (st != N_BODY_SIM_PRO_STATUS_OK) return;
+        }
+    };
+    // Barnes-Hut: a step is enqueued while the one before it runs, so that the
+    // stream does not stand still while the host reads its report. Where that
+    // evaluation turns out to need the host (a repair of the tree, a
+    // per-query walk), the kick behind it has not moved anything, the
+    // evaluation behind that is the same one again, and the host completes
+    // it; until one goes without the host again, none is run ahead of.
+    // (20 steps with a snapshot, each evaluation read before the next was
+    // enqueued / run ahead: 10,000 particles 3.46 / 3.20 ms, 1M 23.9 / 23.8.)
+    auto leapfrog_ahead = [&]() {
+        const bool fp64 = algorithm == NBX_ALGORITHM_BARNES_HUT_FP64;
+        bool ahead = false;   // the last evaluation enqueued has not been read
+        int slot = 0;
+        int k = 0;
+        while (k < steps) {
+            if (!kick_drift(k, ahead ? nbx::bh_gate(e) : nbx::EvaluationGate{nullptr, nullptr})) {
+                return;
+            }
+            slot ^= 1;
+            st = nbx::bh_enqueue(e, gravity, fp64, slot, error);
+            if (st != N_BODY_SIM_PRO_STATUS_OK) return;
+            bool repeated = false;
+            if (ahead) {
+                bool clean = false;
+                st = nbx::bh_peek(e, slot ^ 1, &clean, error);
+                if (st != N_BODY_SIM_PRO_STATUS_OK) return;
+                repeated = !clean;
+            }
+            if (!repeated) {
+                ++k;
+            }
+            ahead = !repeated && k < steps && e->bh.clean;
+            if (!ahead) {
+                st = nbx::bh_end(e, gravity, fp64, slot, error);
+                if (st != N_BODY_SIM_PRO_STATUS_OK) return;
+            }
+        }
+    };
+    if (integrator == N_BODY_SIM_PRO_INTEGRATOR_EULER) {
+        euler();
+    } else {
+        if (nbx::bh_runs_ahead(e, algorithm)) {
+            leapfrog_ahead();
+        } else {
+            leapfrog();
+        }
+        if (st == N_BODY_SIM_PRO_STATUS_OK && steps > 0) {
+            nbx::kick_kernel<<<g, nbx::kThreads, 0, e->stream>>>(e->vx, e->vy, e->vz, e->ax, e->ay,
+                                                                 e->az, n, half);
+            (void)launched();
         }
     }
     e->timed = true;

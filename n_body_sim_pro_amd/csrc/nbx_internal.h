@@ -113,6 +113,10 @@ struct BHState {
     // pinned host block the evaluation's flags, counts, root cube and
     // interaction counters are reported into (BuildReport, kReportBytes)
     void* report = nullptr;
+    unsigned evaluations = 0;      // reports enqueued so far
+    unsigned number[2] = {0, 0};   // the evaluation that each of the two slots awaits
+    int slot = 0;                  // slot of the last finished evaluation
+    bool clean = false;            // it needed no repair and no per-query walk
     float per_query_ms = 0.f;      // the per-query walk that followed the last walk
     bool walked_lists = false;     // there was no other
     // build inputs (x, y, z, m): FP32-rounded copies of the master arrays
@@ -210,6 +214,30 @@ NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exac
                           float* features, NBodySimProError* error);
 // e->timings and the times in e->stats of the evaluation that bh_walk ended.
 void bh_timings(Engine* e);
+// An evaluation in two halves, for a caller that enqueues the next one before
+// it knows how this one went: the kernels up to the report into one of two
+// slots; then the wait, the repairs, the per-query walk and the times. bh_peek
+// waits for the report alone: clean says that the second half would only read.
+NBodySimProStatus bh_enqueue(Engine* e, const NBodySimProGravity* g, bool fp64_exact, int slot,
+                             NBodySimProError* error);
+NBodySimProStatus bh_peek(Engine* e, int slot, bool* clean, NBodySimProError* error);
+NBodySimProStatus bh_end(Engine* e, const NBodySimProGravity* g, bool fp64_exact, int slot,
+                         NBodySimProError* error);
+// Whether such a caller may do so with this algorithm.
+bool bh_runs_ahead(const Engine* e, NBXAlgorithm algorithm);
+// For the kernel between the two evaluations: whether the first was clean.
+struct EvaluationGate {
+    const uint4* flags;
+    const unsigned long long* deferred;
+    __device__ bool open() const {
+        if (flags == nullptr) {
+            return true;
+        }
+        const uint4 f = *flags;
+        return (f.x | f.y | f.z | f.w) == 0 && *deferred == 0;
+    }
+};
+EvaluationGate bh_gate(Engine* e);
 NBodySimProStatus bh_learned(Engine* e, const NBodySimProGravity* g, NBodySimProError* error);
 
 // Stable LSD radix sort of (64-bit key, 32-bit value) pairs, ascending key;

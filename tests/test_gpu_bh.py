@@ -401,3 +401,42 @@ def test_bh_long_run_next_to_ties_in_a_large_system(nbx, oracle):
     assert np.array_equal(acc, oacc)
     assert stats_tuple(s) == stats_tuple(os_)
     assert np.array_equal(sort_rows(rows), sort_rows(orows))
+
+
+@pytest.mark.parametrize("alg,split", [("hip_barnes_hut", True), ("hip_barnes_hut", False),
+                                       ("hip_barnes_hut_fp64", True)])
+@pytest.mark.parametrize("n", [65, 3000, 40000])
+def test_steps_of_one_call_equal_single_steps(nbx, alg, split, n):
+    """Steps of one call are enqueued before the host has looked at the step
+    before; calls of one step are not. Three pairs of particles share a key at
+    the third step and no other (up to 32768 particles that evaluation's tree
+    needs the host); without the split, groups that are not compact leave
+    their queries to the host in every step."""
+    rng = np.random.default_rng(n)
+    a = {k: rng.uniform(-1, 1, n) for k in ("px", "py", "pz")}
+    a.update({k: rng.normal(scale=0.1, size=n) for k in ("vx", "vy", "vz")})
+    a["m"] = rng.uniform(0.5, 1.5, n) / n
+    dt, g = 1.0e-3, 1.0e-20   # straight lines
+    for i in (0, 2, 4):
+        for k in ("px", "py", "pz", "vx", "vy", "vz"):
+            a[k][i + 1] = a[k][i]
+        a["py"][i + 1] += 1.0e-7
+        a["vx"][i + 1] += 2.0
+        a["px"][i + 1] -= 3.0 * dt * 2.0
+    p = Particles(n, a)
+    results = []
+    for calls in ([1, 1, 1, 1, 1, 1, 1], [7], [3, 4]):
+        with nbx.Engine(n, theta=0.6, split=split) as e:
+            e.upload_view(p.view)
+            e.compute_force(alg, G=g, eps=0.01)
+            for k, steps in enumerate(calls):
+                e.advance(alg, dt=dt, steps=steps, G=g, eps=0.01)
+                if calls[0] == 1 and k in (2, 3):
+                    keys = e.bh_morton()[1]
+                    assert any(keys[i] == keys[i + 1] for i in (0, 2, 4)) == (k == 2)
+            results.append((e.download(), e.stats()))
+    for out, stats in results[1:]:
+        for k in ("pos", "vel", "acc"):
+            assert np.array_equal(out[k], results[0][0][k]), k
+        for k in ("node_count", "maximum_depth", "accepted_approximations", "exact_interactions"):
+            assert stats[k] == results[0][1][k], k
