@@ -52,6 +52,7 @@
 // its reference interaction set, in reference order, with no stack. The FP64
 // variant uses the reference arithmetic and is bit-identical. The default FP32
 // walk is a group walk over the level-indexed cells (group_walk_kernel).
+#include "nbx_exact.h"
 #include "nbx_internal.h"
 
 #include <cstring>
@@ -1031,7 +1032,7 @@ __device__ inline double4 finish_cell(int L, int depth, const double4 (&q)[8],
         a.cy = oy;
         a.cz = oz;
         a.m = mass;
-        a.h = h;
+        a.size2 = 4.0 * h * h;
         a.skip = r.y;
         a.leaf = -1;
         c.n64[r.x] = a;
@@ -1376,7 +1377,7 @@ __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
                     a.cy = q.y;
                     a.cz = q.z;
                     a.m = q.w;
-                    a.h = ldexp(c.root[3], -(level + 1));
+                    a.size2 = 0.0;
                     a.skip = li + 1;
                     a.leaf = t;
                     c.n64[li] = a;
@@ -1644,70 +1645,91 @@ __global__ __launch_bounds__(kThreads) void report_kernel(const unsigned* __rest
 
 // ---------------------------------------------------------------- walk
 // FP64 variant: the reference arithmetic (barnes_hut.c:574-613), bit-identical.
-__global__ __launch_bounds__(kThreads) void walk_f64_kernel(
+// One wave per Q consecutive tree positions, one query per lane; it walks the
+// union of their lists in pre-order, so nodes come through scalar loads, and
+// both nodes that can follow are loaded while a node is tested. The size test
+// alone is the reference's (barnes_hut.c:588 also asks for a distance above
+// zero: no size is below theta^2 times zero, and the one of a NaN neither).
+//
+// The bound is the wave's own chain: some 100 instructions a node, one after
+// the other, over a union of two to four times one query's list. While there
+// are waves to spare it pays to give each fewer queries, whose union is
+// shorter: the smallest Q of 8, 16, 32 and 64 that keeps the waves below two
+// per SIMD. Measured on MI355X, theta 0.7, us with 64 / 32 / 16 / 8 queries a
+// wave, two-galaxy model, in brackets before (64 queries, IEEE square root
+// and divide, no loads ahead):
+//   3,000    201 / 166 / 148 / 127    (241)    10,000   296 / 252 / 216 / 199  (393)
+//   30,000   387 / 326 / 326 / 332    (496)    100,000  556 / 537 / 681 / 1008 (643)
+//   300,000  984 / 1222 / 1793 / 2961 (1190)
+// (Terms noted in lists of 64 and formed four at a time, or held back to form
+// two or four at once, were slower: the instructions that hold them cost more
+// than the overlap gives.)
+template <int Q>
+__global__ __launch_bounds__(kWave) void walk_f64_kernel(
     const unsigned* __restrict__ flags, const NodeF64* __restrict__ n64,
     const double4* __restrict__ sp4,
     const uint32_t* __restrict__ tperm, int n, double G, double eps2, double theta2,
     double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
     unsigned long long* __restrict__ counters) {
-    __shared__ unsigned long long block_counts[2];
     phase_begins(counters, PHASE_WALK);
     if (build_failed(flags)) {
         return;
     }
     const int nodes = n + static_cast<int>(flags[kDCount + kMaxLevels]);
-    if (threadIdx.x < 2) {
-        block_counts[threadIdx.x] = 0;
-    }
-    __syncthreads();
-    const int t = blockIdx.x * kThreads + threadIdx.x;
-    const bool valid = t < n;
-    const int tc = valid ? t : n - 1;
+    const int lane = threadIdx.x;
+    const int t = blockIdx.x * Q + lane;
+    const bool valid = lane < Q && t < n;
     int skip_until = valid ? 0 : 0x7FFFFFFF;
     unsigned approx = 0, exact = 0;
-    const double4 qp = sp4[tc];
+    const double4 qp = sp4[valid ? t : n - 1];
     const double qx = qp.x, qy = qp.y, qz = qp.z;
     double acx = 0.0, acy = 0.0, acz = 0.0;
+    // (barnes_hut.c:593-603)
+    auto add = [&](double dx, double dy, double dz, double d2, double m) {
+        const double r2 = d2 + eps2;
+        double y;
+        const double p = r2 * exact_sqrt(r2, y);
+        double inv3 = exact_recip(p, y * y * y);
+        if (__builtin_amdgcn_ballot_w64(exact_odd(r2, p)) != 0) {
+            asm volatile("");   // a branch, not a select
+            inv3 = 1.0 / (r2 * sqrt(r2));
+        }
+        const double s = G * m * inv3;
+        acx += s * dx;
+        acy += s * dy;
+        acz += s * dz;
+    };
     int i = 0;
+    NodeF64 nd = n64[0];
     while (i < nodes) {
-        const NodeF64 nd = n64[__builtin_amdgcn_readfirstlane(i)];
+        const double dx = nd.cx - qx;
+        const double dy = nd.cy - qy;
+        const double dz = nd.cz - qz;
+        const double d2 = dx * dx + dy * dy + dz * dz;
         const bool active = i >= skip_until;
         if (nd.leaf >= 0) {
+            const NodeF64 next = n64[i + 1];
+            __builtin_amdgcn_sched_barrier(0);
             if (active && nd.leaf != t) {
-                const double dx = nd.cx - qx;
-                const double dy = nd.cy - qy;
-                const double dz = nd.cz - qz;
-                const double r2 = dx * dx + dy * dy + dz * dz + eps2;
-                const double inv3 = 1.0 / (r2 * sqrt(r2));
-                const double s = G * nd.m * inv3;
-                acx += s * dx;
-                acy += s * dy;
-                acz += s * dz;
                 ++exact;
+                add(dx, dy, dz, d2, nd.m);
             }
-            i = i + 1;
+            ++i;
+            nd = next;
         } else {
-            bool descend = false;
-            if (active) {
-                const double dx = nd.cx - qx;
-                const double dy = nd.cy - qy;
-                const double dz = nd.cz - qz;
-                const double d2 = dx * dx + dy * dy + dz * dz;
-                const double size2 = 4.0 * nd.h * nd.h;
-                if (d2 > 0.0 && size2 < theta2 * d2) {
-                    const double r2 = d2 + eps2;
-                    const double inv3 = 1.0 / (r2 * sqrt(r2));
-                    const double s = G * nd.m * inv3;
-                    acx += s * dx;
-                    acy += s * dy;
-                    acz += s * dz;
-                    ++approx;
-                    skip_until = nd.skip;
-                } else {
-                    descend = true;
-                }
+            const int skip = nd.skip;
+            const NodeF64 first = n64[i + 1];
+            const NodeF64 after = n64[skip];
+            __builtin_amdgcn_sched_barrier(0);
+            const bool accept = nd.size2 < theta2 * d2;
+            if (active && accept) {
+                ++approx;
+                skip_until = skip;
+                add(dx, dy, dz, d2, nd.m);
             }
-            i = __ballot(descend) != 0 ? i + 1 : nd.skip;
+            const bool open = __builtin_amdgcn_ballot_w64(active && !accept) != 0;
+            i = open ? i + 1 : skip;
+            nd = open ? first : after;
         }
     }
     if (valid) {
@@ -1715,12 +1737,14 @@ __global__ __launch_bounds__(kThreads) void walk_f64_kernel(
         ax[o] = acx;
         ay[o] = acy;
         az[o] = acz;
-        atomicAdd(&block_counts[0], static_cast<unsigned long long>(approx));
-        atomicAdd(&block_counts[1], static_cast<unsigned long long>(exact));
     }
-    __syncthreads();
-    if (threadIdx.x < 2) {
-        atomicAdd(&counters[threadIdx.x], block_counts[threadIdx.x]);
+    for (int off = 32; off > 0; off >>= 1) {
+        approx += __shfl_xor(approx, off);
+        exact += __shfl_xor(exact, off);
+    }
+    if (lane == 0) {
+        atomicAdd(&counters[0], static_cast<unsigned long long>(approx));
+        atomicAdd(&counters[1], static_cast<unsigned long long>(exact));
     }
 }
 
@@ -2759,8 +2783,8 @@ NBodySimProStatus enqueue_cells(Engine* e, NBodySimProError* error) {
     }
     constexpr bool fp64 = std::is_same_v<In, double4>;
     if (fp64) {
-        // FP64 node records feed only the exact FP64 walk
-        NBX_TRY(s.n64.need<NodeF64>(s.n + s.cells, error));
+        // FP64 node records feed only the exact FP64 walk, which loads one ahead
+        NBX_TRY(s.n64.need<NodeF64>(s.n + s.cells + 1, error));
     }
     CellData<In> c;
     c.gnode = B<GroupNode>(s.gnode);
@@ -3077,9 +3101,22 @@ NBodySimProStatus enqueue_walk(Engine* e, const NBodySimProGravity* g, bool fp64
         }
     };
     if (fp64_exact) {
-        walk_f64_kernel<<<blocks, kThreads, 0, st>>>(
-            flags, B<NodeF64>(s.n64), B<double4>(s.sp4), B<uint32_t>(s.tperm), ni,
-            g->gravitational_constant, g->softening_squared, theta2, e->ax, e->ay, e->az, cnts);
+        auto go = [&](auto kernel, int queries) {
+            kernel<<<grid_for(s.n, queries), kWave, 0, st>>>(
+                flags, B<NodeF64>(s.n64), B<double4>(s.sp4), B<uint32_t>(s.tperm), ni,
+                g->gravitational_constant, g->softening_squared, theta2, e->ax, e->ay, e->az,
+                cnts);
+        };
+        const size_t waves = static_cast<size_t>(e->cu_count) * 8;
+        if (s.n <= 8 * waves) {
+            go(walk_f64_kernel<8>, 8);
+        } else if (s.n <= 16 * waves) {
+            go(walk_f64_kernel<16>, 16);
+        } else if (s.n <= 32 * waves) {
+            go(walk_f64_kernel<32>, 32);
+        } else {
+            go(walk_f64_kernel<64>, 64);
+        }
     } else if (!walks_lists(e, fp64_exact)) {
         group_walk();
     }

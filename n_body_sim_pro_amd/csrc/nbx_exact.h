@@ -72,6 +72,13 @@ __device__ inline double exact_inv_sqrt(double x, ExactGuard& guard) {
     return exact_recip(s, y);
 }
 
+// ExactGuard for one argument x and divisor p.
+__device__ inline bool exact_odd(double x, double p) {
+    const unsigned hi = static_cast<unsigned>(__double2hiint(x));
+    return (hi - (423u << 20) >= (1200u << 20)) |
+           (static_cast<unsigned>(__double2loint(p)) == 0xFFFFFFFFu);
+}
+
 // Softened pair potentials m_i m_j / d_ij (numerics.c:83-116) of target i over
 // the kPotSources sources from j0, those with i < j < n; MASKED unless all of
 // them are. Sources are read through scalar loads, so j0 has to be uniform over

@@ -88,7 +88,7 @@ struct alignas(64) GroupNode {
 // FP64 walk node (exact reference arithmetic).
 struct alignas(16) NodeF64 {
     double cx, cy, cz, m;
-    double h;       // cell half size at this depth
+    double size2;   // 4 h^2, h the half size of a cell (leaves: unused)
     int32_t skip;
     int32_t leaf;
 };

@@ -440,3 +440,19 @@ def test_steps_of_one_call_equal_single_steps(nbx, alg, split, n):
             assert np.array_equal(out[k], results[0][0][k]), k
         for k in ("node_count", "maximum_depth", "accepted_approximations", "exact_interactions"):
             assert stats[k] == results[0][1][k], k
+
+
+@pytest.mark.parametrize("n,eps", [(1, 0.0), (7, 0.0), (9, 0.01), (16384, 0.0), (16385, 0.01),
+                                   (32769, 0.01), (65537, 0.0)])
+def test_exact_walk_at_every_wave_width(nbx, oracle, n, eps):
+    """8, 16, 32 or 64 queries a wave by the system's size: bit for bit the
+    oracle's walk, and its counts."""
+    rng = np.random.default_rng(n)
+    p = Particles(n, {k: rng.normal(size=n) for k in ("px", "py", "pz")})
+    p["m"][:] = rng.uniform(0.5, 1.5, n) / n
+    st, ref, so = oracle_bh(oracle, p, 0.7, eps)[:3]
+    assert st == 0
+    e, acc, s = gpu_bh(nbx, p, 0.7, eps, "hip_barnes_hut_fp64")
+    e.close()
+    assert np.array_equal(acc, ref)
+    assert stats_tuple(s) == stats_tuple(so)
