@@ -91,13 +91,15 @@ void free_buf(Buf& b) {
     b.cap = 0;
 }
 
-// Transfers of up to this many bytes go through the engine's pinned block: one
-// copy by the host and one kernel for all arrays, where a copy command an
-// array costs 6 to 15 us each. (Ten arrays, up / down, with copy commands
-// from pageable, from pinned memory, and staged, us: 1,000 particles 92 / 169,
-// 58 / 59, 16 / 16; 10,000: 114 / 152, 114 / 114, 38 / 44; 30,000: 143 / 215,
-// 141 / 140, 90 / 112. From 60,000 on, 4.8 MB, pinned user memory is as fast:
-// 183 / 181 against 161 / 207.)
+// Transfers of pageable memory of up to this many bytes go through the engine's
+// pinned block: one copy by the host and one kernel for all arrays, where a
+// copy command an array costs 6 to 15 us each; beyond, the host's copy (27
+// GB/s) costs as much. Pinned memory needs no block, the kernel reaches it
+// itself. (Ten arrays, up / down, us. Copy commands from pageable, from pinned
+// memory -> staged, kernel alone: 1,000 particles 92 / 169, 58 / 59 -> 16 / 16,
+// 15 / 14; 10,000: 114 / 152, 114 / 114 -> 38 / 46, 28 / 27; 30,000: 143 / 215,
+// 141 / 140 -> 90 / 113, 57 / 56; 200,000: 519 / 944, 378 / 380 -> -, 313 /
+// 312, which is the link's rate.)
 constexpr size_t kStageBytes = size_t{5} << 19;
 
 // ---------------------------------------------------------------- integrator
@@ -355,20 +357,28 @@ struct ArrayList {
     }
 };
 
-// One array a grid row, between device arrays and their places in the pinned block.
+// One array a grid row, between the device arrays and pinned host memory.
 template <bool TO_HOST>
-__global__ __launch_bounds__(kThreads) void stage_kernel(ArrayList list,
-                                                         double* __restrict__ stage, int n) {
+__global__ __launch_bounds__(kThreads) void stage_kernel(ArrayList list, int n) {
     const int i = blockIdx.x * kThreads + threadIdx.x;
     if (i < n) {
         double* d = list.dev[blockIdx.y] + i;
-        double* h = stage + static_cast<size_t>(blockIdx.y) * n + i;
+        double* h = list.host[blockIdx.y] + i;
         if (TO_HOST) {
             *h = *d;
         } else {
             *d = *h;
         }
     }
+}
+
+template <bool TO_HOST>
+NBodySimProStatus enqueue_stage(Engine* e, const ArrayList& list, size_t n,
+                                NBodySimProError* error) {
+    stage_kernel<TO_HOST><<<dim3(grid_for(n, kThreads), list.count), kThreads, 0, e->stream>>>(
+        list, static_cast<int>(n));
+    NBX_HIP(error, hipGetLastError());
+    return N_BODY_SIM_PRO_STATUS_OK;
 }
 
 // The pinned blocks: bh.report for the evaluations' reports and the stage of
@@ -395,48 +405,81 @@ bool pinned_both(Engine* e) {
     return true;
 }
 
-// Whether a transfer goes through the pinned block.
-bool staged(Engine* e, const ArrayList& list, size_t n) {
-    const size_t bytes = list.count * n * sizeof(double);
-    if (bytes == 0 || bytes > kStageBytes) {
-        return false;
+// How a transfer goes: KERNEL where every host array is pinned memory that
+// the device addresses as the host does (one kernel in place of a copy command
+// an array), STAGED through the engine's pinned block where the host's
+// processor can copy the arrays there, COPIES otherwise.
+enum class Route { KERNEL, STAGED, COPIES };
+
+Route route_of(Engine* e, const ArrayList& list, size_t n) {
+    const size_t bytes = n * sizeof(double);
+    if (list.count == 0 || n == 0) {
+        return Route::COPIES;
+    }
+    int direct = 0;
+    for (int k = 0; k < list.count; ++k) {
+        hipPointerAttribute_t at{};
+        if (hipPointerGetAttributes(&at, list.host[k]) != hipSuccess) {
+            (void)hipGetLastError();   // memory HIP does not know: the host's
+            continue;
+        }
+        if (at.type == hipMemoryTypeDevice) {
+            return Route::COPIES;
+        }
+        if (at.type == hipMemoryTypeHost && at.device == e->device &&
+            at.devicePointer == list.host[k]) {
+            hipDeviceptr_t base = nullptr;
+            size_t size = 0;
+            if (hipMemGetAddressRange(&base, &size, list.host[k]) != hipSuccess) {
+                (void)hipGetLastError();
+                continue;
+            }
+            const char* first = reinterpret_cast<const char*>(list.host[k]);
+            const char* start = static_cast<const char*>(base);
+            direct += first >= start && first + bytes <= start + size;   // the whole array
+        }
+    }
+    if (direct == list.count) {
+        return Route::KERNEL;
+    }
+    if (list.count * bytes > kStageBytes) {
+        return Route::COPIES;
     }
     if (e->stage == nullptr && pinned(&e->stage, kStageBytes)) {
         e->stage_bytes = kStageBytes;
     }
-    if (bytes > e->stage_bytes) {
-        return false;
-    }
-    for (int k = 0; k < list.count; ++k) {
-        // a device pointer in a view is the copy engine's business
-        hipPointerAttribute_t at{};
-        if (hipPointerGetAttributes(&at, list.host[k]) != hipSuccess) {
-            (void)hipGetLastError();   // memory HIP does not know: the host's
-        } else if (at.type == hipMemoryTypeDevice) {
-            return false;
-        }
-    }
-    return true;
+    return list.count * bytes <= e->stage_bytes ? Route::STAGED : Route::COPIES;
 }
 
-// Host -> device. Staged: only enqueued, the block must not be written again
-// before the stream has passed it; *enqueued says so. Else complete.
+ArrayList stage_places(Engine* e, const ArrayList& list, size_t n) {
+    ArrayList places = list;
+    for (int k = 0; k < list.count; ++k) {
+        places.host[k] = static_cast<double*>(e->stage) + k * n;
+    }
+    return places;
+}
+
+// Host -> device. *enqueued: the staged values are on their way, and the
+// pinned block must not be written again before the stream has passed them.
+// Else complete.
 NBodySimProStatus copy_in(Engine* e, const ArrayList& list, size_t n, bool* enqueued,
                           NBodySimProError* error) {
-    *enqueued = staged(e, list, n);
-    if (*enqueued) {
-        double* stage = static_cast<double*>(e->stage);
+    const Route route = route_of(e, list, n);
+    *enqueued = route == Route::STAGED;
+    if (route == Route::STAGED) {
+        const ArrayList places = stage_places(e, list, n);
         for (int k = 0; k < list.count; ++k) {
-            std::memcpy(stage + k * n, list.host[k], n * sizeof(double));
+            std::memcpy(places.host[k], list.host[k], n * sizeof(double));
         }
-        stage_kernel<false><<<dim3(grid_for(n, kThreads), list.count), kThreads, 0, e->stream>>>(
-            list, stage, static_cast<int>(n));
-        NBX_HIP(error, hipGetLastError());
-        return N_BODY_SIM_PRO_STATUS_OK;
+        return enqueue_stage<false>(e, places, n, error);
     }
-    for (int k = 0; k < list.count && n > 0; ++k) {
-        NBX_HIP(error, hipMemcpyAsync(list.dev[k], list.host[k], n * sizeof(double),
-                                      hipMemcpyHostToDevice, e->stream));
+    if (route == Route::KERNEL) {
+        NBX_TRY(enqueue_stage<false>(e, list, n, error));
+    } else {
+        for (int k = 0; k < list.count && n > 0; ++k) {
+            NBX_HIP(error, hipMemcpyAsync(list.dev[k], list.host[k], n * sizeof(double),
+                                          hipMemcpyHostToDevice, e->stream));
+        }
     }
     NBX_HIP(error, hipStreamSynchronize(e->stream));
     return N_BODY_SIM_PRO_STATUS_OK;
@@ -444,20 +487,23 @@ NBodySimProStatus copy_in(Engine* e, const ArrayList& list, size_t n, bool* enqu
 
 // Device -> host, complete on return.
 NBodySimProStatus copy_out(Engine* e, const ArrayList& list, size_t n, NBodySimProError* error) {
-    if (staged(e, list, n)) {
-        double* stage = static_cast<double*>(e->stage);
-        stage_kernel<true><<<dim3(grid_for(n, kThreads), list.count), kThreads, 0, e->stream>>>(
-            list, stage, static_cast<int>(n));
-        NBX_HIP(error, hipGetLastError());
+    const Route route = route_of(e, list, n);
+    if (route == Route::STAGED) {
+        const ArrayList places = stage_places(e, list, n);
+        NBX_TRY(enqueue_stage<true>(e, places, n, error));
         NBX_HIP(error, hipStreamSynchronize(e->stream));
         for (int k = 0; k < list.count; ++k) {
-            std::memcpy(list.host[k], stage + k * n, n * sizeof(double));
+            std::memcpy(list.host[k], places.host[k], n * sizeof(double));
         }
         return N_BODY_SIM_PRO_STATUS_OK;
     }
-    for (int k = 0; k < list.count && n > 0; ++k) {
-        NBX_HIP(error, hipMemcpyAsync(list.host[k], list.dev[k], n * sizeof(double),
-                                      hipMemcpyDeviceToHost, e->stream));
+    if (route == Route::KERNEL) {
+        NBX_TRY(enqueue_stage<true>(e, list, n, error));
+    } else {
+        for (int k = 0; k < list.count && n > 0; ++k) {
+            NBX_HIP(error, hipMemcpyAsync(list.host[k], list.dev[k], n * sizeof(double),
+                                          hipMemcpyDeviceToHost, e->stream));
+        }
     }
     NBX_HIP(error, hipStreamSynchronize(e->stream));
     return N_BODY_SIM_PRO_STATUS_OK;

@@ -79,6 +79,37 @@ def test_transfers_bring_every_array(nbx, n, capacity):
         assert np.array_equal(part["m"], c["m"])
 
 
+@pytest.mark.parametrize("n,pinned", [(1, 10), (257, 10), (32768, 7), (40001, 10), (40001, 3)])
+def test_transfers_of_pinned_arrays(nbx, n, pinned):
+    """Arrays in pinned memory are reached by the kernel itself, all or none:
+    with a pageable one among them the other routes serve."""
+    names = ("px", "py", "pz", "vx", "vy", "vz", "ax", "ay", "az", "m")
+    rng = np.random.default_rng(n)
+    lib = nbx.load()   # (symbols of the HIP runtime it is linked to, too)
+    lib.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+    lib.hipHostFree.argtypes = [C.c_void_p]
+
+    def arrays():
+        block = C.c_void_p()
+        assert lib.hipHostMalloc(C.byref(block), pinned * (n + 1) * 8, 0) == 0
+        rows = np.ctypeslib.as_array(C.cast(block, C.POINTER(C.c_double)), (pinned, n + 1))
+        rows[:] = np.nan
+        columns = [r[1:] for r in rows] + [np.full(n, np.nan) for _ in range(10 - pinned)]
+        return block, rows, dict(zip(names, columns))
+
+    block_a, _, a = arrays()
+    block_b, rows_b, b = arrays()
+    for k in names:
+        a[k][:] = rng.normal(size=n)
+    with nbx.Engine(n) as e:
+        e.upload_view(nbx.make_view(n, **a))
+        e.download_view(nbx.make_view(n, **b))
+    for k in names:
+        assert np.array_equal(a[k], b[k]), k
+    assert np.all(np.isnan(rows_b[:, 0]))   # nothing before the arrays was touched
+    assert lib.hipHostFree(block_a) == 0 and lib.hipHostFree(block_b) == 0
+
+
 def test_all_pairs_advance_times_its_last_evaluation(nbx):
     p = Particles(500, {k: np.random.default_rng(7).normal(size=500) for k in ("px", "py", "pz", "m")})
     for alg, per in (("hip_direct_fp64", 56.0), ("hip_direct_fp32", 40.0)):
