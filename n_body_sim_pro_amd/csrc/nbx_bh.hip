@@ -705,14 +705,51 @@ __global__ void place_kernel(const uint32_t* __restrict__ order, const uint64_t*
 // position t starts the cells of depths (delta[t-1], delta[t]] and ends those
 // of depths (delta[t], delta[t-1]]; cells of one depth are disjoint, so the
 // k-th start of depth d and the k-th end of depth d belong to the same cell.
-// The topology kernels give each workgroup one tile of kTopoTile consecutive
+// The topology kernels give each workgroup one tile of 256 to 1024 consecutive
 // positions: per-tile counts of starts and ends per depth, scanned over the
 // tiles, plus wave ballots inside a tile, give every start and end its rank
 // in position order, with no search and no shared global counters.
-constexpr int kTopoItems = 4;
-constexpr int kTopoTile = kThreads * kTopoItems;
+//
+// A small system is the chain of one tile (its levels, deepest first), so its
+// tiles are shorter; a large one has several tiles a CU, and longer ones leave
+// fewer cells that span tiles. Measured on MI355X, tree and centre-of-mass
+// phases, two-galaxy / uniform cloud, us with tiles of 256, 512 and 1024:
+//   8,000    50 / 41, 52 / 43, 58 / 48       24,000   65 / 51, 54 / 45, 65 / 53
+//   60,000   69 / 57, 67 / 55, 68 / 56       200,000  80 / 67, 76 / 68, 82 / 72
+//   400,000  101 / 90, 99 / 86, 90 / 79
+// (256 up to the 64 tiles that one workgroup's span launch covers.)
+template <int POSITIONS, int THREADS>
+struct Tile {
+    static constexpr int kPositions = POSITIONS;
+    static constexpr int kBuildThreads = THREADS;                  // of build_kernel
+    static constexpr int kBuildItems = POSITIONS / THREADS;
+    static constexpr int kBuildWaves = THREADS / kWave;
+    static constexpr int kChunks = POSITIONS / kWave;              // 64-position chunks
+    static constexpr int kLocalCells = POSITIONS / 4 * 3;   // cells a tile can hold in LDS
+                                                            // (usually about half as many as
+                                                            // positions)
+    static_assert(POSITIONS % kThreads == 0 && POSITIONS % THREADS == 0, "whole items");
+};
+using TileSmall = Tile<256, 256>;
+using TileMedium = Tile<512, 512>;
+using TileLarge = Tile<1024, 512>;
 constexpr int kTopoWaves = kThreads / kWave;
-constexpr int kTopoChunks = kTopoTile / kWave;   // 64-position chunks of a tile
+constexpr int kSpanTiles = 64;   // tiles of a span_com_kernel workgroup
+
+// Positions of a tile for n particles.
+inline int tile_positions(size_t n, int cu_count) {
+    return n <= static_cast<size_t>(kSpanTiles) * TileSmall::kPositions ? TileSmall::kPositions
+           : n <= static_cast<size_t>(cu_count) * TileLarge::kPositions ? TileMedium::kPositions
+                                                                        : TileLarge::kPositions;
+}
+
+// f(Tile) for that choice.
+template <typename F>
+auto with_tile(int positions, F f) {
+    return positions == TileSmall::kPositions    ? f(TileSmall{})
+           : positions == TileMedium::kPositions ? f(TileMedium{})
+                                                 : f(TileLarge{});
+}
 // Rows of the per-tile counts: cells started and ended per depth, and all the
 // cells started.
 constexpr int kEndRow = kMaxLevels;
@@ -760,6 +797,7 @@ __device__ inline int wave_max_int(int v) {
 
 // delta[t] = common levels of tree positions t and t+1 (-1 for the last);
 // tile_hist[row * tiles + b] = tile b's counts.
+template <int POSITIONS>
 __global__ __launch_bounds__(kThreads) void delta_kernel(const uint64_t* __restrict__ w,
                                                         const uint64_t* __restrict__ ext, int n,
                                                         int tiles, int32_t* __restrict__ delta,
@@ -781,8 +819,8 @@ __global__ __launch_bounds__(kThreads) void delta_kernel(const uint64_t* __restr
     __syncthreads();
     unsigned mine = 0;
     int cells = 0;
-    for (int i = 0; i < kTopoItems; ++i) {
-        const int t = blockIdx.x * kTopoTile + i * kThreads + threadIdx.x;
+    for (int i = 0; i < POSITIONS / kThreads; ++i) {
+        const int t = blockIdx.x * POSITIONS + i * kThreads + threadIdx.x;
         if (t >= n) {
             break;
         }
@@ -1114,27 +1152,25 @@ __device__ inline void com_node(int L, int depth, const CellData<In>& c) {
 // (k = 1) of depth d in the earlier chunks of the tile; base and next: those
 // of the earlier tiles, without and with this one; local: number of the
 // tile's first cell of depth d among the cells it starts.
-constexpr int kBuildThreads = 512;
-constexpr int kBuildItems = kTopoTile / kBuildThreads;
-constexpr int kBuildWaves = kBuildThreads / kWave;
-constexpr int kLocalCells = 768;   // cells a tile can hold in LDS (usually about 500)
+template <typename T>
 struct TileRanks {
-    unsigned short wcount[2][kTopoChunks][kMaxLevels + 1];
+    unsigned short wcount[2][T::kChunks][kMaxLevels + 1];
     unsigned doff[kMaxLevels];
     unsigned base[2][kMaxLevels];
     unsigned next[2][kMaxLevels];
     unsigned local[kMaxLevels];
-    unsigned chunk_cells[kTopoChunks];
+    unsigned chunk_cells[T::kChunks];
     int deepest;
     unsigned cells;
 };
 
 // The tile's part of the tree in LDS: its particles, and the child tables and
 // centres of mass of the cells that start in it. A child is -1 for none, a
-// position of the tile, or kTopoTile + the number of one of the tile's cells.
+// position of the tile, or T::kPositions + the number of one of the tile's cells.
+template <typename T>
 struct TileCells {
-    double4 item[kTopoTile + kLocalCells];
-    short kids[kLocalCells][8];
+    double4 item[T::kPositions + T::kLocalCells];
+    short kids[T::kLocalCells][8];
 };
 
 // A workgroup barrier that orders LDS only: global stores stay in flight (a
@@ -1171,19 +1207,22 @@ __device__ inline void empty_slots(int32_t* kids, int lo, int hi) {
 // -(tree position + 2); -1 for none) is written slot by slot by several
 // workgroups: every child writes its own slot and the empty ones up to the
 // child before it (children come in descending octant order), the cell's last
-// position those below its last child. A tile with more than kLocalCells
+// position those below its last child. A tile with more than T::kLocalCells
 // cells treats them all like that and sums the local ones from memory.
 //
 // Measured on MI355X: separate launches for ends, starts and every depth took
 // 18 + 20 + 100 us at 1M, and at 10,000 particles 13 + 35 us.
-template <bool QUAD, typename In>
-__global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
+template <bool QUAD, typename In, typename T>
+__global__ __launch_bounds__(T::kBuildThreads, 4) void build_kernel(
     const uint64_t* __restrict__ w, const uint64_t* __restrict__ ext,
     const int32_t* __restrict__ delta, int n, int tiles, int cell_capacity,
     unsigned* __restrict__ flags, const unsigned* __restrict__ tile_base,
     uint32_t* __restrict__ scan, CellData<In> c) {
-    __shared__ TileRanks r;
-    __shared__ TileCells tc;
+    constexpr int kTopoTile = T::kPositions, kTopoChunks = T::kChunks;
+    constexpr int kBuildThreads = T::kBuildThreads, kBuildItems = T::kBuildItems;
+    constexpr int kBuildWaves = T::kBuildWaves, kLocalCells = T::kLocalCells;
+    __shared__ TileRanks<T> r;
+    __shared__ TileCells<T> tc;
     if (build_failed(flags)) {
         return;
     }
@@ -1447,7 +1486,6 @@ __global__ __launch_bounds__(kBuildThreads, 4) void build_kernel(
 // takes from LDS when its depth's turn comes. (Finding and summing each
 // depth's cells from memory: 46 and 33 us for the two launches at 1M.) More
 // cells, units or depths than the tables hold are summed that way.
-constexpr int kSpanTiles = 64;
 constexpr int kSpanLevels = 40;
 template <int T>
 struct SpanTable {
@@ -1460,7 +1498,7 @@ struct SpanTable {
     unsigned present[kMaxLevels];
 };
 
-template <bool QUAD, typename In, int T>
+template <bool QUAD, typename In, int T, int POSITIONS>
 __global__ __launch_bounds__(T) void span_com_kernel(int unit_tiles, int group_units, int tiles,
                                                      const unsigned* __restrict__ flags,
                                                      const unsigned* __restrict__ tile_base,
@@ -1494,7 +1532,7 @@ __global__ __launch_bounds__(T) void span_com_kernel(int unit_tiles, int group_u
     __syncthreads();
     const int unit0 = blockIdx.x * group_units;
     const int units = min(group_units, (tiles + unit_tiles - 1) / unit_tiles - unit0);
-    const int limit = min((unit0 + group_units) * unit_tiles, tiles) * kTopoTile;
+    const int limit = min((unit0 + group_units) * unit_tiles, tiles) * POSITIONS;
     const int levels = s.deepest + 1;
     // level index of the cell of depth d that starts in unit u and ends past
     // it, or -1
@@ -1558,7 +1596,7 @@ __global__ __launch_bounds__(T) void span_com_kernel(int unit_tiles, int group_u
 #pragma unroll
         for (int o = 0; o < 8; ++o) {
             own[o] = -1;
-            const int u = first[o] / (unit_tiles * kTopoTile) - unit0;
+            const int u = first[o] / (unit_tiles * POSITIONS) - unit0;
             if (kid[o] >= 0 && depth + 1 < levels && u >= 0 && u < units) {
                 const int e = s.at[depth + 1][u];
                 own[o] = e >= 0 && s.cell[e].x == kid[o] ? e : -1;
@@ -2754,11 +2792,13 @@ NBodySimProStatus enqueue_depths(Engine* e, NBodySimProError* error) {
     BHState& s = e->bh;
     hipStream_t st = e->stream;
     const int ni = static_cast<int>(s.n);
-    const int nt = static_cast<int>((s.n + kTopoTile - 1) / kTopoTile);
+    const int nt = static_cast<int>(grid_for(s.n, s.tile));
     unsigned* flags = B<unsigned>(s.flags);
-    delta_kernel<<<nt, kThreads, 0, st>>>(B<uint64_t>(s.tword), s.ext_tree, ni, nt,
-                                          B<int32_t>(s.delta), flags, B<unsigned>(s.tile_hist),
-                                          B<unsigned long long>(s.counters));
+    with_tile(s.tile, [&](auto tile) {
+        delta_kernel<decltype(tile)::kPositions><<<nt, kThreads, 0, st>>>(
+            B<uint64_t>(s.tword), s.ext_tree, ni, nt, B<int32_t>(s.delta), flags,
+            B<unsigned>(s.tile_hist), B<unsigned long long>(s.counters));
+    });
     depth_scan_kernel<<<kTopoRows, kThreads, 0, st>>>(B<unsigned>(s.tile_hist), nt,
                                                       B<unsigned>(s.tile_base), flags);
     NBX_HIP(error, hipGetLastError());
@@ -2771,7 +2811,7 @@ NBodySimProStatus enqueue_cells(Engine* e, NBodySimProError* error) {
     BHState& s = e->bh;
     hipStream_t st = e->stream;
     const int ni = static_cast<int>(s.n);
-    const int nt = static_cast<int>((s.n + kTopoTile - 1) / kTopoTile);
+    const int nt = static_cast<int>(grid_for(s.n, s.tile));
     NBX_TRY(s.icom.need<double4>(s.cells, error));
     NBX_TRY(s.irec.need<int4>(s.cells, error));
     NBX_TRY(s.idepth.need<int32_t>(s.cells, error));
@@ -2799,18 +2839,22 @@ NBodySimProStatus enqueue_cells(Engine* e, NBodySimProError* error) {
     unsigned* flags = B<unsigned>(s.flags);
     const unsigned* base = B<unsigned>(s.tile_base);
     unsigned long long* cnts = B<unsigned long long>(s.counters);
-    build_kernel<QUAD, In><<<nt, kBuildThreads, 0, st>>>(
-        B<uint64_t>(s.tword), s.ext_tree, B<int32_t>(s.delta), ni, nt, static_cast<int>(s.cells),
-        flags, base, B<uint32_t>(s.scan), c);
-    if (nt > 1) {
-        span_com_kernel<QUAD, In, 512><<<grid_for(nt, kSpanTiles), 512, 0, st>>>(
-            1, kSpanTiles, nt, flags, base, c, cnts);
-    }
-    if (nt > kSpanTiles) {
-        const int units = (nt + kSpanTiles - 1) / kSpanTiles;
-        span_com_kernel<QUAD, In, 1024><<<1, 1024, 0, st>>>(kSpanTiles, units, nt, flags, base, c,
-                                                           cnts);
-    }
+    with_tile(s.tile, [&](auto tile) {
+        using T = decltype(tile);
+        constexpr int kPositions = T::kPositions;
+        build_kernel<QUAD, In, T><<<nt, T::kBuildThreads, 0, st>>>(
+            B<uint64_t>(s.tword), s.ext_tree, B<int32_t>(s.delta), ni, nt,
+            static_cast<int>(s.cells), flags, base, B<uint32_t>(s.scan), c);
+        if (nt > 1) {
+            span_com_kernel<QUAD, In, 512, kPositions><<<grid_for(nt, kSpanTiles), 512, 0, st>>>(
+                1, kSpanTiles, nt, flags, base, c, cnts);
+        }
+        if (nt > kSpanTiles) {
+            const int units = (nt + kSpanTiles - 1) / kSpanTiles;
+            span_com_kernel<QUAD, In, 1024, kPositions><<<1, 1024, 0, st>>>(
+                kSpanTiles, units, nt, flags, base, c, cnts);
+        }
+    });
     NBX_HIP(error, hipGetLastError());
     return N_BODY_SIM_PRO_STATUS_OK;
 }
@@ -2960,7 +3004,8 @@ NBodySimProStatus bh_build(Engine* e, bool fp32_inputs, NBodySimProError* error,
         NBX_HIP(error, hipHostMalloc(&s.report, kReportBytes, hipHostMallocDefault));
         std::memset(s.report, 0, kReportBytes);   // no evaluation's number
     }
-    const size_t tiles = (n + kTopoTile - 1) / kTopoTile;
+    s.tile = tile_positions(n, e->cu_count);
+    const size_t tiles = grid_for(n, s.tile);
     NBX_TRY(s.tile_hist.need<unsigned>(kTopoRows * tiles, error));
     NBX_TRY(s.tile_base.need<unsigned>(kTopoRows * tiles, error));
     // Room for the cells of usual inputs (about n / 2); a tree with more
@@ -3244,7 +3289,7 @@ void bh_timings(Engine* e) {
     if (s.walked_lists) {
         at[PHASE_WALK] = at[PHASE_END];
     }
-    if (s.n <= static_cast<size_t>(kTopoTile)) {
+    if (s.n <= static_cast<size_t>(s.tile)) {
         at[PHASE_COM] = at[PHASE_WALK];
     }
     auto ms = [&](int from, int to) {

@@ -102,6 +102,7 @@ struct BHState {
     size_t nodes = 0;         // n + internal
     size_t cells = 0;         // internal cells the record buffers are sized for
     size_t cells_n = 0;       // the particle count that size was chosen for
+    int tile = 0;             // tree positions of a topology kernel's workgroup
     int max_depth = 0;
     bool has_n64 = false;     // the last build wrote FP64 node records
     bool has_quad = false;    // the last build wrote quadrupole records

@@ -456,3 +456,21 @@ def test_exact_walk_at_every_wave_width(nbx, oracle, n, eps):
     e.close()
     assert np.array_equal(acc, ref)
     assert stats_tuple(s) == stats_tuple(so)
+
+
+@pytest.mark.parametrize("n", [256, 257, 16384, 16385, 262144, 262145])
+def test_tree_at_every_tile_size(nbx, oracle, n):
+    """256, 512 or 1024 positions a workgroup of the topology kernels by the
+    system's size: every cell's record bit for bit the oracle's."""
+    rng = np.random.default_rng(n)
+    p = Particles(n, {k: rng.normal(size=n) for k in ("px", "py", "pz")})
+    p["m"][:] = rng.uniform(0.5, 1.5, n) / n
+    st, oacc, os_, _, _, oroot, orows = oracle_bh(oracle, p, 1.2, 0.01)
+    assert st == 0
+    e, acc, s = gpu_bh(nbx, p, 1.2, 0.01, "hip_barnes_hut_fp64")
+    root, _, _ = e.bh_morton()
+    rows = e.bh_export_nodes()
+    e.close()
+    assert np.array_equal(root, oroot) and stats_tuple(s) == stats_tuple(os_)
+    assert np.array_equal(sort_rows(rows), sort_rows(orows))
+    assert np.array_equal(acc, oacc)
