@@ -88,8 +88,8 @@ typedef struct NBXConfig {
     uint32_t flags;   /* NBX_FLAG_* bits, 0 for the defaults */
 } NBXConfig;
 
-/* Per-evaluation timings (ms): HIP events on the engine's stream, for the
- * phases of a Barnes-Hut evaluation the device's wall clock. */
+/* Per-evaluation timings (ms) by the device's wall clock; HIP events for the
+ * learned correction, per-query walks and a whole advance(). */
 typedef struct NBXTimings {
     double force_ms;      /* whole force evaluation */
     double bbox_keys_ms;  /* BH: bounding cube + keys */

@@ -1654,7 +1654,7 @@ struct BuildReport {
     unsigned long long counters[kCounters + kPhases];
     unsigned number;   // of the evaluation, written last: the host waits for it
 };
-static_assert(2 * sizeof(BuildReport) <= kReportBytes, "the engine's pinned block holds a report");
+static_assert(2 * sizeof(BuildReport) <= kClocksAt, "the engine's pinned block holds a report");
 
 __global__ __launch_bounds__(kThreads) void report_kernel(const unsigned* __restrict__ flags,
                                                           const double* __restrict__ root,
@@ -3000,10 +3000,6 @@ NBodySimProStatus bh_build(Engine* e, bool fp32_inputs, NBodySimProError* error,
     NBX_TRY(s.s4.need<float4>(n, error));
     NBX_TRY(s.counters.need<unsigned long long>(kCounters + kPhases, error));
     NBX_TRY(s.deferred.need<int32_t>(n, error));
-    if (s.report == nullptr) {
-        NBX_HIP(error, hipHostMalloc(&s.report, kReportBytes, hipHostMallocDefault));
-        std::memset(s.report, 0, kReportBytes);   // no evaluation's number
-    }
     s.tile = tile_positions(n, e->cu_count);
     const size_t tiles = grid_for(n, s.tile);
     NBX_TRY(s.tile_hist.need<unsigned>(kTopoRows * tiles, error));

@@ -153,7 +153,9 @@ __global__ void kick_kick_drift_kernel(double* __restrict__ px, double* __restri
 __global__ void kick_kernel(double* __restrict__ vx, double* __restrict__ vy,
                             double* __restrict__ vz, const double* __restrict__ ax,
                             const double* __restrict__ ay, const double* __restrict__ az, int n,
-                            double half) {
+                            double half,
+                            unsigned long long* __restrict__ clock) {
+    clock_in(clock);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
         vx[i] = vx[i] + ax[i] * half;
@@ -167,7 +169,9 @@ __global__ void euler_kernel(double* __restrict__ px, double* __restrict__ py,
                              double* __restrict__ pz, double* __restrict__ vx,
                              double* __restrict__ vy, double* __restrict__ vz,
                              const double* __restrict__ ax, const double* __restrict__ ay,
-                             const double* __restrict__ az, int n, double dt) {
+                             const double* __restrict__ az, int n, double dt,
+                             unsigned long long* __restrict__ clock) {
+    clock_in(clock);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
         px[i] = px[i] + vx[i] * dt;
@@ -359,7 +363,11 @@ struct ArrayList {
 
 // One array a grid row, between the device arrays and pinned host memory.
 template <bool TO_HOST>
-__global__ __launch_bounds__(kThreads) void stage_kernel(ArrayList list, int n) {
+__global__ __launch_bounds__(kThreads) void stage_kernel(ArrayList list, int n,
+                                                         unsigned long long* __restrict__ clock) {
+    if (blockIdx.y == 0) {
+        clock_in(clock);
+    }
     const int i = blockIdx.x * kThreads + threadIdx.x;
     if (i < n) {
         double* d = list.dev[blockIdx.y] + i;
@@ -376,15 +384,14 @@ template <bool TO_HOST>
 NBodySimProStatus enqueue_stage(Engine* e, const ArrayList& list, size_t n,
                                 NBodySimProError* error) {
     stage_kernel<TO_HOST><<<dim3(grid_for(n, kThreads), list.count), kThreads, 0, e->stream>>>(
-        list, static_cast<int>(n));
+        list, static_cast<int>(n), TO_HOST ? direct_end(e) : nullptr);
     NBX_HIP(error, hipGetLastError());
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 
-// The pinned blocks: bh.report for the evaluations' reports and the stage of
-// the small transfers, each allocated on first use. An allocation takes 260 us
-// and more, so an engine that can stage all it holds gets one block for both
-// when it is created.
+// Pinned memory. An engine that can stage all it holds gets one block for the
+// reports and the stage when it is created (an allocation takes 260 us and
+// more); a larger one gets its stage with its first small transfer.
 bool pinned(void** p, size_t bytes) {
     if (*p == nullptr && hipHostMalloc(p, bytes, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
@@ -393,15 +400,18 @@ bool pinned(void** p, size_t bytes) {
     return *p != nullptr;
 }
 
-bool pinned_both(Engine* e) {
+bool pinned_report(Engine* e) {
     const size_t bytes = e->capacity * 10 * sizeof(double);
-    if (!pinned(&e->bh.report, kReportBytes + bytes)) {
+    const bool both = e->capacity <= kStageBytes / (10 * sizeof(double));
+    if (!pinned(&e->bh.report, kReportBytes + (both ? bytes : 0))) {
         return false;
     }
-    std::memset(e->bh.report, 0, kReportBytes);
-    e->stage = static_cast<char*>(e->bh.report) + kReportBytes;
-    e->stage_bytes = bytes;
-    e->stage_in_report = true;
+    std::memset(e->bh.report, 0, kReportBytes);   // no evaluation's number
+    if (both) {
+        e->stage = static_cast<char*>(e->bh.report) + kReportBytes;
+        e->stage_bytes = bytes;
+        e->stage_in_report = true;
+    }
     return true;
 }
 
@@ -500,6 +510,7 @@ NBodySimProStatus copy_out(Engine* e, const ArrayList& list, size_t n, NBodySimP
     if (route == Route::KERNEL) {
         NBX_TRY(enqueue_stage<true>(e, list, n, error));
     } else {
+        NBX_TRY(direct_timings(e, error));   // (the copies are no part of the evaluation)
         for (int k = 0; k < list.count && n > 0; ++k) {
             NBX_HIP(error, hipMemcpyAsync(list.host[k], list.dev[k], n * sizeof(double),
                                           hipMemcpyDeviceToHost, e->stream));
@@ -517,6 +528,7 @@ NBXEngine* g_default = nullptr;
 NBodySimProStatus compute_force(Engine* e, NBXAlgorithm algorithm, const NBodySimProGravity* g,
                                 NBodySimProError* error) {
     e->pending = 0;
+    e->ended = false;
     switch (algorithm) {
         case NBX_ALGORITHM_DIRECT_FP64:
             return direct_fp64(e, g, error);
@@ -634,9 +646,7 @@ NBXEngine* nbx_engine_create(const NBXConfig* config, NBodySimProError* error) {
     for (auto& ev : e->ev) {
         ok = ok && hipEventCreate(&ev) == hipSuccess;
     }
-    if (e->capacity <= nbx::kStageBytes / (10 * sizeof(double))) {
-        ok = ok && nbx::pinned_both(e);
-    }
+    ok = ok && nbx::pinned_report(e);
     if (!ok) {
         nbx::set_error(error, N_BODY_SIM_PRO_STATUS_OUT_OF_MEMORY, __FILE__, __LINE__,
                        "device allocation failed while creating the engine");
@@ -845,7 +855,7 @@ NBodySimProStatus nbx_engine_advance(NBXEngine* engine, NBXAlgorithm algorithm,
             if (st != N_BODY_SIM_PRO_STATUS_OK) return;
             nbx::euler_kernel<<<g, nbx::kThreads, 0, e->stream>>>(e->px, e->py, e->pz, e->vx, e->vy,
                                                                   e->vz, e->ax, e->ay, e->az, n,
-                                                                  timestep);
+                                                                  timestep, nbx::direct_end(e));
             e->pos4_valid = false;
             if (!launched()) return;
         }
@@ -905,7 +915,7 @@ NBodySimProStatus nbx_engine_advance(NBXEngine* engine, NBXAlgorithm algorithm,
         }
         if (st == N_BODY_SIM_PRO_STATUS_OK && steps > 0) {
             nbx::kick_kernel<<<g, nbx::kThreads, 0, e->stream>>>(e->vx, e->vy, e->vz, e->ax, e->ay,
-                                                                 e->az, n, half);
+                                                                 e->az, n, half, nbx::direct_end(e));
             (void)launched();
         }
     }

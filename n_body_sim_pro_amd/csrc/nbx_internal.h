@@ -94,6 +94,7 @@ struct alignas(16) NodeF64 {
 };
 
 constexpr size_t kReportBytes = 4096;
+constexpr size_t kClocksAt = kReportBytes - 64;   // the all-pairs evaluations' clocks
 
 // Barnes-Hut device workspace (all sized by particle or node capacity).
 struct BHState {
@@ -112,7 +113,7 @@ struct BHState {
     const uint64_t* ext_tree = nullptr;   // tree-order extension words or null (ext below)
     double root[4] = {0, 0, 0, 1};
     // pinned host block the evaluation's flags, counts, root cube and
-    // interaction counters are reported into (BuildReport, kReportBytes)
+    // interaction counters are reported into (BuildReport), kReportBytes
     void* report = nullptr;
     unsigned evaluations = 0;      // reports enqueued so far
     unsigned number[2] = {0, 0};   // the evaluation that each of the two slots awaits
@@ -187,7 +188,8 @@ struct Engine {
     // all-pairs evaluations: what direct_timings has to read, and whether the
     // coming one is to be timed at all
     bool timed = true;
-    int pending = 0;          // 0 nothing, else the number of events recorded
+    int pending = 0;          // 0 nothing, 2 FP64, 3 FP32, 4 FP32 after its staging launch
+    bool ended = false;       // its end has been marked and waited for
     // learned BH correction
     void* mlp = nullptr;
 };
@@ -198,7 +200,12 @@ struct Engine {
 NBodySimProStatus direct_fp64(Engine* e, const NBodySimProGravity* g, NBodySimProError* error);
 NBodySimProStatus direct_fp32(Engine* e, const NBodySimProGravity* g, NBodySimProError* error);
 NBodySimProStatus direct_timings(Engine* e, NBodySimProError* error);
-NBodySimProStatus refresh_pos4(Engine* e, NBodySimProError* error);
+// Where the kernel that follows an evaluation whose times are wanted writes the
+// device clock as it begins (null: none is); the caller then waits for it
+// before direct_timings.
+unsigned long long* direct_end(Engine* e);
+NBodySimProStatus refresh_pos4(Engine* e, NBodySimProError* error,
+                               unsigned long long* clock = nullptr);
 NBodySimProStatus barnes_hut(Engine* e, const NBodySimProGravity* g, bool fp64_exact,
                              NBodySimProError* error);
 NBodySimProStatus bh_build(Engine* e, bool fp32_inputs, NBodySimProError* error,
@@ -258,6 +265,13 @@ NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals
 __device__ inline unsigned lanes_below(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
                                      __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0u));
+}
+
+// The device clock as a kernel begins, from its first workgroup (null: not asked for).
+__device__ inline void clock_in(unsigned long long* __restrict__ clock) {
+    if (clock != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
+        *clock = static_cast<unsigned long long>(wall_clock64());
+    }
 }
 
 inline unsigned grid_for(size_t n, unsigned block) {
