@@ -423,8 +423,8 @@ enum class Route { KERNEL, STAGED, COPIES };
 
 Route route_of(Engine* e, const ArrayList& list, size_t n) {
     const size_t bytes = n * sizeof(double);
-    if (list.count == 0 || n == 0) {
-        return Route::COPIES;
+    if (list.count == 0 || n == 0 || n > 0x7FFFFF00u) {
+        return Route::COPIES;   // (the kernel's positions are ints)
     }
     int direct = 0;
     for (int k = 0; k < list.count; ++k) {
