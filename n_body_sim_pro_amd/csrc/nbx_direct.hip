@@ -538,10 +538,10 @@ __global__ void refresh_pos4_kernel(const double* __restrict__ px, const double*
 template <bool ZERO_EPS>
 void launch_direct_fp32(hipStream_t st, const double* px, const double* py, const double* pz,
                         const double* m, const float4* pos, double* ax, double* ay, double* az,
-                        int n, double G, float eps2, unsigned long long* clock) {
+                        int n, double G, float eps2, bool staged, unsigned long long* clock) {
     if (n <= kSmallN) {
         const unsigned grid = grid_for(static_cast<size_t>(n), kSmallTargets);
-        if (n <= kStageN) {
+        if (!staged) {
             direct_fp32_small_kernel<ZERO_EPS, true><<<grid, kSmallWaves * kWave, 0, st>>>(
                 px, py, pz, m, pos, ax, ay, az, n, G, eps2, clock);
         } else {
@@ -557,17 +557,18 @@ void launch_direct_fp32(hipStream_t st, const double* px, const double* py, cons
             pos, ax, ay, az, n, G, eps2, kSourceTile);
 }
 
-// The FP32 all-pairs evaluation on staged positions (unused up to kStageN).
+// The FP32 all-pairs evaluation; staged: `pos` holds the positions (always
+// beyond kStageN, where one workgroup's LDS does not).
 void launch_direct_fp32(hipStream_t st, const double* px, const double* py, const double* pz,
                         const double* m, const float4* pos, double* ax, double* ay, double* az,
-                        int n, const NBodySimProGravity* g,
+                        int n, const NBodySimProGravity* g, bool staged,
                         unsigned long long* clock = nullptr) {
     const double G = g->gravitational_constant;
     const float eps2 = static_cast<float>(g->softening_squared);
     if (eps2 > 0.f) {
-        launch_direct_fp32<false>(st, px, py, pz, m, pos, ax, ay, az, n, G, eps2, clock);
+        launch_direct_fp32<false>(st, px, py, pz, m, pos, ax, ay, az, n, G, eps2, staged, clock);
     } else {
-        launch_direct_fp32<true>(st, px, py, pz, m, pos, ax, ay, az, n, G, eps2, clock);
+        launch_direct_fp32<true>(st, px, py, pz, m, pos, ax, ay, az, n, G, eps2, staged, clock);
     }
 }
 
@@ -621,7 +622,8 @@ NBodySimProStatus direct_fp32(Engine* e, const NBodySimProGravity* g, NBodySimPr
         NBX_TRY(refresh_pos4(e, error, e->timed ? clocks_of(e) : nullptr));
     }
     launch_direct_fp32(e->stream, e->px, e->py, e->pz, e->m, e->pos4, e->ax, e->ay, e->az,
-                       static_cast<int>(n), g, e->timed ? clocks_of(e) + 1 : nullptr);
+                       static_cast<int>(n), g, n > static_cast<size_t>(kStageN),
+                       e->timed ? clocks_of(e) + 1 : nullptr);
     NBX_HIP(error, hipGetLastError());
     e->pending = e->timed ? (stages ? 4 : 3) : 0;
     return N_BODY_SIM_PRO_STATUS_OK;
@@ -720,6 +722,20 @@ constexpr size_t kNoAllocMaxParticles = size_t(1) << 20;
 constexpr int kNoAllocMaxDevices = 64;
 std::mutex g_noalloc_mutex;
 void* g_noalloc_staging[kNoAllocMaxDevices] = {};
+
+// Whether any of the outputs (n doubles each) covers part of an input.
+bool outputs_over_inputs(const double* const (&in)[4], double* const (&out)[3], size_t n) {
+    const uintptr_t bytes = n * sizeof(double);
+    for (const double* i : in) {
+        for (const double* o : out) {
+            const uintptr_t a = reinterpret_cast<uintptr_t>(i), b = reinterpret_cast<uintptr_t>(o);
+            if (a < b + bytes && b < a + bytes) {
+                return true;
+            }
+        }
+    }
+    return false;
+}
 }  // namespace
 }  // namespace nbx
 
@@ -764,13 +780,20 @@ extern "C" NBodySimProStatus nbx_direct_fp32_noalloc(
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int n = static_cast<int>(count);
-    if (count > static_cast<size_t>(nbx::kStageN)) {
+    // Accelerations may take the place of the inputs: then every input is read
+    // by a launch of its own, also where each workgroup would read them all
+    // itself while others store.
+    const bool staged =
+        count > static_cast<size_t>(nbx::kStageN) ||
+        nbx::outputs_over_inputs({positions_x, positions_y, positions_z, masses},
+                                 {accelerations_x, accelerations_y, accelerations_z}, count);
+    if (staged) {
         nbx::refresh_pos4_kernel<<<nbx::grid_for(count, 256), 256, 0, st>>>(
             positions_x, positions_y, positions_z, masses, staging, n, nullptr);
     }
     // the same kernels as nbx_hip_direct_fp32 (identical results)
     nbx::launch_direct_fp32(st, positions_x, positions_y, positions_z, masses, staging,
-                            accelerations_x, accelerations_y, accelerations_z, n, gravity);
+                            accelerations_x, accelerations_y, accelerations_z, n, gravity, staged);
     NBX_HIP(error, hipGetLastError());
     return N_BODY_SIM_PRO_STATUS_OK;
 }

@@ -104,6 +104,30 @@ def test_noalloc_unsoftened_matches_direct_fp32(nbx):
     assert np.array_equal(a, _engine(nbx, d["pos"], d["m"], 1.0, 0.0))
 
 
+@pytest.mark.parametrize("n,shift", [(1, 0), (17, 0), (1000, 0), (1000, 3), (4096, 16), (4097, 0)])
+def test_noalloc_outputs_in_place_of_the_inputs(nbx, n, shift):
+    """Accelerations stored over positions and masses, also some elements off:
+    every input is read before the first output is written."""
+    d = nbx.plummer(n, seed=n)
+    want = _engine(nbx, d["pos"], d["m"], 1.0, 0.01)
+    fn = _bind(nbx.load())
+    hip = _Hip(nbx)
+    print(f"noalloc in place: N={n}, outputs {shift} elements into y, z and m", flush=True)
+    try:
+        # x | y | z | m | spare, and the outputs from y + shift on
+        p = hip.put(np.concatenate([*d["pos"].T, d["m"], np.zeros(shift)])).value
+        at = [p + 8 * n * k for k in range(4)]
+        out = [p + 8 * (n * (k + 1) + shift) for k in range(3)]
+        err = Error()
+        st = fn(*at, *out, n, C.byref(gravity(1.0, 0.01)), None, C.byref(err))
+        assert st == 0, err.message
+        assert hip.lib.hipDeviceSynchronize() == 0
+        got = np.stack([hip.get(o, n) for o in out], axis=1)
+    finally:
+        hip.free()
+    assert np.array_equal(got, want)
+
+
 def test_noalloc_rejects_oversize_and_missing_arguments(nbx):
     """Rejected on the host before any device work (the pointers are never used)."""
     fn = _bind(nbx.load())
