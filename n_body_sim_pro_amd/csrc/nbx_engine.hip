@@ -415,13 +415,29 @@ bool pinned_report(Engine* e) {
     return true;
 }
 
+// Whether two host arrays of a transfer share memory.
+bool host_arrays_overlap(const ArrayList& list, size_t bytes) {
+    for (int k = 1; k < list.count; ++k) {
+        for (int j = 0; j < k; ++j) {
+            const uintptr_t a = reinterpret_cast<uintptr_t>(list.host[k]);
+            const uintptr_t b = reinterpret_cast<uintptr_t>(list.host[j]);
+            if (a < b + bytes && b < a + bytes) {
+                return true;
+            }
+        }
+    }
+    return false;
+}
+
 // How a transfer goes: KERNEL where every host array is pinned memory that
 // the device addresses as the host does (one kernel in place of a copy command
 // an array), STAGED through the engine's pinned block where the host's
-// processor can copy the arrays there, COPIES otherwise.
+// processor can copy the arrays there, COPIES otherwise. The kernel stores the
+// arrays in any order: to host arrays that share memory it does not go, so the
+// later array of the view stays where they do.
 enum class Route { KERNEL, STAGED, COPIES };
 
-Route route_of(Engine* e, const ArrayList& list, size_t n) {
+Route route_of(Engine* e, const ArrayList& list, size_t n, bool to_host) {
     const size_t bytes = n * sizeof(double);
     if (list.count == 0 || n == 0 || n > 0x7FFFFF00u) {
         return Route::COPIES;   // (the kernel's positions are ints)
@@ -449,7 +465,7 @@ Route route_of(Engine* e, const ArrayList& list, size_t n) {
             direct += first >= start && first + bytes <= start + size;   // the whole array
         }
     }
-    if (direct == list.count) {
+    if (direct == list.count && !(to_host && host_arrays_overlap(list, bytes))) {
         return Route::KERNEL;
     }
     if (list.count * bytes > kStageBytes) {
@@ -474,7 +490,7 @@ ArrayList stage_places(Engine* e, const ArrayList& list, size_t n) {
 // Else complete.
 NBodySimProStatus copy_in(Engine* e, const ArrayList& list, size_t n, bool* enqueued,
                           NBodySimProError* error) {
-    const Route route = route_of(e, list, n);
+    const Route route = route_of(e, list, n, false);
     *enqueued = route == Route::STAGED;
     if (route == Route::STAGED) {
         const ArrayList places = stage_places(e, list, n);
@@ -497,7 +513,7 @@ NBodySimProStatus copy_in(Engine* e, const ArrayList& list, size_t n, bool* enqu
 
 // Device -> host, complete on return.
 NBodySimProStatus copy_out(Engine* e, const ArrayList& list, size_t n, NBodySimProError* error) {
-    const Route route = route_of(e, list, n);
+    const Route route = route_of(e, list, n, true);
     if (route == Route::STAGED) {
         const ArrayList places = stage_places(e, list, n);
         NBX_TRY(enqueue_stage<true>(e, places, n, error));

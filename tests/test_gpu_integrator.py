@@ -110,6 +110,31 @@ def test_transfers_of_pinned_arrays(nbx, n, pinned):
     assert lib.hipHostFree(block_a) == 0 and lib.hipHostFree(block_b) == 0
 
 
+@pytest.mark.parametrize("n,shift", [(1, 0), (257, 0), (257, 100), (40001, 0), (40001, 7)])
+def test_download_into_pinned_arrays_that_share_memory(nbx, n, shift):
+    """The view's later array stays, as with one copy after the other: vx, vy
+    and vz go `shift` elements apart into one pinned block, x to another."""
+    rng = np.random.default_rng(n)
+    src = {k: rng.normal(size=n) for k in ("px", "py", "pz", "vx", "vy", "vz", "m")}
+    lib = nbx.load()
+    lib.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+    lib.hipHostFree.argtypes = [C.c_void_p]
+    block = C.c_void_p()
+    words = 2 * n + 2 * shift
+    assert lib.hipHostMalloc(C.byref(block), words * 8, 0) == 0
+    host = np.ctypeslib.as_array(C.cast(block, C.POINTER(C.c_double)), (words,))
+    host[:] = np.nan
+    want = np.full(n + 2 * shift, np.nan)
+    for k, name in enumerate(("vx", "vy", "vz")):
+        want[k * shift:k * shift + n] = src[name]
+    at = {name: host[n + k * shift:2 * n + k * shift] for k, name in enumerate(("vx", "vy", "vz"))}
+    with nbx.Engine(n) as e:
+        e.upload_view(nbx.make_view(n, **src))
+        e.download_view(nbx.make_view(n, px=host[:n], **at))
+    assert np.array_equal(host[:n], src["px"]) and np.array_equal(host[n:], want)
+    assert lib.hipHostFree(block) == 0
+
+
 def test_all_pairs_advance_times_its_last_evaluation(nbx):
     p = Particles(500, {k: np.random.default_rng(7).normal(size=500) for k in ("px", "py", "pz", "m")})
     for alg, per in (("hip_direct_fp64", 56.0), ("hip_direct_fp32", 40.0)):
