@@ -936,13 +936,15 @@ NBodySimProStatus nbx_engine_advance(NBXEngine* engine, NBXAlgorithm algorithm,
         }
     }
     e->timed = true;
-    (void)hipEventRecord(t1, e->stream);
-    (void)hipEventSynchronize(t1);
+    hipError_t done = hipEventRecord(t1, e->stream);
+    const hipError_t waited = hipEventSynchronize(t1);
+    done = done != hipSuccess ? done : waited;
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, t0, t1);
     (void)hipEventDestroy(t0);
     (void)hipEventDestroy(t1);
     if (st == N_BODY_SIM_PRO_STATUS_OK) {
+        NBX_HIP(error, done);   // all-pairs steps were not waited for before
         st = nbx::direct_timings(e, error);
     }
     e->timings.integrate_ms = ms;
