@@ -2963,6 +2963,22 @@ NBodySimProStatus read_build(Engine* e, int slot, bool* again, NBodySimProError*
 
 }  // namespace
 
+namespace {
+
+// No tree to report on after an evaluation that could not be enqueued or read:
+// s.n is the coming tree's already, its node counts still the last one's.
+NBodySimProStatus or_no_tree(Engine* e, NBodySimProStatus status) {
+    if (status != N_BODY_SIM_PRO_STATUS_OK) {
+        e->bh.n = 0;
+    }
+    return status;
+}
+
+NBodySimProStatus enqueue_build(Engine* e, bool fp32_inputs, bool quadrupoles,
+                                NBodySimProError* error);
+
+}  // namespace
+
 // Enqueues the whole build. No host read: the kernels of the build and of the
 // walk that follows check the flag words, and bh_walk reads them once at its
 // end (the read between the per-depth counts and the cell records left the
@@ -2982,6 +2998,15 @@ NBodySimProStatus bh_build(Engine* e, bool fp32_inputs, NBodySimProError* error,
     if (n > 0x3FFFFFFFull) {
         NBX_FAIL(error, N_BODY_SIM_PRO_STATUS_INVALID_ARGUMENT, "particle count exceeds 2^30");
     }
+    return or_no_tree(e, enqueue_build(e, fp32_inputs, quadrupoles, error));
+}
+
+namespace {
+
+NBodySimProStatus enqueue_build(Engine* e, bool fp32_inputs, bool quadrupoles,
+                                NBodySimProError* error) {
+    BHState& s = e->bh;
+    const size_t n = e->n;
     // build inputs: float4 for FP32-rounded inputs, double4 for FP64 ones
     NBX_TRY(s.b4.need<char>(n * (fp32_inputs ? sizeof(float4) : sizeof(double4)), error));
     NBX_TRY(s.partial.need<double>(6 * kBBoxBlocks + 8, error));
@@ -3018,6 +3043,8 @@ NBodySimProStatus bh_build(Engine* e, bool fp32_inputs, NBodySimProError* error,
     NBX_TRY(enqueue_depths(e, error));
     return enqueue_cells(e, error);
 }
+
+}  // namespace
 
 NBodySimProStatus bh_node_records(Engine* e, NBodySimProError* error) {
     BHState& s = e->bh;
@@ -3170,12 +3197,12 @@ NBodySimProStatus enqueue_walk(Engine* e, const NBodySimProGravity* g, bool fp64
 NBodySimProStatus bh_enqueue(Engine* e, const NBodySimProGravity* g, bool fp64_exact, int slot,
                              NBodySimProError* error) {
     NBX_TRY(bh_build(e, !fp64_exact, error));
-    NBX_TRY(enqueue_walk(e, g, fp64_exact, nullptr, error));
-    return enqueue_report(e, slot, error);
+    NBX_TRY(or_no_tree(e, enqueue_walk(e, g, fp64_exact, nullptr, error)));
+    return or_no_tree(e, enqueue_report(e, slot, error));
 }
 
 NBodySimProStatus bh_peek(Engine* e, int slot, bool* clean, NBodySimProError* error) {
-    NBX_TRY(await_report(e, slot, error));
+    NBX_TRY(or_no_tree(e, await_report(e, slot, error)));
     *clean = report_clean(report_of(e->bh, slot));
     return N_BODY_SIM_PRO_STATUS_OK;
 }
@@ -3229,14 +3256,10 @@ NBodySimProStatus bh_finish(Engine* e, const NBodySimProGravity* g, bool fp64_ex
     bool again = true;
     for (int attempt = 0; again && attempt < 4; ++attempt) {
         if (attempt > 0) {
-            NBX_TRY(enqueue_walk(e, g, fp64_exact, features, error));
-            NBX_TRY(enqueue_report(e, slot, error));
+            NBX_TRY(or_no_tree(e, enqueue_walk(e, g, fp64_exact, features, error)));
+            NBX_TRY(or_no_tree(e, enqueue_report(e, slot, error)));
         }
-        const NBodySimProStatus status = read_build(e, slot, &again, error);
-        if (status != N_BODY_SIM_PRO_STATUS_OK) {
-            s.n = 0;   // no tree
-            return status;
-        }
+        NBX_TRY(or_no_tree(e, read_build(e, slot, &again, error)));
         s.clean = attempt == 0 && !again && report_of(s, slot)->counters[2] == 0;
     }
     if (again) {
@@ -3272,8 +3295,8 @@ NBodySimProStatus bh_finish(Engine* e, const NBodySimProGravity* g, bool fp64_ex
 
 NBodySimProStatus bh_walk(Engine* e, const NBodySimProGravity* g, bool fp64_exact, float* features,
                           NBodySimProError* error) {
-    NBX_TRY(enqueue_walk(e, g, fp64_exact, features, error));
-    NBX_TRY(enqueue_report(e, 0, error));
+    NBX_TRY(or_no_tree(e, enqueue_walk(e, g, fp64_exact, features, error)));
+    NBX_TRY(or_no_tree(e, enqueue_report(e, 0, error)));
     return bh_finish(e, g, fp64_exact, features, 0, error);
 }
 

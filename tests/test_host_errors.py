@@ -66,3 +66,24 @@ assert fails(lambda: e.advance("{algorithm}", dt=1e-3, steps=3, integrator={inte
 hip.hip_double_fail(b"hipEventSynchronize", 0, 719)
 assert fails(lambda: e.advance("{algorithm}", dt=1e-3, steps=3, integrator={integrator})) == INVALID_STATE
 """)
+
+
+@pytest.mark.parametrize("algorithm", ["hip_barnes_hut", "hip_barnes_hut_fp64"])
+@pytest.mark.parametrize("n", [5000, 40000])
+def test_no_tree_after_an_evaluation_out_of_memory(double, algorithm, n):
+    """Whichever allocation of an evaluation fails, there is no tree to report
+    on after it: the counts of the last one would not fit the new arrays."""
+    run(double, f"""
+hip.hip_double_left.restype = C.c_int
+k = 0
+while True:
+    e = engine({n})
+    hip.hip_double_fail(b"hipMalloc", k, 2)
+    status = fails(lambda: e.compute_force("{algorithm}"))
+    if hip.hip_double_left() >= 0:
+        break
+    assert status == OUT_OF_MEMORY, (k, status)
+    assert fails(e.bh_morton) == INVALID_STATE, k
+    k += 1
+assert k > 15, k
+""")
