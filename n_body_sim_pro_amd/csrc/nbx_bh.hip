@@ -384,14 +384,18 @@ __device__ inline void place(int t, uint64_t key, uint32_t o, const In* __restri
 // four of the seven 9-bit passes); order_kernel then orders each run of equal
 // top bits by the low kSortLowBits and puts every particle at its tree
 // position. The runs are short (two-galaxy input: at most 10 particles at 1M,
-// 53 at 10M). A run longer than kFinishRun raises FLAG_LONG_RUN, and the host
-// orders on all the bits after reading the flags.
+// 53 at 10M). A run longer than kFinishRun raises FLAG_LONG_RUN: the host, after
+// reading the flags, sorts on all 63 bits (an escaper far out is enough: a
+// Plummer sphere of 100,000 and one particle at 600 scale radii), and only where
+// more than kFinishRun particles share a whole key on the extension words too.
+// (Measured on MI355X, that input: 0.49 ms an evaluation, 0.30 without the
+// escaper; 1.25 with the extension words of every particle sorted at once.)
 constexpr int kSortLowBits = 27;
 constexpr int kSortTopBits = 63 - kSortLowBits;
 constexpr int kFinishRun = 64;
 static_assert(kSortTopBits % 9 == 0, "whole 9-bit radix passes");
 
-// Input: sorted (stably, from index order) by key >> kSortLowBits. Element p
+// Input: sorted (stably, from index order) by key >> low_bits. Element p
 // goes to its run's first position plus the number of run members before it
 // in key order. Members that share the whole key are ordered by their deeper
 // digits, and their extension words go to ext (nobody reads a position's
@@ -404,20 +408,20 @@ __global__ __launch_bounds__(kThreads) void order_kernel(
     const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin, int n,
     const In* __restrict__ b4, const double* __restrict__ root, uint32_t* __restrict__ tperm,
     uint64_t* __restrict__ tword, uint64_t* __restrict__ ext, double4* __restrict__ sp4,
-    float4* __restrict__ s4, unsigned* __restrict__ flags) {
+    float4* __restrict__ s4, unsigned* __restrict__ flags, int low_bits) {
     const int p = blockIdx.x * kThreads + threadIdx.x;
     if (p >= n) {
         return;
     }
     const uint64_t key = kin[p];
-    const uint64_t top = key >> kSortLowBits;
+    const uint64_t top = key >> low_bits;
     // the run's bounds, at most kFinishRun steps to each side
     int a = p;
-    while (a > 0 && p - a < kFinishRun && (kin[a - 1] >> kSortLowBits) == top) {
+    while (a > 0 && p - a < kFinishRun && (kin[a - 1] >> low_bits) == top) {
         --a;
     }
     int b = p;
-    while (b < n - 1 && b - p < kFinishRun && (kin[b + 1] >> kSortLowBits) == top) {
+    while (b < n - 1 && b - p < kFinishRun && (kin[b + 1] >> low_bits) == top) {
         ++b;
     }
     int dst = p;
@@ -655,7 +659,8 @@ __global__ __launch_bounds__(kThreads) void merge_order_kernel(
     }
 }
 
-// ---- ordering on all the bits (FLAG_LONG_RUN, or FLAG_TIE of a small system)
+// ---- ordering on the extension words too (FLAG_LONG_RUN after a sort on all the
+// key bits, or FLAG_TIE of a small system)
 template <typename In>
 __global__ void ext_words_kernel(const In* __restrict__ b4, int n,
                                  const double* __restrict__ root, uint64_t* __restrict__ ext) {
@@ -2699,6 +2704,18 @@ const In* tree_inputs(BHState& s) {
     }
 }
 
+// Tree positions from the particles in sk0/sv0, sorted by key >> low_bits.
+template <typename In>
+void enqueue_runs(Engine* e, int low_bits) {
+    BHState& s = e->bh;
+    order_kernel<In><<<grid_for(s.n, kThreads), kThreads, 0, e->stream>>>(
+        B<uint64_t>(s.sk0), B<uint32_t>(s.sv0), static_cast<int>(s.n), B<In>(s.b4), root_of(s),
+        B<uint32_t>(s.tperm), B<uint64_t>(s.tword), B<uint64_t>(s.ext),
+        std::is_same_v<In, double4> ? B<double4>(s.sp4) : nullptr, B<float4>(s.s4),
+        B<unsigned>(s.flags), low_bits);
+    s.sorted_low_bits = low_bits;
+}
+
 // The bounding cube, the keys and the tree order of e's particles.
 template <typename In>
 NBodySimProStatus enqueue_order(Engine* e, NBodySimProError* error) {
@@ -2723,6 +2740,7 @@ NBodySimProStatus enqueue_order(Engine* e, NBodySimProError* error) {
             B<uint64_t>(s.sk0), B<uint32_t>(s.sv0), ni, b4, B<uint32_t>(s.tperm),
             B<uint64_t>(s.tword), sp4, B<float4>(s.s4));
         s.ext_tree = nullptr;   // a shared key raises FLAG_TIE
+        s.sorted_low_bits = 0;
     } else {
         keys_kernel<In><<<g < 1024u ? g : 1024u, kThreads, 0, st>>>(
             b4, ni, B<double>(s.partial), static_cast<int>(bb_blocks), root, B<uint64_t>(s.sk0));
@@ -2735,16 +2753,26 @@ NBodySimProStatus enqueue_order(Engine* e, NBodySimProError* error) {
                                  B<uint32_t>(s.sv1), s.n, kSortTopBits, s.hist, error, nullptr,
                                  nullptr, kSortLowBits, true,
                                  cnts + kCounters + PHASE_SORT));
-        order_kernel<In><<<g, kThreads, 0, st>>>(B<uint64_t>(s.sk0), B<uint32_t>(s.sv0), ni, b4,
-                                                 root, B<uint32_t>(s.tperm), B<uint64_t>(s.tword),
-                                                 B<uint64_t>(s.ext), sp4, B<float4>(s.s4), flags);
+        enqueue_runs<In>(e, kSortLowBits);
         s.ext_tree = B<uint64_t>(s.ext);
     }
     NBX_HIP(error, hipGetLastError());
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 
-// The same order on all the bits: (key, ext0, ..., ext5), least significant
+// The same order after FLAG_LONG_RUN, from a sort on all the key bits: sk0 and sv0
+// still hold the pairs, stably sorted on the top ones from index order.
+template <typename In>
+NBodySimProStatus enqueue_key_order(Engine* e, NBodySimProError* error) {
+    BHState& s = e->bh;
+    NBX_TRY(radix_sort_pairs(e->stream, B<uint64_t>(s.sk0), B<uint32_t>(s.sv0),
+                             B<uint64_t>(s.sk1), B<uint32_t>(s.sv1), s.n, 63, s.hist, error));
+    enqueue_runs<In>(e, 0);
+    NBX_HIP(error, hipGetLastError());
+    return N_BODY_SIM_PRO_STATUS_OK;
+}
+
+// The same order from all the words: (key, ext0, ..., ext5), least significant
 // word first, stable from index order.
 template <typename In>
 NBodySimProStatus enqueue_full_order(Engine* e, NBodySimProError* error) {
@@ -2925,8 +2953,13 @@ NBodySimProStatus read_build(Engine* e, int slot, bool* again, NBodySimProError*
     *again = false;
     if (report->flags[FLAG_LONG_RUN] != 0 || report->flags[FLAG_TIE] != 0) {
         NBX_HIP(error, hipMemsetAsync(flags, 0, kFlagWords * sizeof(unsigned), st));
-        NBX_TRY(s.inputs_fp64 ? enqueue_full_order<double4>(e, error)
-                              : enqueue_full_order<float4>(e, error));
+        if (s.sorted_low_bits > 0) {
+            NBX_TRY(s.inputs_fp64 ? enqueue_key_order<double4>(e, error)
+                                  : enqueue_key_order<float4>(e, error));
+        } else {
+            NBX_TRY(s.inputs_fp64 ? enqueue_full_order<double4>(e, error)
+                                  : enqueue_full_order<float4>(e, error));
+        }
         NBX_TRY(enqueue_depths(e, error));
         *again = true;
         return enqueue_cells(e, error);
@@ -3251,8 +3284,8 @@ NBodySimProStatus bh_finish(Engine* e, const NBodySimProGravity* g, bool fp64_ex
     const bool group = !fp64_exact && !lists;
     float per_query_ms = 0.f;
     s.slot = slot;
-    // Each repetition follows a repaired build: an order on all the bits, then
-    // room for its cells, at most.
+    // Each repetition follows a repaired build: an order on all the key bits,
+    // then on the extension words too, then room for its cells, at most.
     bool again = true;
     for (int attempt = 0; again && attempt < 4; ++attempt) {
         if (attempt > 0) {

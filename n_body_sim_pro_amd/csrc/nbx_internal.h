@@ -103,6 +103,7 @@ struct BHState {
     size_t nodes = 0;         // n + internal
     size_t cells = 0;         // internal cells the record buffers are sized for
     size_t cells_n = 0;       // the particle count that size was chosen for
+    int sorted_low_bits = 0;  // key bits below the last build's radix sort
     int tile = 0;             // tree positions of a topology kernel's workgroup
     int max_depth = 0;
     bool has_n64 = false;     // the last build wrote FP64 node records
@@ -129,13 +130,13 @@ struct BHState {
     Buf sk0, sk1, sv0, sv1;   // sort ping-pong
     Buf hist;                 // sort histograms
     Buf mkey;                 // Morton keys in original order, on demand (true-path keys while
-                              // an order on all the bits is made)
+                              // an order on all the words is made)
     Buf mperm;                // Morton order: sorted position -> original index, on demand
     Buf tperm;                // tree position -> original index
     Buf tword;                // tree-order true keys (descending)
     Buf ext;                  // extension key words (6 per tree position; only those of
                               // positions that share their key with a neighbour are read)
-    Buf ext_orig;             // the same in original order (order on all the bits)
+    Buf ext_orig;             // the same in original order (order on all the words)
     Buf delta;                // int32 common levels between tree positions t, t+1
     Buf scan;                 // internal cells started before each tree position
     Buf sp4;                  // tree-order FP64 (x, y, z, m), FP64 builds only

@@ -403,6 +403,51 @@ def test_bh_long_run_next_to_ties_in_a_large_system(nbx, oracle):
     assert np.array_equal(sort_rows(rows), sort_rows(orows))
 
 
+def device_bytes(e):
+    e.lib.nbx_engine_device_bytes.argtypes = [C.c_void_p]
+    e.lib.nbx_engine_device_bytes.restype = C.c_size_t
+    return e.lib.nbx_engine_device_bytes(e.h)
+
+
+@pytest.mark.parametrize("case", ["escaper", "core", "one_key"])
+def test_bh_long_runs(nbx, oracle, case):
+    """Runs of equal top key bits too long for the order kernel. An escaper far
+    out: sorted on all the key bits, in the memory that the system takes
+    without it. A core of 300 particles among them that shares fewer levels, and
+    100 particles that share a whole key: on the extension words too."""
+    n = 40000
+    rng = np.random.default_rng(5)
+    pos = rng.normal(size=(n, 3))
+    m = rng.uniform(0.5, 1.0, n)
+    base = pos.copy()
+    pos[7] = [3000.0, -2000.0, 1000.0]
+    if case == "core":
+        pos[100:400] = [0.3, 0.2, 0.1] + rng.uniform(-1e-2, 1e-2, (300, 3))
+    elif case == "one_key":
+        pos[100:200] = [0.3, 0.2, 0.1] + rng.uniform(-1e-8, 1e-8, (100, 3))
+    p = Particles(n, {"px": pos[:, 0], "py": pos[:, 1], "pz": pos[:, 2], "m": m})
+    st, oacc, os_, okeys, operm, oroot, orows = oracle_bh(oracle, p, 0.7, 0.01)
+    assert st == 0
+    with nbx.Engine(n, theta=0.7) as e:
+        e.upload(base, m)
+        e.compute_force("hip_barnes_hut_fp64", eps=0.01)
+        without = device_bytes(e)
+    with nbx.Engine(n, theta=0.7) as e:
+        e.upload_view(p.view)
+        for _ in range(2):
+            e.compute_force("hip_barnes_hut_fp64", eps=0.01)
+            assert np.array_equal(e.accelerations(), oacc)
+            assert stats_tuple(e.stats()) == stats_tuple(os_)
+        assert case != "escaper" or device_bytes(e) == without
+        root, keys, perm = e.bh_morton()
+        rows = e.bh_export_nodes()
+    top = np.unique(okeys >> np.uint64(27), return_counts=True)[1].max()
+    assert top > 64 and (case != "one_key" or np.unique(okeys, return_counts=True)[1].max() > 64)
+    assert np.array_equal(root, oroot) and np.array_equal(keys, okeys)
+    assert np.array_equal(perm, operm)
+    assert np.array_equal(sort_rows(rows), sort_rows(orows))
+
+
 @pytest.mark.parametrize("alg,split", [("hip_barnes_hut", True), ("hip_barnes_hut", False),
                                        ("hip_barnes_hut_fp64", True)])
 @pytest.mark.parametrize("n", [65, 3000, 40000])
