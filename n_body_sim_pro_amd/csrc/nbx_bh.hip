@@ -66,9 +66,18 @@ constexpr int kThreads = 256;
 constexpr int kExtWords = 6;
 constexpr int kMaxLevels = 129;  // a shared depth-129 cell means depth > 128 (barnes_hut.c:149-153)
 // What the host has to handle before the tree is valid: particles that share a
-// whole key (small systems), a tree deeper than the reference's limit, a run of
-// equal top key bits too long for order_kernel, more cells than there is room for.
+// whole key (small systems), a tree deeper than the reference's limit, an order
+// that order_kernel could not finish, more cells than there is room for.
 enum { FLAG_TIE = 0, FLAG_OVERFLOW = 1, FLAG_LONG_RUN = 2, FLAG_CELLS = 3 };
+// FLAG_LONG_RUN: a run too long; tied positions that found no slot for their
+// extension words.
+enum { ORDER_RUN = 1u, ORDER_SLOTS = 2u };
+// Flag words, the number of tied positions, the per-depth cell counts and their
+// total.
+constexpr int kTiedCount = 4;
+constexpr int kDCount = 8;
+constexpr int kFlagWords = 160;
+static_assert(kDCount + kMaxLevels + 1 <= kFlagWords, "depth counts and total");
 
 __device__ inline uint64_t spread3(uint64_t a) {
     uint64_t x = a & 0x1FFFFFull;
@@ -112,18 +121,30 @@ __device__ inline int word_levels(uint64_t x) {
     return (__clzll(static_cast<long long>(x)) - 1) / 3;
 }
 
-__device__ inline int common_levels(const uint64_t* __restrict__ w,
-                                    const uint64_t* __restrict__ ext, int a, int b) {
+// The extension words of tree positions, six each (words null: none are made).
+// With `slot`, position t's are those of slot[t], which only positions that
+// share their key with a neighbour have.
+struct ExtTable {
+    const uint64_t* words;
+    const uint32_t* slot;
+    __device__ const uint64_t* of(int t) const {
+        return words + static_cast<size_t>(slot != nullptr ? slot[t] : t) * kExtWords;
+    }
+};
+
+__device__ inline int common_levels(const uint64_t* __restrict__ w, const ExtTable& ext, int a,
+                                    int b) {
     const uint64_t x = w[a] ^ w[b];
     if (x != 0) {
         return word_levels(x);
     }
-    if (ext == nullptr) {
+    if (ext.words == nullptr) {
         return 21;
     }
+    const uint64_t* ea = ext.of(a);
+    const uint64_t* eb = ext.of(b);
     for (int k = 0; k < kExtWords; ++k) {
-        const uint64_t y = ext[static_cast<size_t>(a) * kExtWords + k] ^
-                           ext[static_cast<size_t>(b) * kExtWords + k];
+        const uint64_t y = ea[k] ^ eb[k];
         if (y != 0) {
             const int l = 21 * (k + 1) + word_levels(y);
             return l < kMaxLevels ? l : kMaxLevels;
@@ -133,11 +154,10 @@ __device__ inline int common_levels(const uint64_t* __restrict__ w,
 }
 
 // Octant digit of tree position t at level `level` (the octant of its depth
-// level+1 cell inside its depth `level` cell).
-__device__ inline int digit_at(const uint64_t* __restrict__ w, const uint64_t* __restrict__ ext,
-                               int t, int level) {
-    const uint64_t word = level < 21 ? w[t]
-                                     : ext[static_cast<size_t>(t) * kExtWords + (level / 21 - 1)];
+// level+1 cell inside its depth `level` cell, which holds a neighbour too).
+__device__ inline int digit_at(const uint64_t* __restrict__ w, const ExtTable& ext, int t,
+                               int level) {
+    const uint64_t word = level < 21 ? w[t] : ext.of(t)[level / 21 - 1];
     return static_cast<int>((word >> (60 - 3 * (level % 21))) & 7u);
 }
 
@@ -398,17 +418,19 @@ static_assert(kSortTopBits % 9 == 0, "whole 9-bit radix passes");
 // Input: sorted (stably, from index order) by key >> low_bits. Element p
 // goes to its run's first position plus the number of run members before it
 // in key order. Members that share the whole key are ordered by their deeper
-// digits, and their extension words go to ext (nobody reads a position's
-// words unless it shares its key with a neighbour). (Two of 25 evaluations of
-// the 10M two-galaxy input hold such a pair; sorting all extension words of
-// all particles took 8 ms each time.) Elements of a run longer than kFinishRun
-// stay where they are (the output is still a permutation) and raise the flag.
+// digits, and each takes one of `slots` slots of ext for its extension words
+// (nobody reads a position's words unless it shares its key with a neighbour).
+// (Two of 25 evaluations of the 10M two-galaxy input hold such a pair; sorting
+// all extension words of all particles took 8 ms each time.) Too few slots, or
+// a run longer than kFinishRun, whose elements stay where they are (the output
+// is still a permutation), raise the flag.
 template <typename In>
 __global__ __launch_bounds__(kThreads) void order_kernel(
     const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin, int n,
     const In* __restrict__ b4, const double* __restrict__ root, uint32_t* __restrict__ tperm,
-    uint64_t* __restrict__ tword, uint64_t* __restrict__ ext, double4* __restrict__ sp4,
-    float4* __restrict__ s4, unsigned* __restrict__ flags, int low_bits) {
+    uint64_t* __restrict__ tword, uint64_t* __restrict__ ext, uint32_t* __restrict__ slot,
+    unsigned slots, double4* __restrict__ sp4, float4* __restrict__ s4,
+    unsigned* __restrict__ flags, int low_bits) {
     const int p = blockIdx.x * kThreads + threadIdx.x;
     if (p >= n) {
         return;
@@ -430,7 +452,7 @@ __global__ __launch_bounds__(kThreads) void order_kernel(
     if (b - a + 1 > kFinishRun) {
         // every member of a run this long sees a window of more than
         // kFinishRun positions, so the whole run stays in place
-        atomicOr(&flags[FLAG_LONG_RUN], 1u);
+        atomicOr(&flags[FLAG_LONG_RUN], ORDER_RUN);
     } else {
         int rank = 0;
         for (int q = a; q <= b; ++q) {
@@ -448,7 +470,13 @@ __global__ __launch_bounds__(kThreads) void order_kernel(
     const int t = n - 1 - dst;
     place(t, key, o, b4, tperm, tword, sp4, s4);
     if (tied) {
-        extension_words(widen(b4[o]), root, ext + static_cast<size_t>(t) * kExtWords);
+        const unsigned k = atomicAdd(&flags[kTiedCount], 1u);
+        if (k < slots) {
+            slot[t] = k;
+            extension_words(widen(b4[o]), root, ext + static_cast<size_t>(k) * kExtWords);
+        } else {
+            atomicOr(&flags[FLAG_LONG_RUN], ORDER_SLOTS);
+        }
     }
 }
 
@@ -761,10 +789,6 @@ constexpr int kEndRow = kMaxLevels;
 constexpr int kCellRow = 2 * kMaxLevels;
 constexpr int kTopoRows = 2 * kMaxLevels + 1;
 
-// Flag words, then the per-depth cell counts and their total.
-constexpr int kDCount = 8;
-constexpr int kFlagWords = 160;
-static_assert(kDCount + kMaxLevels + 1 <= kFlagWords, "depth counts and total");
 
 // Whether an earlier kernel of this build found something the host has to
 // handle first (the tree is not valid then): later kernels of the evaluation
@@ -804,7 +828,7 @@ __device__ inline int wave_max_int(int v) {
 // tile_hist[row * tiles + b] = tile b's counts.
 template <int POSITIONS>
 __global__ __launch_bounds__(kThreads) void delta_kernel(const uint64_t* __restrict__ w,
-                                                        const uint64_t* __restrict__ ext, int n,
+                                                        ExtTable ext, int n,
                                                         int tiles, int32_t* __restrict__ delta,
                                                         unsigned* __restrict__ flags,
                                                         unsigned* __restrict__ tile_hist,
@@ -841,7 +865,7 @@ __global__ __launch_bounds__(kThreads) void delta_kernel(const uint64_t* __restr
         for (int d = dcur + 1; d <= etop; ++d) {
             atomicAdd(&hist[kEndRow + d], 1u);
         }
-        if (ext == nullptr && dcur >= 21) {
+        if (ext.words == nullptr && dcur >= 21) {
             mine |= 1u;
         }
         if (dcur >= kMaxLevels) {
@@ -1219,8 +1243,7 @@ __device__ inline void empty_slots(int32_t* kids, int lo, int hi) {
 // 18 + 20 + 100 us at 1M, and at 10,000 particles 13 + 35 us.
 template <bool QUAD, typename In, typename T>
 __global__ __launch_bounds__(T::kBuildThreads, 4) void build_kernel(
-    const uint64_t* __restrict__ w, const uint64_t* __restrict__ ext,
-    const int32_t* __restrict__ delta, int n, int tiles, int cell_capacity,
+    const uint64_t* __restrict__ w, ExtTable ext, const int32_t* __restrict__ delta, int n, int tiles, int cell_capacity,
     unsigned* __restrict__ flags, const unsigned* __restrict__ tile_base,
     uint32_t* __restrict__ scan, CellData<In> c) {
     constexpr int kTopoTile = T::kPositions, kTopoChunks = T::kChunks;
@@ -1360,8 +1383,7 @@ __global__ __launch_bounds__(T::kBuildThreads, 4) void build_kernel(
         const uint32_t sc = tile_cells + r.chunk_cells[chunk] + static_cast<unsigned>(below[i]);
         const int li = static_cast<int>(sc) + cells + t;   // the leaf's node index
         auto digit = [&](uint64_t key, int pos, int level) {
-            const uint64_t v =
-                level < 21 ? key : ext[static_cast<size_t>(pos) * kExtWords + (level / 21 - 1)];
+            const uint64_t v = level < 21 ? key : ext.of(pos)[level / 21 - 1];
             return static_cast<int>((v >> (60 - 3 * (level % 21))) & 7u);
         };
         if (valid) {
@@ -2067,8 +2089,8 @@ constexpr int kGroupCell = 2048;     // compact: the group's smallest enclosing 
 constexpr int kRunStride = kGroupCell / kWave;
 static_assert(kRunStride == kWave / 2, "the fine round probes one stride per half wave");
 
-__device__ inline bool run_compact(const uint64_t* __restrict__ w, const uint64_t* __restrict__ ext,
-                                   int n, int a, int b, int c, int lane) {
+__device__ inline bool run_compact(const uint64_t* __restrict__ w, const ExtTable& ext, int n,
+                                   int a, int b, int c, int lane) {
     const int r = b + kRunStride * (lane + 1);
     const int l = a - kRunStride * (lane + 1);
     const bool in_r = r < n && common_levels(w, ext, b, r) >= c;
@@ -2186,7 +2208,7 @@ __global__ __launch_bounds__(W * kWave) void group_walk_kernel(
     const unsigned* __restrict__ flags, int* __restrict__ deferred,
     const GroupNode* __restrict__ gnode, const float4* __restrict__ s4,
     const uint32_t* __restrict__ tperm, const uint64_t* __restrict__ tword,
-    const uint64_t* __restrict__ ext, int n, float G, float eps2, float theta2,
+    ExtTable ext, int n, float G, float eps2, float theta2,
     double* __restrict__ ax, double* __restrict__ ay,
     double* __restrict__ az, unsigned long long* __restrict__ counters,
     float* __restrict__ features, const float4* __restrict__ gquad,
@@ -2559,7 +2581,7 @@ __global__ __launch_bounds__(W * kWave) void group_walk_kernel(
     // members of a range that cannot be split within the budget of
     // `max_walks` shared walks per wave are deferred to the per-query walk.
     const int last = t0 + kWave - 1 < n ? t0 + kWave - 1 : n - 1;
-    const int max_level = ext != nullptr ? kMaxLevels : 21;
+    const int max_level = ext.words != nullptr ? kMaxLevels : 21;
     int rsp = 1, walks = 0;
     if (lane == 0) {
         ranges[0] = make_int2(t0, last);
@@ -2578,7 +2600,8 @@ __global__ __launch_bounds__(W * kWave) void group_walk_kernel(
         if (!shared && rsp + 8 <= kRangeStack && walks + rsp + 2 <= max_walks) {
             // octant of each member's depth c + 1 cell; runs of equal octants
             // (a and b differ in that octant, so there are at least two)
-            const int dig = digit_at(tword, ext, valid ? t : a, c);
+            // (lanes outside the range need not have extension words)
+            const int dig = digit_at(tword, ext, t >= a && t <= b ? t : a, c);
             const int prev = __shfl_up(dig, 1);
             cut = __ballot(t > a && t <= b && dig != prev);
         }
@@ -2691,6 +2714,10 @@ InternalSoA internal_soa(BHState& s) {
     return in;
 }
 
+ExtTable ext_table(const BHState& s) {
+    return {s.ext_tree, s.ext_slot};
+}
+
 double* root_of(BHState& s) {
     return B<double>(s.partial) + 6 * kBBoxBlocks;
 }
@@ -2710,10 +2737,13 @@ void enqueue_runs(Engine* e, int low_bits) {
     BHState& s = e->bh;
     order_kernel<In><<<grid_for(s.n, kThreads), kThreads, 0, e->stream>>>(
         B<uint64_t>(s.sk0), B<uint32_t>(s.sv0), static_cast<int>(s.n), B<In>(s.b4), root_of(s),
-        B<uint32_t>(s.tperm), B<uint64_t>(s.tword), B<uint64_t>(s.ext),
+        B<uint32_t>(s.tperm), B<uint64_t>(s.tword), B<uint64_t>(s.ext), B<uint32_t>(s.tmp32),
+        static_cast<unsigned>(s.ext_slots),
         std::is_same_v<In, double4> ? B<double4>(s.sp4) : nullptr, B<float4>(s.s4),
         B<unsigned>(s.flags), low_bits);
     s.sorted_low_bits = low_bits;
+    s.ext_tree = B<uint64_t>(s.ext);
+    s.ext_slot = B<uint32_t>(s.tmp32);
 }
 
 // The bounding cube, the keys and the tree order of e's particles.
@@ -2740,12 +2770,14 @@ NBodySimProStatus enqueue_order(Engine* e, NBodySimProError* error) {
             B<uint64_t>(s.sk0), B<uint32_t>(s.sv0), ni, b4, B<uint32_t>(s.tperm),
             B<uint64_t>(s.tword), sp4, B<float4>(s.s4));
         s.ext_tree = nullptr;   // a shared key raises FLAG_TIE
+        s.ext_slot = nullptr;
         s.sorted_low_bits = 0;
     } else {
         keys_kernel<In><<<g < 1024u ? g : 1024u, kThreads, 0, st>>>(
             b4, ni, B<double>(s.partial), static_cast<int>(bb_blocks), root, B<uint64_t>(s.sk0));
         NBX_HIP(error, hipGetLastError());
-        NBX_TRY(s.ext.need<uint64_t>(s.n * kExtWords, error));
+        NBX_TRY(s.ext.need<uint64_t>(s.ext_slots * kExtWords, error));
+        NBX_TRY(s.tmp32.need<uint32_t>(s.n, error));
         // stable on the top key bits (the result stays in sk0/sv0), then the
         // short runs. (Measured on MI355X, two-galaxy, against seven passes
         // on all 63 bits: sort 1M 0.171 -> 0.108 ms, 10M 0.894 -> 0.641 ms.)
@@ -2754,7 +2786,6 @@ NBodySimProStatus enqueue_order(Engine* e, NBodySimProError* error) {
                                  nullptr, kSortLowBits, true,
                                  cnts + kCounters + PHASE_SORT));
         enqueue_runs<In>(e, kSortLowBits);
-        s.ext_tree = B<uint64_t>(s.ext);
     }
     NBX_HIP(error, hipGetLastError());
     return N_BODY_SIM_PRO_STATUS_OK;
@@ -2811,7 +2842,8 @@ NBodySimProStatus enqueue_full_order(Engine* e, NBodySimProError* error) {
         P, key, ext, ni, b4, B<uint32_t>(s.tperm), B<uint64_t>(s.tword), B<uint64_t>(s.ext),
         std::is_same_v<In, double4> ? B<double4>(s.sp4) : nullptr, B<float4>(s.s4));
     NBX_HIP(error, hipGetLastError());
-    s.ext_tree = B<uint64_t>(s.ext);
+    s.ext_tree = B<uint64_t>(s.ext);   // by position
+    s.ext_slot = nullptr;
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 
@@ -2824,7 +2856,7 @@ NBodySimProStatus enqueue_depths(Engine* e, NBodySimProError* error) {
     unsigned* flags = B<unsigned>(s.flags);
     with_tile(s.tile, [&](auto tile) {
         delta_kernel<decltype(tile)::kPositions><<<nt, kThreads, 0, st>>>(
-            B<uint64_t>(s.tword), s.ext_tree, ni, nt, B<int32_t>(s.delta), flags,
+            B<uint64_t>(s.tword), ext_table(s), ni, nt, B<int32_t>(s.delta), flags,
             B<unsigned>(s.tile_hist), B<unsigned long long>(s.counters));
     });
     depth_scan_kernel<<<kTopoRows, kThreads, 0, st>>>(B<unsigned>(s.tile_hist), nt,
@@ -2871,7 +2903,7 @@ NBodySimProStatus enqueue_cells(Engine* e, NBodySimProError* error) {
         using T = decltype(tile);
         constexpr int kPositions = T::kPositions;
         build_kernel<QUAD, In, T><<<nt, T::kBuildThreads, 0, st>>>(
-            B<uint64_t>(s.tword), s.ext_tree, B<int32_t>(s.delta), ni, nt,
+            B<uint64_t>(s.tword), ext_table(s), B<int32_t>(s.delta), ni, nt,
             static_cast<int>(s.cells), flags, base, B<uint32_t>(s.scan), c);
         if (nt > 1) {
             span_com_kernel<QUAD, In, 512, kPositions><<<grid_for(nt, kSpanTiles), 512, 0, st>>>(
@@ -2953,7 +2985,16 @@ NBodySimProStatus read_build(Engine* e, int slot, bool* again, NBodySimProError*
     *again = false;
     if (report->flags[FLAG_LONG_RUN] != 0 || report->flags[FLAG_TIE] != 0) {
         NBX_HIP(error, hipMemsetAsync(flags, 0, kFlagWords * sizeof(unsigned), st));
-        if (s.sorted_low_bits > 0) {
+        if (report->flags[FLAG_LONG_RUN] == ORDER_SLOTS) {
+            const size_t tied = report->flags[kTiedCount];
+            s.ext_slots = tied + tied / 8;
+            NBX_TRY(s.ext.need<uint64_t>(s.ext_slots * kExtWords, error));
+            if (s.inputs_fp64) {
+                enqueue_runs<double4>(e, s.sorted_low_bits);
+            } else {
+                enqueue_runs<float4>(e, s.sorted_low_bits);
+            }
+        } else if (s.sorted_low_bits > 0) {
             NBX_TRY(s.inputs_fp64 ? enqueue_key_order<double4>(e, error)
                                   : enqueue_key_order<float4>(e, error));
         } else {
@@ -3062,10 +3103,12 @@ NBodySimProStatus enqueue_build(Engine* e, bool fp32_inputs, bool quadrupoles,
     const size_t tiles = grid_for(n, s.tile);
     NBX_TRY(s.tile_hist.need<unsigned>(kTopoRows * tiles, error));
     NBX_TRY(s.tile_base.need<unsigned>(kTopoRows * tiles, error));
-    // Room for the cells of usual inputs (about n / 2); a tree with more
-    // raises FLAG_CELLS and is built again with room for its count.
+    // Room for the cells of usual inputs (about n / 2) and for a few tied
+    // positions; a tree with more raises FLAG_CELLS or FLAG_LONG_RUN, and that
+    // part is repeated with room for its count.
     if (s.cells_n != n) {
         s.cells = n / 4 * 3 + 1024;
+        s.ext_slots = n / 64 + 1024;
         s.cells_n = n;
     }
     s.n = n;
@@ -3183,13 +3226,13 @@ NBodySimProStatus enqueue_walk(Engine* e, const NBodySimProGravity* g, bool fp64
         if (features != nullptr) {
             group_walk_kernel<true, 1><<<grid_g, kWave, 0, st>>>(
                 flags, deferred, gn, B<float4>(s.s4), B<uint32_t>(s.tperm),
-                B<uint64_t>(s.tword), s.ext_tree, ni, Gf, e2, th2, e->ax, e->ay, e->az, cnts,
+                B<uint64_t>(s.tword), ext_table(s), ni, Gf, e2, th2, e->ax, e->ay, e->az, cnts,
                 features, gq, max_walks, member_test, chunk_log);
         } else {
             auto go = [&](auto kernel) {
                 kernel<<<grid_g, team * kWave, 0, st>>>(
                     flags, deferred, gn, B<float4>(s.s4), B<uint32_t>(s.tperm),
-                    B<uint64_t>(s.tword), s.ext_tree, ni, Gf, e2, th2, e->ax, e->ay, e->az, cnts,
+                    B<uint64_t>(s.tword), ext_table(s), ni, Gf, e2, th2, e->ax, e->ay, e->az, cnts,
                     nullptr, nullptr, max_walks, member_test, chunk_log);
             };
             if (team == 4) {
@@ -3285,7 +3328,8 @@ NBodySimProStatus bh_finish(Engine* e, const NBodySimProGravity* g, bool fp64_ex
     float per_query_ms = 0.f;
     s.slot = slot;
     // Each repetition follows a repaired build: an order on all the key bits,
-    // then on the extension words too, then room for its cells, at most.
+    // then room for the extension words or an order on all of those, then room
+    // for its cells, at most.
     bool again = true;
     for (int attempt = 0; again && attempt < 4; ++attempt) {
         if (attempt > 0) {

@@ -1124,9 +1124,14 @@ NBodySimProStatus nbx_engine_bh_export_nodes(NBXEngine* engine, double* rows,
         cz[k] = sp[4 * t + 2];
         m[k] = sp[4 * t + 3];
     }
+    std::vector<uint32_t> slot;
     if (s.ext_tree != nullptr) {
-        ext.resize(n * 6);
-        NBX_HIP(error, hipMemcpy(ext.data(), s.ext_tree, n * 6 * 8, hipMemcpyDeviceToHost));
+        ext.resize((s.ext_slot != nullptr ? s.ext_slots : n) * 6);
+        NBX_HIP(error, hipMemcpy(ext.data(), s.ext_tree, ext.size() * 8, hipMemcpyDeviceToHost));
+    }
+    if (s.ext_slot != nullptr) {
+        slot.resize(n);
+        NBX_HIP(error, hipMemcpy(slot.data(), s.ext_slot, n * 4, hipMemcpyDeviceToHost));
     }
     for (size_t k = 0; k < nodes; ++k) {
         // Replay the cell centre from the root along the node's octant path
@@ -1135,7 +1140,8 @@ NBodySimProStatus nbx_engine_bh_export_nodes(NBXEngine* engine, double* rows,
         double h = s.root[3];
         const int t = start[k];
         for (int d = 0; d < depth[k]; ++d) {
-            uint64_t w = d < 21 ? word[t] : ext[static_cast<size_t>(t) * 6 + (d / 21 - 1)];
+            const size_t at = d < 21 || slot.empty() ? static_cast<size_t>(t) : slot[t];
+            uint64_t w = d < 21 ? word[t] : ext[at * 6 + (d / 21 - 1)];
             const int o = static_cast<int>((w >> (60 - 3 * (d % 21))) & 7u);
             const double off = h * 0.5;
             c[0] = c[0] + ((o & 1) ? off : -off);

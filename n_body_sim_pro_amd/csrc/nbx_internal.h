@@ -111,7 +111,9 @@ struct BHState {
     bool has_n32 = false;     // the FP32 pre-order records of the last build are written
     bool has_morton = false;  // mkey and mperm hold the last build's Morton order
     bool inputs_fp64 = false; // the last build ran on FP64 inputs (b4 and sp4 are double4)
-    const uint64_t* ext_tree = nullptr;   // tree-order extension words or null (ext below)
+    const uint64_t* ext_tree = nullptr;   // extension words or null (ext below)
+    const uint32_t* ext_slot = nullptr;   // tree position -> its slot there (tmp32), null: itself
+    size_t ext_slots = 0;     // slots that are made (sized with the cells)
     double root[4] = {0, 0, 0, 1};
     // pinned host block the evaluation's flags, counts, root cube and
     // interaction counters are reported into (BuildReport), kReportBytes
@@ -134,8 +136,9 @@ struct BHState {
     Buf mperm;                // Morton order: sorted position -> original index, on demand
     Buf tperm;                // tree position -> original index
     Buf tword;                // tree-order true keys (descending)
-    Buf ext;                  // extension key words (6 per tree position; only those of
-                              // positions that share their key with a neighbour are read)
+    Buf ext;                  // extension key words, 6 per slot: a slot for each tree position
+                              // that shares its key with a neighbour, or (order on all the
+                              // words) for every position
     Buf ext_orig;             // the same in original order (order on all the words)
     Buf delta;                // int32 common levels between tree positions t, t+1
     Buf scan;                 // internal cells started before each tree position
@@ -155,7 +158,8 @@ struct BHState {
     // per-query walks reach them through the level index in their node
     // records), learned path only
     Buf im2, gquad;
-    Buf tmp32;                // scratch permutation
+    Buf tmp32;                // slots of the extension words (systems above kSmallSort), or
+                              // the permutation while an order on all the words is made
     Buf counters;             // unsigned long long [approx, exact, deferred queries]
     Buf deferred;             // tree positions the group walk leaves to the per-query walk
 };

@@ -409,6 +409,48 @@ def device_bytes(e):
     return e.lib.nbx_engine_device_bytes(e.h)
 
 
+@pytest.mark.parametrize("path,most", [("hip_barnes_hut", 298)])
+def test_bh_device_memory(nbx, path, most):
+    """Bytes a particle of an engine for 1,000,000 after an evaluation: what it
+    took when the cell arrays were sized by the tree's own count and extension
+    words made only where particles share a key."""
+    n = 1_000_000
+    d = nbx.two_galaxy(n, seed=1)
+    with nbx.Engine(n) as e:
+        e.upload(d["pos"], d["m"])
+        e.bh_features() if path == "features" else e.compute_force(path)
+        assert device_bytes(e) <= most * n
+
+
+@pytest.mark.parametrize("n,tied", [(40000, 1649), (40000, 1650), (40001, 40000)])
+def test_bh_slots_of_extension_words(nbx, oracle, n, tied):
+    """As many tied positions as there are slots at first (n / 64 + 1024), one more,
+    and nearly all: the exact build and walk, then in the same engine those of a
+    system without ties and of this one again."""
+    rng = np.random.default_rng(tied)
+    pos = rng.uniform(-1, 1, size=(n, 3))
+    even = tied - tied % 2
+    pos[1:even:2] = pos[0:even:2] + rng.uniform(0.1, 1, size=(even // 2, 3)) * 1e-12
+    if tied % 2:
+        pos[even] = pos[0] - 3e-13
+    m = rng.uniform(0.5, 1.0, n)
+    order = rng.permutation(n)
+    p = Particles(n, {"px": pos[order, 0], "py": pos[order, 1], "pz": pos[order, 2], "m": m})
+    other = Particles(n, dict(zip(("px", "py", "pz"), rng.uniform(-1, 1, (3, n))), m=m))
+    with nbx.Engine(n, theta=0.7) as e:
+        for q in (p, other, p):
+            st, oacc, os_, okeys, operm, oroot, orows = oracle_bh(oracle, q, 0.7, 0.01)
+            assert st == 0
+            shared = np.unique(okeys, return_counts=True)[1]
+            assert shared[shared > 1].sum() == (tied if q is p else 0)
+            e.upload_view(q.view)
+            e.compute_force("hip_barnes_hut_fp64", eps=0.01)
+            assert np.array_equal(e.accelerations(), oacc)
+            assert stats_tuple(e.stats()) == stats_tuple(os_)
+            rows = e.bh_export_nodes()
+            assert np.array_equal(sort_rows(rows), sort_rows(orows))
+
+
 @pytest.mark.parametrize("case", ["escaper", "core", "one_key"])
 def test_bh_long_runs(nbx, oracle, case):
     """Runs of equal top key bits too long for the order kernel. An escaper far
