@@ -3053,6 +3053,8 @@ NBodySimProStatus enqueue_build(Engine* e, bool fp32_inputs, bool quadrupoles,
 
 }  // namespace
 
+constexpr size_t kRoomyCells = size_t{1} << 20;   // particles
+
 // Enqueues the whole build. No host read: the kernels of the build and of the
 // walk that follows check the flag words, and bh_walk reads them once at its
 // end (the read between the per-depth counts and the cell records left the
@@ -3103,11 +3105,15 @@ NBodySimProStatus enqueue_build(Engine* e, bool fp32_inputs, bool quadrupoles,
     const size_t tiles = grid_for(n, s.tile);
     NBX_TRY(s.tile_hist.need<unsigned>(kTopoRows * tiles, error));
     NBX_TRY(s.tile_base.need<unsigned>(kTopoRows * tiles, error));
-    // Room for the cells of usual inputs (about n / 2) and for a few tied
-    // positions; a tree with more raises FLAG_CELLS or FLAG_LONG_RUN, and that
-    // part is repeated with room for its count.
+    // Room for the cells of usual inputs and for a few tied positions; a tree
+    // with more raises FLAG_CELLS or FLAG_LONG_RUN, and that part is repeated
+    // with room for its count. Points of any smooth density make 0.469 n to
+    // 0.492 n cells (the sum over levels of 8^d (1 - exp(-u) (1 + u)), u =
+    // n / 8^d), two galaxies of 100,000 to 10M 0.503 n to 0.483 n, and points of
+    // a plane about n / ln 4 = 0.72 n: there is room for those while it costs
+    // little memory, and beyond for a quarter more than the smooth ones.
     if (s.cells_n != n) {
-        s.cells = n / 4 * 3 + 1024;
+        s.cells = (n <= kRoomyCells ? n / 4 * 3 : n / 8 * 5) + 1024;
         s.ext_slots = n / 64 + 1024;
         s.cells_n = n;
     }

@@ -409,12 +409,13 @@ def device_bytes(e):
     return e.lib.nbx_engine_device_bytes(e.h)
 
 
-@pytest.mark.parametrize("path,most", [("hip_barnes_hut", 298)])
+@pytest.mark.parametrize("path,most", [("hip_barnes_hut", 298), ("hip_barnes_hut_fp64", 433),
+                                       ("features", 527)])
 def test_bh_device_memory(nbx, path, most):
-    """Bytes a particle of an engine for 1,000,000 after an evaluation: what it
+    """Bytes a particle of an engine for 2,000,000 after an evaluation: what it
     took when the cell arrays were sized by the tree's own count and extension
     words made only where particles share a key."""
-    n = 1_000_000
+    n = 2_000_000
     d = nbx.two_galaxy(n, seed=1)
     with nbx.Engine(n) as e:
         e.upload(d["pos"], d["m"])
