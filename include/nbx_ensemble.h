@@ -70,9 +70,10 @@ NBodySimProStatus nbx_ensemble_set_tile(NBXEnsemble* ensemble, const NBXTileConf
                                         NBodySimProError* error);
 /*
  * Autotuner: for every size bucket present, times the force launch with 1, 2
- * and 4 targets per lane on that bucket's clusters alone and keeps the
- * fastest; then times 1..8 blocks per CU and 64..512-source tiles on the whole
- * ensemble. Results are cached per (device architecture, bucket histogram) in
+ * and 4 targets per lane on that bucket's clusters alone; then times that
+ * mixture and one width for all buckets with 1..8 blocks per CU on the whole
+ * ensemble, in the step's order of launches, and 64..512-source tiles with the
+ * fastest. The shape in use stays if none is faster. Results are cached per (device architecture, bucket histogram) in
  * the file named by `cache_path` (NULL: no file). `report` (nullable) gets a
  * one-line JSON summary.
  */

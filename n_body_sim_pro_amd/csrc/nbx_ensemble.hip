@@ -51,6 +51,7 @@ struct Ensemble {
     float4* pos4 = nullptr;
     Buf items;       // LPT-ordered, dealt to queues
     int nitems = 0;
+    int widest = 1;  // most targets per lane of an item
     Buf eitems;      // cluster-ordered items of 64 targets (energies)
     std::vector<int> eitem_first;  // first energy item of each cluster (+ sentinel)
     Buf epart;       // energy partials per energy item
@@ -423,6 +424,10 @@ NBodySimProStatus upload_items(Ensemble& s, const std::vector<WorkItem>& v,
                                  hipMemcpyHostToDevice));
     }
     s.nitems = static_cast<int>(v.size());
+    s.widest = 1;
+    for (const WorkItem& w : v) {
+        s.widest = std::max(s.widest, w.r);
+    }
     return N_BODY_SIM_PRO_STATUS_OK;
 }
 
@@ -433,13 +438,14 @@ void launch_force(Ensemble& s, float G, float eps2) {
         kernel<<<grid, kThreads, 0, s.stream>>>(s.pos4, s.ax, s.ay, s.az, s.items.as<WorkItem>(),
                                                 s.nitems, s.queue, G, eps2, s.tile.source_tile);
     };
-    const int widest = *std::max_element(s.tile.targets_per_lane, s.tile.targets_per_lane + kBuckets);
     if (eps2 > 0.f) {
-        widest == 1 ? go(ens_force_kernel<false, 1>)
-                    : (widest == 2 ? go(ens_force_kernel<false, 2>) : go(ens_force_kernel<false, 4>));
+        s.widest == 1   ? go(ens_force_kernel<false, 1>)
+        : s.widest == 2 ? go(ens_force_kernel<false, 2>)
+                        : go(ens_force_kernel<false, 4>);
     } else {
-        widest == 1 ? go(ens_force_kernel<true, 1>)
-                    : (widest == 2 ? go(ens_force_kernel<true, 2>) : go(ens_force_kernel<true, 4>));
+        s.widest == 1   ? go(ens_force_kernel<true, 1>)
+        : s.widest == 2 ? go(ens_force_kernel<true, 2>)
+                        : go(ens_force_kernel<true, 4>);
     }
 }
 
@@ -449,6 +455,26 @@ void drop_graph(Ensemble& s) {
     s.graph_exec = nullptr;
     s.graph = nullptr;
     s.graph_steps = 0;
+}
+
+// Ends the capture whatever the launches returned, so the stream never stays in
+// capture mode; a failed capture leaves no graph behind.
+NBodySimProStatus end_capture(Ensemble& s, NBodySimProError* error) {
+    const hipError_t launched = hipGetLastError();
+    hipGraph_t graph = nullptr;
+    const hipError_t ended = hipStreamEndCapture(s.stream, &graph);
+    s.graph = graph;
+    if (launched != hipSuccess || ended != hipSuccess) {
+        drop_graph(s);
+        NBX_HIP(error, launched != hipSuccess ? launched : ended);
+    }
+    const hipError_t inst = hipGraphInstantiate(&s.graph_exec, s.graph, nullptr, nullptr, 0);
+    if (inst != hipSuccess) {
+        s.graph_exec = nullptr;
+        drop_graph(s);
+        NBX_HIP(error, inst);
+    }
+    return N_BODY_SIM_PRO_STATUS_OK;
 }
 
 void enqueue_steps(Ensemble& s, float G, float eps2, double dt, int steps) {
@@ -465,6 +491,7 @@ void enqueue_steps(Ensemble& s, float G, float eps2, double dt, int steps) {
     }
 }
 
+// Median time of the force launch alone.
 float time_force(Ensemble& s, float G, float eps2, int reps) {
     std::vector<float> t;
     for (int k = 0; k < reps; ++k) {
@@ -478,6 +505,39 @@ float time_force(Ensemble& s, float G, float eps2, int reps) {
     }
     std::sort(t.begin(), t.end());
     return t[t.size() / 2];
+}
+
+// Time of the force launch as the steps run it: in replays of a graph, behind a
+// launch over all particles (here the FP32 positions, written again), and with
+// that launch. How a grid spreads over the chip depends on what ran before it:
+// 64 clusters of 64 to 4,096, one target per lane, take 0.124 / 0.142 ms a step
+// with 8 / 2 blocks per CU, where the launch alone is faster with 2 (0.103).
+// (Tuned by the launch alone, ms a step of 64 / 512 / 4,096 / 200 small clusters:
+// 0.145 / 0.43 / 2.48 to 2.52 / 0.043; so: 0.122 / 0.43 / 2.45 / 0.039; untuned
+// 0.124 / 0.44 / 2.45 / 0.057.)
+NBodySimProStatus time_in_graph(Ensemble& s, float G, float eps2, float* ms,
+                                NBodySimProError* error) {
+    constexpr int kForces = 4, kReplays = 5;
+    drop_graph(s);
+    NBX_HIP(error, hipStreamBeginCapture(s.stream, hipStreamCaptureModeThreadLocal));
+    for (int k = 0; k < kForces; ++k) {
+        ens_pos4_kernel<<<grid_for(s.total, kThreads), kThreads, 0, s.stream>>>(
+            s.px, s.py, s.pz, s.m, s.pos4, static_cast<int>(s.total));
+        launch_force(s, G, eps2);
+    }
+    NBX_TRY(end_capture(s, error));
+    std::vector<float> t(kReplays);
+    for (float& one : t) {
+        NBX_HIP(error, hipEventRecord(s.ev0, s.stream));
+        NBX_HIP(error, hipGraphLaunch(s.graph_exec, s.stream));
+        NBX_HIP(error, hipEventRecord(s.ev1, s.stream));
+        NBX_HIP(error, hipEventSynchronize(s.ev1));
+        NBX_HIP(error, hipEventElapsedTime(&one, s.ev0, s.ev1));
+    }
+    drop_graph(s);
+    std::sort(t.begin(), t.end());
+    *ms = t[kReplays / 2] / kForces;
+    return N_BODY_SIM_PRO_STATUS_OK;
 }
 
 }  // namespace
@@ -698,22 +758,7 @@ NBodySimProStatus nbx_ensemble_advance(NBXEnsemble* e, const NBodySimProGravity*
         nbx::drop_graph(s);
         NBX_HIP(error, hipStreamBeginCapture(s.stream, hipStreamCaptureModeThreadLocal));
         nbx::enqueue_steps(s, G, eps2, dt, graph_steps);
-        // End the capture whatever the launches returned, so the stream never
-        // stays in capture mode; a failed capture leaves no graph behind.
-        const hipError_t launched = hipGetLastError();
-        hipGraph_t graph = nullptr;
-        const hipError_t ended = hipStreamEndCapture(s.stream, &graph);
-        s.graph = graph;
-        if (launched != hipSuccess || ended != hipSuccess) {
-            nbx::drop_graph(s);
-            NBX_HIP(error, launched != hipSuccess ? launched : ended);
-        }
-        const hipError_t inst = hipGraphInstantiate(&s.graph_exec, s.graph, nullptr, nullptr, 0);
-        if (inst != hipSuccess) {
-            s.graph_exec = nullptr;
-            nbx::drop_graph(s);
-            NBX_HIP(error, inst);
-        }
+        NBX_TRY(nbx::end_capture(s, error));
         s.graph_steps = graph_steps;
         s.graph_dt = dt;
         s.graph_g = g->gravitational_constant;
@@ -819,14 +864,15 @@ NBodySimProStatus nbx_ensemble_autotune(NBXEnsemble* e, const NBodySimProGravity
     double best_ms = 0.0;
     if (!cached) {
         // 1) targets per lane, bucket by bucket, on that bucket's clusters alone
+        NBXTileConfig mixed = best;
         for (int b = 0; b < nbx::kBuckets; ++b) {
             if (hist[b] == 0) continue;
             std::vector<char> use(s.clusters, 0);
             for (size_t c = 0; c < s.clusters; ++c) use[c] = nbx::bucket_of(s.sizes[c]) == b;
             float bt = 1e30f;
-            int br = best.targets_per_lane[b];
+            int br = mixed.targets_per_lane[b];
             for (int r : {1, 2, 4}) {
-                NBXTileConfig t = best;
+                NBXTileConfig t = mixed;
                 t.targets_per_lane[b] = r;
                 s.tile = t;
                 NBX_TRY(nbx::upload_items(s, nbx::build_items(s, t, use), error));
@@ -837,27 +883,42 @@ NBodySimProStatus nbx_ensemble_autotune(NBXEnsemble* e, const NBodySimProGravity
                     br = r;
                 }
             }
-            best.targets_per_lane[b] = br;
+            mixed.targets_per_lane[b] = br;
         }
-        // 2) persistent-grid width and compensation tile on the whole ensemble
+        // 2) on the whole ensemble, in the step's order of launches: the shape
+        // as it was, that mixture (its widest bucket gives every item its
+        // registers) and one width for all, each with 1 to 8 blocks per CU; then
+        // the compensation tile. A shape takes the place of one before it if it
+        // is faster by more than two runs of one shape differ.
         float bt = 1e30f;
-        NBXTileConfig keep = best;
-        for (int bpc : {1, 2, 4, 8}) {
-            for (int st : {64, 128, 256, 512}) {
-                NBXTileConfig t = keep;
+        auto try_tile = [&](const NBXTileConfig& t) -> NBodySimProStatus {
+            s.tile = t;
+            NBX_TRY(nbx::upload_items(s, nbx::build_items(s, t, {}), error));
+            float ms = 0.f;
+            NBX_TRY(nbx::time_in_graph(s, G, eps2, &ms, error));
+            if (ms < 0.99f * bt) {
+                bt = ms;
+                best = t;
+            }
+            return N_BODY_SIM_PRO_STATUS_OK;
+        };
+        NBX_TRY(try_tile(best));
+        for (int width : {0, 1, 2, 4}) {
+            NBXTileConfig t = mixed;
+            for (int b = 0; b < nbx::kBuckets && width > 0; ++b) t.targets_per_lane[b] = width;
+            for (int bpc : {8, 4, 2, 1}) {
                 t.blocks_per_cu = bpc;
-                t.source_tile = st;
-                s.tile = t;
-                NBX_TRY(nbx::upload_items(s, nbx::build_items(s, t, {}), error));
-                nbx::time_force(s, G, eps2, 1);
-                const float ms = nbx::time_force(s, G, eps2, 3);
-                if (ms < bt) {
-                    bt = ms;
-                    best = t;
-                }
+                NBX_TRY(try_tile(t));
             }
         }
-        best_ms = bt;
+        NBXTileConfig t = best;
+        for (int st : {64, 128, 256, 512}) {
+            t.source_tile = st;
+            NBX_TRY(try_tile(t));
+        }
+        s.tile = best;
+        NBX_TRY(nbx::upload_items(s, nbx::build_items(s, best, {}), error));
+        best_ms = nbx::time_force(s, G, eps2, 3);
         if (cache_path != nullptr) {
             if (FILE* f = std::fopen(cache_path, "a")) {
                 std::fprintf(f, "%s %d %d %d %d %d %d %d %d %d %d\n", key.c_str(),

@@ -140,6 +140,25 @@ def test_autotune_returns_valid_cached_config(nbx, small_ensemble, tmp_path):
     assert np.median(err) < 1e-6
 
 
+def test_autotune_does_not_leave_a_slower_shape(nbx):
+    """64 clusters leave the chip room that depends on the launch before: steps
+    with the tuned shape take no longer than with the one before tuning (a
+    shape has to be 1% faster to be taken; runs of one shape differ by 2%)."""
+    sizes = nbx.ensemble_sizes(64, lo=64, hi=4096, seed=42)
+    d = nbx.ensemble_clusters(sizes, seed=7)
+    with nbx.Ensemble(sizes) as ens:
+        ens.upload(d["pos"], d["vel"], d["m"])
+        ens.force(eps=0.01)
+
+        def ms():
+            return min(ens.advance(1e-9, 10, graph_steps=10, eps=0.01) for _ in range(5))
+        before = ms()
+        rep = ens.autotune(eps=0.01)
+        tuned = ms()
+    print(f"steps before {before:.4f} ms, tuned {tuned:.4f} ms, {rep}")
+    assert tuned <= 1.06 * before
+
+
 @pytest.mark.parametrize("eps", [0.01, 0.0])
 @pytest.mark.parametrize("targets_per_lane", [1, 2, 4])
 def test_cluster_sizes_around_the_source_split(nbx, oracle, targets_per_lane, eps):
