@@ -73,9 +73,10 @@ NBodySimProStatus nbx_ensemble_set_tile(NBXEnsemble* ensemble, const NBXTileConf
  * and 4 targets per lane on that bucket's clusters alone; then times that
  * mixture and one width for all buckets with 1..8 blocks per CU on the whole
  * ensemble, in the step's order of launches, and 64..512-source tiles with the
- * fastest. The shape in use stays if none is faster. Results are cached per (device architecture, bucket histogram) in
- * the file named by `cache_path` (NULL: no file). `report` (nullable) gets a
- * one-line JSON summary.
+ * fastest. The shape in use stays if none is faster. Results are cached per
+ * (device architecture, way of dividing the work, bucket histogram) in the file
+ * named by `cache_path` (NULL: no file). `report` (nullable) gets a one-line
+ * JSON summary.
  */
 NBodySimProStatus nbx_ensemble_autotune(NBXEnsemble* ensemble, const NBodySimProGravity* gravity,
                                         const char* cache_path, char* report, size_t report_size,

@@ -395,6 +395,11 @@ bool tile_ok(const NBXTileConfig* t) {
            t->source_tile % 4 == 0;
 }
 
+// In the keys of stored shapes: a shape tuned for another way of dividing the work
+// (items of one wave, with four blocks per CU) must not match. To be changed
+// with it.
+constexpr const char* kShapeTag = ":workgroup-items";
+
 // LPT-ordered items for the clusters selected by `use` (all when empty),
 // dealt round-robin to the per-XCD queues (item k goes to queue k % 8).
 std::vector<WorkItem> build_items(const Ensemble& s, const NBXTileConfig& t,
@@ -834,10 +839,10 @@ NBodySimProStatus nbx_ensemble_autotune(NBXEnsemble* e, const NBodySimProGravity
     NBX_HIP(error, hipSetDevice(s.device));
     const float G = static_cast<float>(g->gravitational_constant);
     const float eps2 = static_cast<float>(g->softening_squared);
-    // cache key: architecture + per-bucket cluster counts
+    // cache key: architecture, what a shape means, per-bucket cluster counts
     std::vector<size_t> hist(nbx::kBuckets, 0);
     for (uint32_t n : s.sizes) hist[nbx::bucket_of(n)]++;
-    std::string key = s.arch;
+    std::string key = s.arch + nbx::kShapeTag;
     for (size_t h : hist) key += ":" + std::to_string(h);
     NBXTileConfig best = s.tile;
     bool cached = false;

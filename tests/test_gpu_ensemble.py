@@ -140,6 +140,25 @@ def test_autotune_returns_valid_cached_config(nbx, small_ensemble, tmp_path):
     assert np.median(err) < 1e-6
 
 
+def test_autotune_ignores_shapes_stored_for_other_work_items(nbx, small_ensemble, tmp_path):
+    """A line whose key is the architecture and the bucket counts alone comes
+    from a library whose work item was one wave."""
+    sizes, d = small_ensemble
+    cache = tmp_path / "tune.txt"
+    name = C.create_string_buffer(256)
+    nbx.load().nbx_device_info(0, name, C.c_size_t(256), None)
+    arch = name.value.decode().rsplit("(", 1)[1].rstrip(")")
+    with nbx.Ensemble(sizes) as ens:
+        ens.upload(d["pos"], d["vel"], d["m"])
+        assert ens.autotune(eps=0.01, cache_path=str(cache))["cached"] is False
+        key = cache.read_text().split()[0]
+        assert key.startswith(arch + ":")
+        counts = key.split(":")[-8:]
+        cache.write_text(":".join([arch, *counts]) + " 4 4 4 4 4 4 4 4 4 256\n")
+        rep = ens.autotune(eps=0.01, cache_path=str(cache))
+    assert rep["cached"] is False
+
+
 def test_autotune_does_not_leave_a_slower_shape(nbx):
     """64 clusters leave the chip room that depends on the launch before: steps
     with the tuned shape take no longer than with the one before tuning (a
