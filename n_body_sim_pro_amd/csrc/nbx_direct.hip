@@ -313,14 +313,15 @@ __global__ __launch_bounds__(256) void direct_fp64_lane_kernel(
 // Launches the FP64 all-pairs kernel over `count` targets (all n particles,
 // or the SUBSET `targets`) that suits the grid. A workgroup of the tile kernel
 // takes 16 targets. Up to one per CU, eight waves form terms; up to three per
-// CU, six; beyond, three, of which four workgroups fit a CU. From 1.75 waves
-// of targets per SIMD on the lane kernel, which has no LDS traffic, fills the
-// chip by itself. Measured on MI355X, ms per evaluation with 8 / 6 / 3 waves
+// CU, six; beyond, three, of which four workgroups fit a CU. From 1.6 waves of
+// targets per SIMD on the lane kernel, which has no LDS traffic, fills the chip
+// by itself: its time is that of the SIMDs with two waves. Measured on MI355X, ms per evaluation with 8 / 6 / 3 waves
 // and the lane kernel (every result bit for bit the same):
 //   N = 1000   0.0137 / 0.0147 / 0.0178 / 0.096    N = 4096  0.0445 / 0.0476 / 0.0623 / 0.375
 //   N = 8192   0.163  / 0.147  / 0.164  / 0.75     N = 12288 0.353  / 0.314  / 0.320  / -
 //   N = 16384  0.604  / 0.522  / 0.492  / 1.54     N = 40000 3.44   / -      / 2.56   / 4.0
-//   N = 98304  3 waves 14.7, lane 15.7;  110000: 18.5, 17.8;  131072: 25.4, 22.9
+//   3 waves / lane: N = 98304 14.9 / 15.7, 104448 17.0 / 17.1, 106496 17.4 / 17.4,
+//   108544 18.5 / 17.8, 110592 18.8 / 17.9, 131072 25.4 / 22.9
 // The kernel this replaced (64 targets per workgroup, IEEE sqrt and divide):
 // 0.049 ms at 1000, 0.186 at 4096, 0.79 at 16384, 4.28 at 40000, 9.05 at 65536
 // (now 6.9). The bound is FP64 issue: about 38 instructions and a v_rsq_f64 a
@@ -341,7 +342,7 @@ void launch_direct_fp64(hipStream_t st, int cu_count, const double* px, const do
         go(direct_fp64_tile_kernel<SUBSET, 8, 4>, blocks, 9 * kWave);
     } else if (blocks <= 3 * cus) {
         go(direct_fp64_tile_kernel<SUBSET, 6, 4>, blocks, 7 * kWave);
-    } else if (blocks < 28 * cus) {
+    } else if (blocks < 26 * cus) {
         go(direct_fp64_tile_kernel<SUBSET, 3, 4>, blocks, 4 * kWave);
     } else {
         launch_clock(st, clock);

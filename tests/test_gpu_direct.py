@@ -200,6 +200,21 @@ def test_direct_fp64_kernel_edges_bit_identical(nbx, oracle, n):
     assert np.array_equal(acc[rows], out)
 
 
+@pytest.mark.parametrize("n", [106480, 106481])
+def test_direct_fp64_where_the_lane_kernel_takes_over(nbx, oracle, n):
+    """The last size of the tile kernel and the first of one target per lane on
+    256 CUs (26 workgroups of 16 targets each): rows against the oracle, bit for
+    bit."""
+    p = from_gen(nbx.plummer(n, seed=8))
+    acc = gpu_force(nbx, p, "hip_direct_fp64", 0.01, G=0.5)
+    rows = np.unique(np.linspace(0, n - 1, 101).astype(np.int64))
+    out = np.zeros((rows.size, 3))
+    oracle.nbo_direct_openmp_subset(C.byref(p.view), C.byref(gravity(0.5, 0.01)),
+                                    rows.ctypes.data_as(C.POINTER(C.c_int64)), rows.size,
+                                    out.ctypes.data_as(C.POINTER(C.c_double)))
+    assert np.array_equal(acc[rows], out)
+
+
 @pytest.mark.parametrize("n", [40, 5000])
 @pytest.mark.parametrize("scale", [1.0, 1e-170, 1e-95, 1e95, 1e170])
 def test_direct_fp64_outside_the_fast_range_bit_identical(nbx, oracle, n, scale):
