@@ -1719,13 +1719,21 @@ __global__ __launch_bounds__(kThreads) void report_kernel(const unsigned* __rest
 // The bound is the wave's own chain: some 100 instructions a node, one after
 // the other, over a union of two to four times one query's list. While there
 // are waves to spare it pays to give each fewer queries, whose union is
-// shorter: the smallest Q of 8, 16, 32 and 64 that keeps the waves below two
-// per SIMD. Measured on MI355X, theta 0.7, us with 64 / 32 / 16 / 8 queries a
+// shorter: 8 and 16 while that keeps the waves below two per SIMD, 32 up to 2.6
+// of them. Measured on MI355X, theta 0.7, us with 64 / 32 / 16 / 8 queries a
 // wave, two-galaxy model, in brackets before (64 queries, IEEE square root
 // and divide, no loads ahead):
 //   3,000    201 / 166 / 148 / 127    (241)    10,000   296 / 252 / 216 / 199  (393)
 //   30,000   387 / 326 / 326 / 332    (496)    100,000  556 / 537 / 681 / 1008 (643)
 //   300,000  984 / 1222 / 1793 / 2961 (1190)
+// Around the line, with 64 / 32, two galaxies of two seeds, Plummer, cloud:
+//   70,000   729 / 495, 536 / 466, 690 / 678, 483 / 466
+//   82,000   807 / 536, 565 / 525, 720 / 761, 509 / 456
+//   88,000   544 / 544, 571 / 556, 716 / 765, 498 / 499
+//   97,000   548 / 556, 611 / 556, 733 / 795, 502 / 502
+//   115,000  594 / 632, -, 784 / 922, 553 / 581
+// (64 a wave are little more than one wave a SIMD there: those SIMDs that get
+// two long ones set the time.)
 // (Terms noted in lists of 64 and formed four at a time, or held back to form
 // two or four at once, were slower: the instructions that hold them cost more
 // than the overlap gives.)
@@ -3257,12 +3265,12 @@ NBodySimProStatus enqueue_walk(Engine* e, const NBodySimProGravity* g, bool fp64
                 g->gravitational_constant, g->softening_squared, theta2, e->ax, e->ay, e->az,
                 cnts);
         };
-        const size_t waves = static_cast<size_t>(e->cu_count) * 8;
+        const size_t waves = static_cast<size_t>(e->cu_count) * 8;   // two per SIMD
         if (s.n <= 8 * waves) {
             go(walk_f64_kernel<8>, 8);
         } else if (s.n <= 16 * waves) {
             go(walk_f64_kernel<16>, 16);
-        } else if (s.n <= 32 * waves) {
+        } else if (s.n <= 42 * waves) {
             go(walk_f64_kernel<32>, 32);
         } else {
             go(walk_f64_kernel<64>, 64);

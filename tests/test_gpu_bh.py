@@ -546,6 +546,20 @@ def test_exact_walk_at_every_wave_width(nbx, oracle, n, eps):
     assert stats_tuple(s) == stats_tuple(so)
 
 
+@pytest.mark.parametrize("n", [86016, 86017])
+def test_exact_walk_where_64_queries_take_over(nbx, oracle, n):
+    """The last size with 32 queries a wave and the first with 64 on 256 CUs."""
+    rng = np.random.default_rng(n)
+    p = Particles(n, {k: rng.normal(size=n) for k in ("px", "py", "pz")})
+    p["m"][:] = rng.uniform(0.5, 1.5, n) / n
+    st, ref, so = oracle_bh(oracle, p, 1.0, 0.01)[:3]
+    assert st == 0
+    e, acc, s = gpu_bh(nbx, p, 1.0, 0.01, "hip_barnes_hut_fp64")
+    e.close()
+    assert np.array_equal(acc, ref)
+    assert stats_tuple(s) == stats_tuple(so)
+
+
 @pytest.mark.parametrize("n", [256, 257, 16384, 16385, 262144, 262145])
 def test_tree_at_every_tile_size(nbx, oracle, n):
     """256, 512 or 1024 positions a workgroup of the topology kernels by the
