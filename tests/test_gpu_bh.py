@@ -530,6 +530,84 @@ def test_steps_of_one_call_equal_single_steps(nbx, alg, split, n):
             assert stats[k] == results[0][1][k], k
 
 
+def meeting_particles(case, n):
+    """Particles on straight lines (no gravity to speak of, exact in binary) that
+    meet at the third step: partners 1e-5 apart (more cells than there is room
+    for), 300 in one cell of the top key bits, partners that share a whole key,
+    one pair in one point."""
+    rng = np.random.default_rng(n)
+    dt = 2.0 ** -10
+    grid = 2.0 ** -40
+    pos = np.round(rng.uniform(-1, 1, (n, 3)) / grid) * grid
+    vel = np.round(rng.uniform(0.01, 0.1, (n, 3)) * 2 ** 12) / 2 ** 12
+    pairs = {"cells": n // 2, "slots": 1000, "depth": 1}.get(case, 0)
+    gap = {"cells": 1e-5, "slots": 1e-9}.get(case, 0.0)
+    a, b = slice(0, pairs), slice(pairs, 2 * pairs)
+    pos[b] = pos[a] + np.round(rng.uniform(0.5, 1, (pairs, 3)) * gap / grid) * grid
+    vel[b] = vel[a]
+    vel[b, 0] += 128.0
+    pos[b, 0] -= 3 * dt * 128.0
+    if case == "run":
+        c = slice(0, 300)
+        vel[c] = np.round(rng.uniform(-128, 128, (300, 3)))
+        vel[c] += np.where(vel[c] == 0, 1, 0)
+        pos[c] = 0.25 + np.round(rng.uniform(0, 1e-5, (300, 3)) / grid) * grid - 3 * dt * vel[c]
+    return dict(zip(("px", "py", "pz"), pos.T), **dict(zip(("vx", "vy", "vz"), vel.T)),
+                m=rng.uniform(0.5, 1.5, n) / n), dt
+
+
+@pytest.mark.parametrize("case,n,alg", [
+    ("cells", 3000, "hip_barnes_hut"), ("cells", 40000, "hip_barnes_hut_fp64"),
+    ("run", 40000, "hip_barnes_hut"), ("run", 40000, "hip_barnes_hut_fp64"),
+    ("slots", 40000, "hip_barnes_hut_fp64"), ("depth", 3000, "hip_barnes_hut"),
+    ("depth", 3000, "hip_barnes_hut_fp64"), ("depth", 40000, "hip_barnes_hut"),
+    ("depth", 40000, "hip_barnes_hut_fp64")])
+def test_steps_that_need_the_host_while_running_ahead(nbx, case, n, alg):
+    """The third step's tree needs the host, which learns it when the fourth is
+    enqueued: particles, tree and status as after calls of one step, for a tree
+    too deep those before the error."""
+    a, dt = meeting_particles(case, n)
+    p = Particles(n, a)
+    g = 1.0e-20
+    results = []
+    for calls in ([1] * 6, [6], [2, 4]):
+        with nbx.Engine(n, theta=0.6) as e:
+            e.upload_view(p.view)
+            e.compute_force(alg, G=g, eps=0.01)
+            status, tree = 0, None
+            for k, steps in enumerate(calls):
+                try:
+                    e.advance(alg, dt=dt, steps=steps, G=g, eps=0.01)
+                except nbx.NBXError as error:
+                    status = error.status
+                    break
+                if k == 2 and steps == 1:
+                    cells = e.stats()["internal_node_count"]
+                    keys = e.bh_morton()[1]
+                    shared = np.unique(keys, return_counts=True)[1]
+                    top = np.unique(keys >> np.uint64(27), return_counts=True)[1].max()
+                    assert case != "cells" or cells > n / 4 * 3 + 1024
+                    assert case != "run" or top > 64
+                    assert case != "slots" or shared[shared > 1].sum() > n / 64 + 1024
+            out = e.download()
+            if status == 0:
+                tree = (e.stats()["node_count"], e.bh_morton()[1])
+            else:
+                with pytest.raises(nbx.NBXError):
+                    e.bh_morton()
+            # and the engine goes on with other particles
+            e.upload(np.stack([a["px"], a["py"], a["pz"]], 1), a["m"])
+            e.compute_force(alg, eps=0.01)
+            results.append((out, status, tree, e.accelerations()))
+    for out, status, tree, after in results:
+        assert status == results[0][1] == (6 if case == "depth" else 0)   # OVERFLOW
+        for k in ("pos", "vel", "acc"):
+            assert np.array_equal(out[k], results[0][0][k]), k
+        assert np.array_equal(after, results[0][3])
+        if tree is not None:
+            assert tree[0] == results[0][2][0] and np.array_equal(tree[1], results[0][2][1])
+
+
 @pytest.mark.parametrize("n,eps", [(1, 0.0), (7, 0.0), (9, 0.01), (16384, 0.0), (16385, 0.01),
                                    (32769, 0.01), (65537, 0.0)])
 def test_exact_walk_at_every_wave_width(nbx, oracle, n, eps):
