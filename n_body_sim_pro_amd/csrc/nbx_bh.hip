@@ -3312,13 +3312,13 @@ NBodySimProStatus bh_finish(Engine* e, const NBodySimProGravity* g, bool fp64_ex
     BHState& s = e->bh;
     hipStream_t st = e->stream;
     const int ni = static_cast<int>(s.n);
-    const float4* gq = features != nullptr ? B<float4>(s.gquad) : nullptr;
     const float Gf = static_cast<float>(g->gravitational_constant);
     const float e2 = static_cast<float>(g->softening_squared);
     const float th2 = static_cast<float>(e->theta * e->theta);
     unsigned long long* cnts = B<unsigned long long>(s.counters);
     // per-query reference-list walk of nq queries (all tree positions, or the
-    // listed ones) on the FP32 pre-order records
+    // listed ones) on the FP32 pre-order records (a repair moves the cells'
+    // arrays, so their addresses are taken here)
     auto per_query_walk = [&](const int* list, int nq) -> NBodySimProStatus {
         NBX_TRY(bh_node_records(e, error));
         const unsigned wblocks = grid_for(static_cast<size_t>(nq), kThreads * kWalkQueries);
@@ -3328,7 +3328,7 @@ NBodySimProStatus bh_finish(Engine* e, const NBodySimProGravity* g, bool fp64_ex
         if (features != nullptr) {
             walk_f32_kernel<true, kWalkQueries><<<wgrid, kThreads, 0, st>>>(
                 n32, nn, B<float4>(s.s4), B<uint32_t>(s.tperm), list, nq, Gf, e2, th2, e->ax,
-                e->ay, e->az, cnts, features, gq);
+                e->ay, e->az, cnts, features, B<float4>(s.gquad));
         } else {
             walk_f32_kernel<false, kWalkQueries><<<wgrid, kThreads, 0, st>>>(
                 n32, nn, B<float4>(s.s4), B<uint32_t>(s.tperm), list, nq, Gf, e2, th2, e->ax,

@@ -276,6 +276,24 @@ def test_feature_walk_matches_numpy_restatement(nbx):
     assert np.abs(frames[ok, 1].astype(np.float64) - e2[ok]).max() < 1e-3
 
 
+@pytest.mark.parametrize("kw", [{"reference_lists": True}, {"split": False}])
+@pytest.mark.parametrize("n", [3001, 40001])
+def test_features_of_a_tree_that_needs_room(nbx, n, kw):
+    """Close pairs make more cells than an engine has room for at first: the
+    per-query walk then runs on arrays that have moved. Its features are those
+    of the same engine's next evaluation, whose arrays stay."""
+    rng = np.random.default_rng(n)
+    base = rng.uniform(-1, 1, (n // 2 + 1, 3))
+    pos = np.concatenate([base, base + rng.uniform(0.1, 1, base.shape) * 1e-5])[:n]
+    m = rng.uniform(0.5, 1, n) / n
+    with nbx.Engine(n, theta=1.0, **kw) as e:
+        e.upload(pos, m)
+        first = e.bh_features(1.0, 0.01)
+        assert e.stats()["internal_node_count"] > n / 4 * 3 + 1024
+        second = e.bh_features(1.0, 0.01)
+    assert np.isfinite(first).all() and np.array_equal(first, second)
+
+
 def test_group_walk_features_are_consistent(nbx):
     """Default engine: the feature walk is the group walk with the member
     test. Its accelerations are the plain group walk's with that test up to
