@@ -276,6 +276,117 @@ def test_feature_walk_matches_numpy_restatement(nbx):
     assert np.abs(frames[ok, 1].astype(np.float64) - e2[ok]).max() < 1e-3
 
 
+def _quadrupole_features_of(rows, perm, pos32, m32, theta, eps2, queries):
+    """Features 0, 1, 5, 6 and the interaction counts of some particles, as
+    _walk_features_numpy states them, from the exported nodes: (query, node)
+    pairs opened level by level, second moments from prefix sums over the leaves
+    in long double."""
+    nodes = len(rows)
+    depth = rows[:, 0].astype(int)
+    skip = np.empty(nodes, dtype=int)
+    stack = []
+    for k in range(nodes):
+        while stack and depth[stack[-1]] >= depth[k]:
+            skip[stack.pop()] = k
+        stack.append(k)
+    skip[stack] = nodes
+    leaf = rows[:, 10] >= 0
+    particle = np.where(leaf, perm[np.maximum(rows[:, 10], 0).astype(int)], -1)
+    first = np.cumsum(leaf) - leaf                      # leaves before a node
+    x = pos32[particle[leaf]].astype(np.longdouble)
+    w = m32[particle[leaf]].astype(np.longdouble)
+    outer = x[:, :, None] * x[:, None, :]
+
+    def over(v):                                        # sums over each node's leaves
+        p = np.concatenate([np.zeros_like(v[:1]), np.cumsum(v, axis=0)])
+        return p[first + rows[:, 5].astype(int)] - p[first]
+    mass, mx, mxx = over(w), over(w[:, None] * x), over(w[:, None, None] * outer)
+    com = rows[:, 7:10]
+    c = com.astype(np.longdouble)
+    m2 = (mxx - c[:, :, None] * mx[:, None, :] - mx[:, :, None] * c[:, None, :]
+          + mass[:, None, None] * c[:, :, None] * c[:, None, :]).astype(np.float64)
+    quad = 3 * m2 - np.trace(m2, axis1=1, axis2=2)[:, None, None] * np.eye(3)
+    q = pos32[queries].astype(np.float64)
+    nq = len(queries)
+    tot, qf = np.zeros((nq, 3)), np.zeros((nq, 3))
+    cells, leaves, q2_sum = np.zeros(nq), np.zeros(nq), np.zeros(nq)
+    q2_min = np.full(nq, np.inf)
+    i, k = np.arange(nq), np.zeros(nq, dtype=int)
+    while len(i):
+        d = com[k] - q[i]
+        d2 = (d * d).sum(1)
+        r2 = d2 + eps2
+        size2 = 4.0 * rows[k, 4] ** 2
+        take = np.where(leaf[k], particle[k] != queries[i],
+                        (d2 > 0) & (size2 < theta * theta * d2))
+        np.add.at(tot, i[take], (rows[k, 6] / (r2 * np.sqrt(r2)))[take, None] * d[take])
+        np.add.at(leaves, i[take & leaf[k]], 1)
+        cell = take & ~leaf[k]
+        ic, dc, rc = i[cell], d[cell], r2[cell]
+        Qd = np.einsum("pi,pij->pj", dc, quad[k[cell]])
+        np.add.at(qf, ic, (2.5 * (dc * Qd).sum(1) / rc)[:, None] * dc / rc[:, None] ** 2.5
+                  - Qd / rc[:, None] ** 2.5)
+        np.add.at(cells, ic, 1)
+        ratio = d2[cell] / size2[cell]
+        np.add.at(q2_sum, ic, ratio)
+        np.minimum.at(q2_min, ic, ratio)
+        opened = ~leaf[k] & ~take
+        i, end, k = i[opened], skip[k[opened]], k[opened] + 1
+        ni, nk = [], []
+        while len(i):                                   # the opened cells' children
+            ni.append(i)
+            nk.append(k)
+            k = skip[k]
+            more = k < end
+            i, end, k = i[more], end[more], k[more]
+        i = np.concatenate(ni) if ni else np.zeros(0, dtype=int)
+        k = np.concatenate(nk) if nk else np.zeros(0, dtype=int)
+    a = np.linalg.norm(tot, axis=1)
+    q_par = (qf * tot).sum(1) / a
+    q_perp = np.linalg.norm(qf - (q_par / a)[:, None] * tot, axis=1)
+    return (np.sqrt(q2_sum / np.maximum(cells, 1)), np.sqrt(q2_min), q_par / a, q_perp / a,
+            cells, leaves)
+
+
+@pytest.mark.parametrize("case,n", [
+    ("plummer", 3000),      # (tiles of 256 positions, one launch for the cells that span them)
+    ("plummer", 16385),     # tiles of 512
+    ("plummer", 40001),     # and more than 64 of them: a second launch
+    ("pairs", 40001),       # more cells than a tile's table in LDS holds
+    ("plummer", 262145),    # tiles of 1024
+])
+def test_second_moments_at_every_tile_size(nbx, case, n):
+    """The quadrupole force of 300 particles' walks against moments summed over
+    each cell's particles. A cell at distance d is off by 6e-8 / d of its term
+    (positions of order one in FP32), a few 1e-6 of |a| in all; 5e-5 is a
+    fraction of one near cell's term."""
+    rng = np.random.default_rng(n)
+    if case == "plummer":
+        d = nbx.plummer(n, seed=13)
+        pos, m = d["pos"], d["m"]
+    else:
+        base = rng.uniform(-1, 1, (n // 2 + 1, 3))
+        pos = np.concatenate([base, base + rng.uniform(0.1, 1, base.shape) * 1e-5])[:n]
+        m = rng.uniform(0.5, 1, n) / n
+    with nbx.Engine(n, theta=1.0, reference_lists=True) as e:
+        e.upload(pos, m)
+        feats = e.bh_features(1.0, 0.01)
+        rows = e.bh_export_nodes()
+        perm = e.bh_morton()[2]
+    queries = np.sort(rng.choice(n, 300, replace=False))
+    rms, least, par, perp, cells, leaves = _quadrupole_features_of(
+        rows, perm, pos.astype(np.float32), m.astype(np.float32), 1.0, 1e-4, queries)
+    f = feats[queries].astype(np.float64)
+    same = (np.rint(np.exp2(f[:, 3]) - 1) == cells) & (np.rint(np.exp2(f[:, 4]) - 1) == leaves)
+    worst = max(np.abs(f[same, 5] - par[same]).max(), np.abs(f[same, 6] - perp[same]).max())
+    print(f"{case} {n}: same lists {same.mean():.3f}, |q|/|a| median "
+          f"{np.median(np.hypot(par, perp)):.2e}, largest difference {worst:.2e}")
+    assert same.mean() > 0.97
+    assert worst < 5e-5
+    assert np.allclose(f[same, 0], rms[same], rtol=1e-5) and np.allclose(f[same, 1], least[same],
+                                                                        rtol=1e-5)
+
+
 @pytest.mark.parametrize("kw", [{"reference_lists": True}, {"split": False}])
 @pytest.mark.parametrize("n", [3001, 40001])
 def test_features_of_a_tree_that_needs_room(nbx, n, kw):
