@@ -2168,26 +2168,6 @@ inline int walk_team(size_t groups, int cu_count) {
 // One query per lane in the group walk (measured on MI355X: two per lane, a
 // group of 128, is 7% slower at 10M particles and 16% slower at 1M).
 
-// Exclusive prefix max over the wave of non-negative ints, with DPP row
-// shifts and row broadcasts (no LDS round trips); `total` = max over the wave.
-__device__ inline int dpp_max(int v, int shifted) {
-    return v > shifted ? v : shifted;
-}
-
-__device__ inline int wave_prefix_max_exclusive(int v, int lane, int& total) {
-    // inclusive scan within each 16-lane row (out-of-row sources read 0)
-    v = dpp_max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));   // row_shr:1
-    v = dpp_max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));   // row_shr:2
-    v = dpp_max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));   // row_shr:4
-    v = dpp_max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));   // row_shr:8
-    // across rows: lane 15 of each row into the next row, lane 31 into rows 2, 3
-    v = dpp_max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));   // row_bcast:15
-    v = dpp_max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));   // row_bcast:31
-    total = __builtin_amdgcn_readlane(v, kWave - 1);
-    const int e = __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, false);      // wave_shr:1
-    return lane == 0 ? 0 : e;
-}
-
 __device__ inline float wave_min(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -2790,9 +2770,8 @@ NBodySimProStatus enqueue_order(Engine* e, NBodySimProError* error) {
         // short runs. (Measured on MI355X, two-galaxy, against seven passes
         // on all 63 bits: sort 1M 0.171 -> 0.108 ms, 10M 0.894 -> 0.641 ms.)
         NBX_TRY(radix_sort_pairs(st, B<uint64_t>(s.sk0), B<uint32_t>(s.sv0), B<uint64_t>(s.sk1),
-                                 B<uint32_t>(s.sv1), s.n, kSortTopBits, s.hist, error, nullptr,
-                                 nullptr, kSortLowBits, true,
-                                 cnts + kCounters + PHASE_SORT));
+                                 B<uint32_t>(s.sv1), s.n, kSortTopBits, s.hist, error, kSortLowBits,
+                                 true, cnts + kCounters + PHASE_SORT));
         enqueue_runs<In>(e, kSortLowBits);
     }
     NBX_HIP(error, hipGetLastError());

@@ -49,10 +49,6 @@ NBodySimProStatus map_hip_error(hipError_t e);
 
 // Grows a device allocation to at least `bytes` (contents not preserved).
 NBodySimProStatus ensure(void** ptr, size_t* cap, size_t bytes, NBodySimProError* error);
-template <typename T>
-inline NBodySimProStatus ensure_n(T** ptr, size_t* cap, size_t count, NBodySimProError* error) {
-    return ensure(reinterpret_cast<void**>(ptr), cap, count * sizeof(T), error);
-}
 
 struct Buf {
     void* p = nullptr;
@@ -183,10 +179,9 @@ struct Engine {
     Buf scratch;              // diagnostics / misc
     Buf scratch2;
     BHState bh;
-    NodeF32* learned_dummy = nullptr;
     NBodySimProBarnesHutStats stats{};
     NBXTimings timings{};
-    hipEvent_t ev[3]{};
+    hipEvent_t ev[2]{};       // around a per-query walk, the learned correction's kernel
     void* stage = nullptr;    // pinned host memory of the small transfers
     size_t stage_bytes = 0;
     bool stage_in_report = false;   // it is the rest of bh.report's block
@@ -256,15 +251,12 @@ NBodySimProStatus bh_learned(Engine* e, const NBodySimProGravity* g, NBodySimPro
 // Stable LSD radix sort of (64-bit key, 32-bit value) pairs, ascending key;
 // equal keys keep their input order. It sorts by key bits first_bit ..
 // first_bit + bits - 1 (the bits below first_bit are ignored: equal there
-// counts as equal). The result goes to keys_out/vals_out when given (they
-// must not alias the alternate buffers), else back into keys/vals. iota: the
-// values are the input positions (vals is not read).
+// counts as equal). The result is in keys/vals again. iota: the values are the
+// input positions (vals is not read).
 NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals,
                                    uint64_t* keys_alt, uint32_t* vals_alt, size_t n, int bits,
-                                   Buf& hist, NBodySimProError* error,
-                                   uint64_t* keys_out = nullptr, uint32_t* vals_out = nullptr,
-                                   int first_bit = 0, bool iota = false,
-                                   unsigned long long* start_clock = nullptr);
+                                   Buf& hist, NBodySimProError* error, int first_bit = 0,
+                                   bool iota = false, unsigned long long* start_clock = nullptr);
 // Bits of `mask` set in the lanes below this one (v_mbcnt_lo/hi: two VALU
 // instructions, where and-ing a per-lane mask and counting bits takes four).
 __device__ inline unsigned lanes_below(uint64_t mask) {

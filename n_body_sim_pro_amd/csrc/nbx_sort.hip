@@ -234,28 +234,13 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter(
 
 NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals,
                                    uint64_t* keys_alt, uint32_t* vals_alt, size_t n, int bits,
-                                   Buf& hist, NBodySimProError* error, uint64_t* keys_out,
-                                   uint32_t* vals_out, int first_bit, bool iota,
+                                   Buf& hist, NBodySimProError* error, int first_bit, bool iota,
                                    unsigned long long* start_clock) {
-    if (keys_out == nullptr || vals_out == nullptr) {
-        keys_out = keys;
-        vals_out = vals;
-    }
-    if (n == 0) {
+    if (n == 0 || (n == 1 && !iota)) {
         return N_BODY_SIM_PRO_STATUS_OK;
     }
     if (n > 0xFFFFFFFFull) {
         NBX_FAIL(error, N_BODY_SIM_PRO_STATUS_INVALID_ARGUMENT, "sort size exceeds 2^32");
-    }
-    if (n == 1) {
-        if (iota) {
-            NBX_HIP(error, hipMemsetAsync(vals, 0, sizeof(uint32_t), s));
-        }
-        if (keys_out != keys) {
-            NBX_HIP(error, hipMemcpyAsync(keys_out, keys, sizeof(uint64_t), hipMemcpyDeviceToDevice, s));
-            NBX_HIP(error, hipMemcpyAsync(vals_out, vals, sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
-        }
-        return N_BODY_SIM_PRO_STATUS_OK;
     }
     const bool large = n >= kLargeSort;
     const unsigned tiles = grid_for(n, kSortThreads * (large ? 8 : 4));
@@ -267,14 +252,9 @@ NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals
     const uint32_t* vin = iota ? nullptr : vals;
     for (int p = 0; p < passes; ++p) {
         const int shift = first_bit + kDigitBits * p;
-        // ping-pong between the two buffers; the last pass writes the output
-        const bool last = p == passes - 1;
-        uint64_t* kout = last ? keys_out : ((p & 1) ? keys : keys_alt);
-        uint32_t* vout = last ? vals_out : ((p & 1) ? vals : vals_alt);
-        if (last && (kout == kin || static_cast<const uint32_t*>(vout) == vin)) {
-            kout = (kin == keys) ? keys_alt : keys;     // output aliases the input: one more hop
-            vout = (kout == keys) ? vals : vals_alt;
-        }
+        // ping-pong between the two buffers
+        uint64_t* kout = (p & 1) ? keys : keys_alt;
+        uint32_t* vout = (p & 1) ? vals : vals_alt;
         if (large) {
             sort_histogram<8><<<tiles, kSortThreads, 0, s>>>(kin, n, shift, h, tiles,
                                                              start_clock);
@@ -295,9 +275,9 @@ NBodySimProStatus radix_sort_pairs(hipStream_t s, uint64_t* keys, uint32_t* vals
         vin = vout;
     }
     NBX_HIP(error, hipGetLastError());
-    if (kin != keys_out) {
-        NBX_HIP(error, hipMemcpyAsync(keys_out, kin, n * sizeof(uint64_t), hipMemcpyDeviceToDevice, s));
-        NBX_HIP(error, hipMemcpyAsync(vals_out, vin, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
+    if (kin != keys) {   // an odd number of passes
+        NBX_HIP(error, hipMemcpyAsync(keys, kin, n * sizeof(uint64_t), hipMemcpyDeviceToDevice, s));
+        NBX_HIP(error, hipMemcpyAsync(vals, vin, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
     }
     return N_BODY_SIM_PRO_STATUS_OK;
 }
