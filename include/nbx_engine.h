@@ -197,7 +197,8 @@ NBodySimProStatus nbx_hip_bh_learned(const NBodySimProParticleSystemView* view,
  * (a hipStream_t; NULL = the null stream): the caller synchronizes. The
  * FP32 staging lives in a fixed per-device array of the library, so
  * count <= 1048576 (larger counts: INVALID_ARGUMENT), and calls that overlap
- * on one GPU race on it.
+ * on one GPU race on it. Accelerations may be stored over the inputs: every
+ * input is read first.
  */
 NBodySimProStatus nbx_direct_fp32_noalloc(const double* positions_x, const double* positions_y,
                                           const double* positions_z, const double* masses,

@@ -36,15 +36,15 @@
 //
 // Centre of mass. Computed in FP64 from the children in octant order 0..7
 // (barnes_hut.c:230-244), one thread per cell, deepest level first. A
-// workgroup builds the cells that lie within its tile of 1,024 tree positions
-// in LDS, child tables and centres of mass together (build_kernel); two more
-// launches do those that span tiles (span_com_kernel). A cell reads its
+// workgroup builds the cells that lie within its tile of 256 to 1,024 tree
+// positions in LDS, child tables and centres of mass together (build_kernel); one
+// or two more launches do those that span tiles (span_com_kernel). A cell reads its
 // children through an 8-slot child table, so results are deterministic and
 // bit-identical to the reference.
 //
-// Walks. The FP64 walk (and the FP32 walk with reference lists): one wave =
-// 64 consecutive queries in tree order; the node index is wave-uniform (node
-// records come in through scalar loads). Each lane keeps "skip_until": it is
+// Walks. The FP64 walk (and the FP32 walk with reference lists): one wave = 8 to
+// 64 (128) consecutive queries in tree order; the node index is wave-uniform
+// (node records come in through scalar loads). Each lane keeps "skip_until": it is
 // active at node i iff i >= skip_until. Active lanes apply the reference's
 // own test (d^2 > 0 and 4h^2 < theta^2 d^2, unsoftened) and either take the
 // monopole/leaf term (then skip the subtree) or descend. The wave moves to i+1
@@ -2437,8 +2437,13 @@ __global__ __launch_bounds__(W * kWave) void group_walk_kernel(
                 }
             }
             ccnt += static_cast<int>(__popcll(cbal));
-            // opened cells: children in octant order, one octant per round
-            // (at most 64 new leaves and 64 new cells per round)
+            // opened cells: children in octant order. The feature walk goes an
+            // octant a round (at most 64 new leaves and 64 new cells) and
+            // flushes where the leaves of one do not fit, which keeps the order
+            // of its sums (a model's features) as it was. The plain walk places
+            // all eight octants' children at once, without branches, after one
+            // flush where they do not fit; a step with more leaves than the list
+            // holds takes the rounds.
             const bool open = act && !accepted;
             const int kid[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
             if (FEATURES) {

@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256) void direct_fp64_lane_kernel(
 //   108544 18.5 / 17.8, 110592 18.8 / 17.9, 131072 25.4 / 22.9
 // The kernel this replaced (64 targets per workgroup, IEEE sqrt and divide):
 // 0.049 ms at 1000, 0.186 at 4096, 0.79 at 16384, 4.28 at 40000, 9.05 at 65536
-// (now 6.9). The bound is FP64 issue: about 38 instructions and a v_rsq_f64 a
+// (now 6.9). The bound is FP64 issue: about 36 instructions and a v_rsq_f64 a
 // pair, 84 ns per 64 pairs and SIMD, against 72 instructions and two
 // transcendentals before; a tile kernel's adder and row broadcasts add 12.
 template <bool SUBSET>
@@ -534,8 +534,10 @@ __global__ void refresh_pos4_kernel(const double* __restrict__ px, const double*
 //   N = 16384 221 -> 113, 32768 396 -> 363, 65536 1533 -> 1305,
 //     131072 5668 -> 5064, 262144 20800 -> 19800  (8 ranges: 111, 387, 1363,
 //     5151, 19965; 256-source tiles instead of 64: 262144 20046)
-// At 262144 that is 3,470 G pairs/s: the issue bound of 12 full-rate
-// instructions per pair is 3,277 at the nominal 2.4 GHz.
+// At 262144 that is 3,470 G pairs/s, 44.7 cycles per wave of 64 pairs and SIMD at
+// the 2.38 GHz that the chip ran at. The bound is issue: 12 instructions of 2
+// cycles and a v_rsq_f32 of 8 are 32, and a loop of 12 v_fma_f32 and one v_rsq_f32
+// alone measured 38.7.
 template <bool ZERO_EPS>
 void launch_direct_fp32(hipStream_t st, const double* px, const double* py, const double* pz,
                         const double* m, const float4* pos, double* ax, double* ay, double* az,
