@@ -867,7 +867,7 @@ NBodySimProStatus nbx_ensemble_autotune(NBXEnsemble* e, const NBodySimProGravity
         }
     }
     double best_ms = 0.0;
-    if (!cached) {
+    auto tune = [&]() -> NBodySimProStatus {
         // 1) targets per lane, bucket by bucket, on that bucket's clusters alone
         NBXTileConfig mixed = best;
         for (int b = 0; b < nbx::kBuckets; ++b) {
@@ -924,6 +924,18 @@ NBodySimProStatus nbx_ensemble_autotune(NBXEnsemble* e, const NBodySimProGravity
         s.tile = best;
         NBX_TRY(nbx::upload_items(s, nbx::build_items(s, best, {}), error));
         best_ms = nbx::time_force(s, G, eps2, 3);
+        return N_BODY_SIM_PRO_STATUS_OK;
+    };
+    if (!cached) {
+        const NBXTileConfig before = s.tile;
+        const NBodySimProStatus status = tune();
+        if (status != N_BODY_SIM_PRO_STATUS_OK) {
+            // the shape as it was, with every cluster's items
+            s.tile = before;
+            nbx::drop_graph(s);
+            (void)nbx::upload_items(s, nbx::build_items(s, before, {}), nullptr);
+            return status;
+        }
         if (cache_path != nullptr) {
             if (FILE* f = std::fopen(cache_path, "a")) {
                 std::fprintf(f, "%s %d %d %d %d %d %d %d %d %d %d\n", key.c_str(),

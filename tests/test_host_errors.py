@@ -87,3 +87,15 @@ while True:
     k += 1
 assert k > 15, k
 """)
+
+
+def test_autotune_that_fails_leaves_the_shape(double):
+    """Timing goes through a graph, which the double does not offer: the tuner's
+    candidates must not stay behind."""
+    run(double, """
+e = nbx.Ensemble(np.array([70, 300, 5], dtype=np.uint32))
+e.set_tile([2] * 8, 3, 128)
+before = e.tile()
+assert fails(lambda: e.autotune()) != 0
+assert e.tile() == before
+""")
