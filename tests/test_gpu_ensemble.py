@@ -162,7 +162,9 @@ def test_autotune_ignores_shapes_stored_for_other_work_items(nbx, small_ensemble
 def test_autotune_does_not_leave_a_slower_shape(nbx):
     """64 clusters leave the chip room that depends on the launch before: steps
     with the tuned shape take no longer than with the one before tuning (a
-    shape has to be 1% faster to be taken; runs of one shape differ by 2%)."""
+    shape has to be 1% faster to be taken, and runs of one shape differ by some
+    percent; the shape that the launch alone would choose takes 1.16 times as
+    long)."""
     sizes = nbx.ensemble_sizes(64, lo=64, hi=4096, seed=42)
     d = nbx.ensemble_clusters(sizes, seed=7)
     with nbx.Ensemble(sizes) as ens:
@@ -175,7 +177,7 @@ def test_autotune_does_not_leave_a_slower_shape(nbx):
         rep = ens.autotune(eps=0.01)
         tuned = ms()
     print(f"steps before {before:.4f} ms, tuned {tuned:.4f} ms, {rep}")
-    assert tuned <= 1.06 * before
+    assert tuned <= 1.1 * before
 
 
 @pytest.mark.parametrize("eps", [0.01, 0.0])
